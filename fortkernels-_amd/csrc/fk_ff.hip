@@ -14,18 +14,21 @@
 // cf[n1][my_igp] = conj(aqsm[n1][igp]) and vg[my_igp] = vcoul[igp] (zero for a
 // skipped column).  tempz is never stored.
 //
-// Kernels: ff_coef_kernel (cf, vg), ff_fused_kernel (MFMA GEMM tile with
-// fragments loaded straight from global memory + row contraction of the
-// tile -> per-tile partials), ff_reduce_kernel (fixed-order sums).
+// Kernels: ff_coef_kernel (cf, vg), ff_fused_kernel (MFMA GEMM tile through
+// an LDS ring + row contraction of the tile -> per-tile partials),
+// ff_reduce_kernel (fixed-order sums).
 #include "fk_complex.h"
 #include "fk_internal.h"
+#include "fk_mfma_ring.h"
 
 #include <algorithm>
 
 namespace fk {
 namespace {
 
-typedef double d4 __attribute__((ext_vector_type(4)));
+using ring::d4;
+using ring::mfma;
+using ring::mfma_nega;
 constexpr int kXcds = 8;
 
 struct FfArgs {
@@ -34,21 +37,11 @@ struct FfArgs {
     const double2 *cf;      // [nb][G]  conj(aqsm[n1][igp])
     const double *vg;       // [G]      vcoul[igp]
     double2 *partials;      // [nfreq][mtiles][nb][2] (schDt part, schDv part)
-    int nb, C, G, nfreq, nks;
+    int nb, C, G, nfreq, nks;       // nks: ff_fused_kernel: stages of 8 ig; ff_fewband_kernel: k-steps of 4
     int tiles_m, tiles_n, mtiles;   // tiles_n = nfreq * mtiles
-    int stagger_lo, stagger_hi, stagger_ticks;
     int ksplit;             // ig ranges per column block (1: the whole range)
-    int kper;               // ff_fused_kernel with KSPLIT: k-steps per range (a multiple of P)
+    int kper;               // ff_fused_kernel: stages per range
 };
-
-__device__ __forceinline__ d4 mfma(double a, double b, d4 c)
-{
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ d4 mfma_nega(double a, double b, d4 c)
-{
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 1);
-}
 
 // Workgroup b -> tile (tm over bands fastest within an XCD's range, so the
 // band tiles that share one block of X run back to back on one XCD).
@@ -78,105 +71,80 @@ __global__ void ff_coef_kernel(const double2 *aqsm, const double *vcoul, const i
     }
 }
 
-template <int MB, int NB>
-struct Frags {
-    double2 a[MB], b[NB];
-};
-
 // 16x16x4 FP64 MFMA: lane l supplies A[l%16][l/16] (here aqsn[n1 = row l%16]
 // [ig = l/16]) and B[l/16][l%16] (X[m = col l%16][ig = l/16]); accumulator
 // register r of lane l holds T[4r + l/16][l%16].
-// KSPLIT: the ig range is split into ksplit parts of kper k-steps, one per
+//
+// Both operands are ig-contiguous in memory.  A stage is 8 ig of the
+// workgroup's BM bands and BN columns: one 128-byte line per row, and one
+// direct load moves 8 rows.  Lane l of a load takes row l/8 and, of the row's
+// line, ig (l%8) ^ (l/8), so row r keeps ig k at 16-byte slot k ^ (r%8) and
+// the 16 rows a fragment reads at one ig fall in different banks
+// (SQ_LDS_BANK_CONFLICT stays near 0).
+//
+// Tile and ring: waves of 32x32 (96 accumulator registers, 152 in all), so
+// three workgroups of 64x64 share a CU with a ring of three 16 KB stages each;
+// measured at 256/4096/4096/16: 65 TFLOP/s executed, against 63 with four
+// stages and two workgroups, 60-62 with 64x128 tiles of 8 waves, 60 with 32x64
+// waves at one wave per SIMD.
+//
+// The ig range may be split into ksplit parts of kper stages, one per
 // workgroup (column tile index = column block * ksplit + part), for problems
 // with too few tiles to fill the GPU; each part writes its own partial.
-template <int MB, int NB, int P, int WGM, int WGN, int MINW, bool KSPLIT>
+template <int MB, int NB, int WGM, int WGN, int NS, int MINW>
 __global__ __launch_bounds__(64 * WGM * WGN, MINW) void ff_fused_kernel(FfArgs a)
 {
     constexpr int NWAVES = WGM * WGN;
     constexpr int WM = MB * 16, WN = NB * 16, BM = WM * WGM, BN = WN * WGN;
-    __shared__ double2 red[NWAVES][2 * WM];
+    constexpr int kLoads = (BM + BN) / 8, LPW = kLoads / NWAVES;   // direct loads of a stage, of a wave
+    static_assert(kLoads % NWAVES == 0, "every wave moves the same number of rows");
+    __shared__ __attribute__((aligned(128))) char lds[NS][(BM + BN) * 128];
+    __shared__ double2 red[WGM][2 * WM];
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave % WGM, wn = wave / WGM;
-    if ((int)blockIdx.x >= a.stagger_lo && (int)blockIdx.x < a.stagger_hi) {
-        const uint64_t t0 = wall_clock64();
-        while (wall_clock64() - t0 < (uint64_t)a.stagger_ticks) __builtin_amdgcn_s_sleep(32);
-    }
     int tm, tn;
     tile_coords(blockIdx.x, a.tiles_m, a.tiles_m * a.tiles_n, tm, tn);
     const int f = tn / a.mtiles, mt = tn % a.mtiles;
-    const int kpart = KSPLIT ? mt % a.ksplit : 0;
-    const int s_beg = KSPLIT ? kpart * a.kper : 0;
-    const int s_end = KSPLIT ? min(a.nks, s_beg + a.kper) : a.nks;
-    const int rowbase = tm * BM + wm * WM;            // band n1
-    const int colbase = (KSPLIT ? mt / a.ksplit : mt) * BN + wn * WN;   // my_igp within frequency f
+    const int s_beg = mt % a.ksplit * a.kper;
+    const int nst = min(a.nks - s_beg, a.kper);
+    const int row0 = tm * BM, col0 = mt / a.ksplit * BN;
+    const int rowbase = row0 + wm * WM;               // band n1
+    const int colbase = col0 + wn * WN;               // my_igp within frequency f
     const int kl = lane >> 4, cl = lane & 15;
 
-    // the complex product as three real GEMMs (the 3M method; Higham, SIAM
-    // J. Matrix Anal. Appl. 13(3), 1992): T1 = (ar + ai) xr, T2 = ar (xi - xr),
-    // T3 = ai (xr + xi); re T = T1 - T3, im T = T1 + T2 (acc_re, acc_im,
-    // acc_t3 hold T1, T2, T3): 12 MFMAs per k-step where four real products
-    // take 16
-    d4 acc_re[MB][NB], acc_im[MB][NB], acc_t3[MB][NB];
+    // this wave's loads of a stage: rows 8 g .. 8 g + 7 of the tile (bands
+    // first, then columns), g = LPW wave + j.  Rows past nb and columns past
+    // G are clamped and dropped in the epilogue, ig past C is zeroed in A.
+    const double2 *src[LPW];
 #pragma unroll
-    for (int i = 0; i < MB; ++i)
-#pragma unroll
-        for (int j = 0; j < NB; ++j) {
-            acc_re[i][j] = d4{0, 0, 0, 0};
-            acc_im[i][j] = d4{0, 0, 0, 0};
-            acc_t3[i][j] = d4{0, 0, 0, 0};
-        }
-
-    // row / column addresses clamped into the arrays; rows past nb and
-    // columns past G are dropped in the epilogue, k past C is zeroed
-    const double2 *pa[MB];
-    const double2 *pb[NB];
-#pragma unroll
-    for (int i = 0; i < MB; ++i) pa[i] = a.aqsn + (size_t)min(rowbase + i * 16 + cl, a.nb - 1) * a.C;
-#pragma unroll
-    for (int j = 0; j < NB; ++j)
-        pb[j] = a.X + ((size_t)f * a.G + min(colbase + j * 16 + cl, a.G - 1)) * a.C;
-    auto load = [&](Frags<MB, NB> &fr, int s) {
-        s = min(s, s_end - 1);
-        const int k = 4 * s + kl;
-        const int kc = min(k, a.C - 1);
-        const bool kok = k < a.C;
-#pragma unroll
-        for (int i = 0; i < MB; ++i) {
-            double2 v = pa[i][kc];
-            fr.a[i] = kok ? v : make_double2(0.0, 0.0);
-        }
-#pragma unroll
-        for (int j = 0; j < NB; ++j) fr.b[j] = pb[j][kc];
-    };
-    auto mma = [&](const Frags<MB, NB> &fr) {
-        double as[MB], bd[NB], bs[NB];
-#pragma unroll
-        for (int i = 0; i < MB; ++i) as[i] = fr.a[i].x + fr.a[i].y;
-#pragma unroll
-        for (int j = 0; j < NB; ++j) {
-            bd[j] = fr.b[j].y - fr.b[j].x;
-            bs[j] = fr.b[j].x + fr.b[j].y;
-        }
-#pragma unroll
-        for (int i = 0; i < MB; ++i)
-#pragma unroll
-            for (int j = 0; j < NB; ++j) {
-                acc_re[i][j] = mfma(as[i], fr.b[j].x, acc_re[i][j]);
-                acc_im[i][j] = mfma(fr.a[i].x, bd[j], acc_im[i][j]);
-                acc_t3[i][j] = mfma(fr.a[i].y, bs[j], acc_t3[i][j]);
-            }
-    };
-    Frags<MB, NB> ring[P];
-#pragma unroll
-    for (int q = 0; q < P; ++q) load(ring[q], s_beg + q);
-    for (int s0 = s_beg; s0 < s_end; s0 += P) {
-#pragma unroll
-        for (int q = 0; q < P; ++q) {
-            mma(ring[q]);
-            load(ring[q], s0 + q + P);
-        }
+    for (int j = 0; j < LPW; ++j) {
+        const int g = LPW * wave + j;
+        if (g < BM / 8) src[j] = a.aqsn + (size_t)min(row0 + 8 * g + (lane >> 3), a.nb - 1) * a.C;
+        else src[j] = a.X + ((size_t)f * a.G + min(col0 + 8 * g - BM + (lane >> 3), a.G - 1)) * a.C;
     }
+    const int kx = 8 * s_beg + ((lane & 7) ^ (lane >> 3));
+    auto issue = [&](int s, int slot) {
+        const int ig = min(8 * s + kx, a.C - 1);
+#pragma unroll
+        for (int j = 0; j < LPW; ++j) ring::lds_load16(src[j] + ig, &lds[slot][(LPW * wave + j) * 1024]);
+    };
+    auto read = [&](ring::Frags<MB, NB> &fr, int s, int slot, int q) {
+        const char *st = &lds[slot][cl * 128 + (((4 * q + kl) ^ (cl & 7)) << 4)];
+#pragma unroll
+        for (int i = 0; i < MB; ++i) fr.a[i] = *reinterpret_cast<const double2 *>(st + (wm * WM + 16 * i) * 128);
+#pragma unroll
+        for (int j = 0; j < NB; ++j) fr.b[j] = *reinterpret_cast<const double2 *>(st + (BM + wn * WN + 16 * j) * 128);
+        const int k0 = 8 * (s_beg + s);
+        if (k0 + 8 > a.C) {   // the last stage of a ragged ig range
+            const bool kok = k0 + 4 * q + kl < a.C;
+#pragma unroll
+            for (int i = 0; i < MB; ++i) fr.a[i] = kok ? fr.a[i] : make_double2(0.0, 0.0);
+        }
+    };
+    ring::Acc3<MB, NB> acc;
+    acc.zero();
+    ring::main_loop<MB, NB, NS, LPW>(nst, acc, issue, read);
 
     // ---- epilogue: contract each row with cf (and vg cf) over the tile's columns
     double2 rt[MB][4], rv[MB][4];     // per row (i, r): schDt and schDv partials
@@ -195,8 +163,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void ff_fused_kernel(FfArgs a
             for (int r = 0; r < 4; ++r) {
                 const int row = rowbase + i * 16 + 4 * r + kl;
                 const double2 c = a.cf[(size_t)min(row, a.nb - 1) * a.G + min(col, a.G - 1)];
-                const double2 t = make_double2(acc_re[i][j][r] - acc_t3[i][j][r], acc_re[i][j][r] + acc_im[i][j][r]);
-                const double2 p = cmul(t, c);
+                const double2 p = cmul(acc.value(i, j, r), c);
                 if (cok) {
                     rt[i][r] = cadd(rt[i][r], p);
                     rv[i][r] = cadd(rv[i][r], make_double2(p.x * vgc, p.y * vgc));
@@ -423,34 +390,45 @@ __global__ __launch_bounds__(256) void ff_achs_kernel(const double2 *achs_rows, 
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-struct FfCfg { int bm, bn, p, minw; };
+struct FfCfg { int bm, bn; };
 // config ids (fk_options.config = id + 1)
-//   0: 32x32 waves, 2x2 waves (64x64 tile), ring 3, 2 workgroups/CU
-//   1: 32x64 waves, 2x2 waves (64x128 tile), ring 3, 1 workgroup/CU (default:
-//      15.4 ms against 16.2 ms for id 0 at 256/4096/4096/32 on MI355X)
+//   0: 64x64 tile, 2x2 waves, ring of 3 stages, 3 workgroups/CU (default)
+//   1: 64x128 tile, 2x4 waves, ring of 6 stages, 1 workgroup/CU
 //   2: ff_fewband_kernel, 16x64 tile through LDS (chunks of 16 ig = 4
 //      k-steps): for 16 bands or fewer, where the product is bound by
 //      reading X and a 64-row tile would spend 4x the MFMA work
 //      (kFfConfigFewBands)
-constexpr FfCfg kFfCfgs[] = {{64, 64, 3, 2}, {64, 128, 3, 1}, {kFbBM, kFbBN, 4, 2}};
+constexpr FfCfg kFfCfgs[] = {{64, 64}, {64, 128}, {kFbBM, kFbBN}};
 static_assert(kFfConfigFewBands == 3, "kFfConfigFewBands names the 16-row tile");
-constexpr int kFfDefaultCfg = 1;
 constexpr int kNumFfCfgs = sizeof(kFfCfgs) / sizeof(kFfCfgs[0]);
 
 void launch_ff_fused(int cfg, int tiles, hipStream_t s, const FfArgs &a)
 {
-    const bool ks = a.ksplit > 1;
     switch (cfg) {
-    case 0:
-        if (ks) hipLaunchKernelGGL((ff_fused_kernel<2, 2, 3, 2, 2, 2, true>), dim3(tiles), dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((ff_fused_kernel<2, 2, 3, 2, 2, 2, false>), dim3(tiles), dim3(256), 0, s, a);
-        break;
+    case 1: hipLaunchKernelGGL((ff_fused_kernel<2, 2, 2, 4, 6, 2>), dim3(tiles), dim3(512), 0, s, a); break;
     case 2: hipLaunchKernelGGL(ff_fewband_kernel, dim3(tiles), dim3(256), 0, s, a); break;
-    default:
-        if (ks) hipLaunchKernelGGL((ff_fused_kernel<2, 4, 3, 2, 2, 1, true>), dim3(tiles), dim3(256), 0, s, a);
-        else hipLaunchKernelGGL((ff_fused_kernel<2, 4, 3, 2, 2, 1, false>), dim3(tiles), dim3(256), 0, s, a);
-        break;
+    default: hipLaunchKernelGGL((ff_fused_kernel<2, 2, 2, 2, 3, 3>), dim3(tiles), dim3(256), 0, s, a); break;
     }
+}
+
+// Parts of the ig range per tile (`stages` of 8 ig) for problems with too few
+// tiles to fill the GPU: the time of the busiest CU, counting a part's
+// set-up and epilogue as kPartCost stages and one or two workgroups on a CU
+// as slower than three (they leave the MFMA pipes idle at their barriers).
+constexpr int kPartCost = 24;
+int ig_parts(int tiles, int stages, int most, int least_stages)
+{
+    const double rate[4] = {0.0, 0.75, 0.92, 1.0};
+    int best = 1;
+    double best_cost = 1e300;
+    for (int k = 1; k <= most && (k == 1 || stages >= k * least_stages); ++k) {
+        const int per = div_up(stages, k);
+        if (div_up(stages, per) != k) continue;   // no part empty
+        const int on_cu = (int)(((int64_t)tiles * k + 255) / 256);
+        const double cost = (double)on_cu * (per + kPartCost) / rate[std::min(on_cu, 3)];
+        if (cost < best_cost) { best_cost = cost; best = k; }
+    }
+    return best;
 }
 
 }  // namespace
@@ -461,7 +439,7 @@ FfLayout ff_plan(const fk_ff_problem *p, const fk_options *o, Scratch &ws)
 {
     FfLayout L;
     L.split = o->precision == FK_PREC_MIXED;
-    L.cfg = o->config > 0 ? o->config - 1 : kFfDefaultCfg;
+    L.cfg = o->config > 0 ? o->config - 1 : 0;
     if (L.split) {
         ff_split_plan(p->number_bands, p->ncouls, p->ngpown, p->nfreq, o->config, ws, L.sp);
         L.cfg = 0;
@@ -472,27 +450,19 @@ FfLayout ff_plan(const fk_ff_problem *p, const fk_options *o, Scratch &ws)
         const FfCfg &c = kFfCfgs[L.cfg];
         L.tiles_m = div_up(std::max(p->number_bands, 1), c.bm);
         L.mtiles = div_up(p->ngpown, c.bn);
-        L.nks = div_up(p->ncouls, 4 * c.p) * c.p;
+        const int tiles = L.tiles_m * p->nfreq * L.mtiles;
         if (L.cfg == kFfConfigFewBands - 1) {
             // split the ig range until there are about four workgroups per
             // CU, keeping at least two chunks per part
-            const int tiles = L.tiles_m * p->nfreq * L.mtiles, chunks = L.nks / 4;
+            L.nks = div_up(p->ncouls, kFbKC) * (kFbKC / 4);
+            const int chunks = L.nks / 4;
             while (tiles * L.ksplit < 1024 && L.ksplit < 8 && chunks / (2 * L.ksplit) >= 2) L.ksplit *= 2;
-            L.mtiles *= L.ksplit;
         } else {
-            // too few tiles for two rounds over the CUs (small problems,
-            // the per-band row contraction): split the ig range, each part
-            // at least 16 ring passes, no part empty
-            const int tiles = L.tiles_m * p->nfreq * L.mtiles, rounds = L.nks / c.p;
-            int ks = 1;
-            while (tiles * ks < 512 * c.minw && ks < 8 && rounds >= 2 * ks * 16) ks *= 2;
-            if (ks > 1) {
-                const int per = div_up(rounds, ks);
-                L.ksplit = div_up(rounds, per);
-                L.kper = per * c.p;
-                L.mtiles *= L.ksplit;
-            }
+            L.nks = div_up(p->ncouls, 8);
+            L.ksplit = o->config > 0 ? ig_parts(tiles, L.nks, 8, 24) : ig_parts(tiles, L.nks, 32, 8);
+            L.kper = div_up(L.nks, L.ksplit);
         }
+        L.mtiles *= L.ksplit;
     }
     L.off_cf = ws.plan(sizeof(double2) * (size_t)std::max(p->number_bands, 1) * p->ngpown);
     L.off_vg = ws.plan(sizeof(double) * (size_t)p->ngpown);
@@ -543,18 +513,6 @@ static int ff_fp64_gemm(const FfLayout &L, const double2 *aqsn, const double2 *X
     a.ksplit = L.ksplit;
     a.kper = L.kper;
     const int tiles = a.tiles_m * a.tiles_n;
-    a.stagger_lo = a.stagger_hi = a.stagger_ticks = 0;
-    if (kFfCfgs[L.cfg].minw == 2 && L.cfg != kFfConfigFewBands - 1 && L.ksplit == 1) {   // MFMA-bound tiles only
-        int dev = 0, ncu = 0;
-        FK_HIP(hipGetDevice(&dev));
-        FK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-        if (tiles > 2 * ncu) {
-            const double tile_cycles = 8.0 * kFfCfgs[L.cfg].bm * kFfCfgs[L.cfg].bn * 4.0 * L.nks / 64.0;
-            a.stagger_lo = ncu;
-            a.stagger_hi = 2 * ncu;
-            a.stagger_ticks = (int)std::min(0.5 * tile_cycles / 24.0, 1.0e6);
-        }
-    }
     FK_TRY(timer.start());
     launch_ff_fused(L.cfg, tiles, s, a);
     FK_HIP(hipGetLastError());
