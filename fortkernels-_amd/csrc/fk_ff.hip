@@ -41,6 +41,7 @@ struct FfArgs {
     int tiles_m, tiles_n, mtiles;   // tiles_n = nfreq * mtiles
     int ksplit;             // ig ranges per column block (1: the whole range)
     int kper;               // ff_fused_kernel: stages per range
+    int aligned;            // aqsn and X are 16-byte aligned
 };
 
 // Workgroup b -> tile (tm over bands fastest within an XCD's range, so the
@@ -126,8 +127,14 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void ff_fused_kernel(FfArgs a
     const int kx = 8 * s_beg + ((lane & 7) ^ (lane >> 3));
     auto issue = [&](int s, int slot) {
         const int ig = min(8 * s + kx, a.C - 1);
+        char *dst = &lds[slot][LPW * wave * 1024];
+        if (a.aligned) {
 #pragma unroll
-        for (int j = 0; j < LPW; ++j) ring::lds_load16(src[j] + ig, &lds[slot][(LPW * wave + j) * 1024]);
+            for (int j = 0; j < LPW; ++j) ring::lds_load16(src[j] + ig, dst + 1024 * j);
+        } else {
+#pragma unroll
+            for (int j = 0; j < LPW; ++j) reinterpret_cast<double2 *>(dst + 1024 * j)[lane] = ring::load16(src[j] + ig);
+        }
     };
     auto read = [&](ring::Frags<MB, NB> &fr, int s, int slot, int q) {
         const char *st = &lds[slot][cl * 128 + (((4 * q + kl) ^ (cl & 7)) << 4)];
@@ -512,6 +519,7 @@ static int ff_fp64_gemm(const FfLayout &L, const double2 *aqsn, const double2 *X
     a.tiles_m = L.tiles_m; a.mtiles = L.mtiles; a.tiles_n = nf * L.mtiles;
     a.ksplit = L.ksplit;
     a.kper = L.kper;
+    a.aligned = ((reinterpret_cast<uintptr_t>(aqsn) | reinterpret_cast<uintptr_t>(X)) & 15) == 0;
     const int tiles = a.tiles_m * a.tiles_n;
     FK_TRY(timer.start());
     launch_ff_fused(L.cfg, tiles, s, a);

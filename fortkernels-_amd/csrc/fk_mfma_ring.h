@@ -44,6 +44,15 @@ __device__ __forceinline__ void lds_load16(const void *g, const void *lds)
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(la) : "memory", "m0");
 }
 
+// The element at g where g need not be 16-byte aligned (an array of complex
+// numbers is aligned to its 8-byte parts only): such sources are staged by
+// way of registers, stored to LDS when the direct load would be issued.
+__device__ __forceinline__ double2 load16(const double2 *g)
+{
+    const __attribute__((address_space(1))) double *p = (const __attribute__((address_space(1))) double *)g;
+    return make_double2(p[0], p[1]);
+}
+
 // Wait until at most N of this wave's loads are in flight and its LDS reads
 // are done, then meet the other waves of the workgroup.
 template <int N>

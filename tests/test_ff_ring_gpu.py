@@ -30,3 +30,39 @@ def test_ring_edges(fk, fko, config, nb, C, G, nf):
     t, v, a, _ = fk.ff_problem(p, achs_freq=0, config=config)
     assert _rel(t, rt) <= 1e-12 and _rel(v, rv) <= 1e-12
     assert abs(complex(a[0]) - ra) <= 1e-12 * max(abs(ra), float(np.max(np.abs(rv))))
+
+
+def _off8(a):
+    """A device copy of a complex array that starts 8 bytes past a 16-byte line."""
+    import torch
+    f = np.ascontiguousarray(a).view(np.float64).reshape(-1)
+    v = torch.empty(f.size + 2, dtype=torch.float64, device="cuda:0")[1:1 + f.size]
+    v.copy_(torch.from_numpy(f))
+    assert v.data_ptr() % 16 == 8
+    return v
+
+
+def _device_options(fk):
+    o = fk.default_options()
+    o.memory, o.precision, o.config = fk.FK_MEM_DEVICE, fk.FK_PREC_FP64, 0
+    return o
+
+
+def test_inputs_aligned_to_8_bytes(fk, fko):
+    import ctypes
+
+    import torch
+    p = fko.ff_random(37, 150, 70, 3, seed=4)
+    m = torch.from_numpy(np.ascontiguousarray(p.aqsm)).to("cuda:0")
+    v = torch.from_numpy(np.ascontiguousarray(p.vcoul)).to("cuda:0")
+    n, x = _off8(p.aqsn), _off8(p.I_eps)
+    inv, ind = np.ascontiguousarray(p.inv_igp_index, np.int32), np.ascontiguousarray(p.indinv, np.int32)
+    t = torch.zeros(2, 37, 3, dtype=torch.complex128, device="cuda:0")
+    prob = fk.FfProblem(37, 150, 70, 3, m.data_ptr(), n.data_ptr(), x.data_ptr(), v.data_ptr(), inv.ctypes.data,
+                        ind.ctypes.data, 0)
+    torch.cuda.synchronize()
+    assert fk.lib.ff_kernel(ctypes.byref(prob), ctypes.byref(_device_options(fk)), t[0].data_ptr(), t[1].data_ptr(),
+                            None) == 0
+    torch.cuda.synchronize()
+    rt, rv, _ = fko.ff(p, achs_freq=0)
+    assert _rel(t[0].cpu().numpy(), rt) <= 1e-12 and _rel(t[1].cpu().numpy(), rv) <= 1e-12
