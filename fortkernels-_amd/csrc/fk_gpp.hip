@@ -16,7 +16,10 @@
 // Kernels (one call = three launches on the caller's stream):
 //   gpp_coef_kernel   c[Kpad][ldc] from aqsm / vcoul / the column map, with
 //                     the occupied bands first, zero-padded to a k-step
-//   gpp_fused_kernel  MFMA GEMM tile with operand fragments loaded straight
+//   gpp_ring_kernel   FP64, up to 16 occupied bands: MFMA GEMM tile with its
+//                     operands through an LDS ring, the pole/SX epilogue and
+//                     a wave/workgroup reduction -> per-tile partials
+//   gpp_fused_kernel  otherwise: MFMA GEMM tile with operand fragments loaded straight
 //                     from global memory into a register ring (no LDS, no
 //                     barriers), the occupied-band partial sum taken as a
 //                     register snapshot, then the pole/SX epilogue and a
@@ -26,6 +29,7 @@
 #include "fk_complex.h"
 #include "fk_gpp_common.h"
 #include "fk_internal.h"
+#include "fk_mfma_ring.h"
 
 #include <algorithm>
 #include <cmath>
@@ -52,6 +56,7 @@ struct GppArgs {
     int nb, nv, C, G, nw, ldc, Kpad;
     int nvpad;             // occupied bands rounded up to a k-step (4)
     int nks;               // k-steps (Kpad / 4)
+    int aligned;           // gpp_ring_tile: aqsn is 16-byte aligned
     int tiles_m, tiles_n, group_m;
     int stagger_lo, stagger_hi;   // workgroups that start late ...
     int stagger_ticks;            // ... by this many wall-clock ticks (100 MHz)
@@ -455,6 +460,241 @@ __device__ __forceinline__ void gpp_tile(const GppArgs<E> &a, int tm, int tn, Ti
     }
 }
 
+// ---------------------------------------------------------------------------
+// The FP64 64 x 64 tile on the LDS ring of fk_mfma_ring.h, for at most
+// kRingOcc occupied bands: 4 waves of 32 x 32, three workgroups per CU.
+//
+// gpp_tile's fragments come straight from global memory, each twice per
+// workgroup, and its MFMA pipes wait for them (70% busy); the FF contraction
+// found the same and the ring cured it.  What gpp_tile keeps in 64 KB of LDS,
+// the occupied-band sums, does not fit beside a ring at three workgroups
+// per CU.  So the main loop runs over the unoccupied bands only and the
+// epilogue contracts the few occupied ones per 16 x 16 block just before it
+// needs them: Bo for asxtemp, and B = Bu + Bo.  To leave registers for that
+// (168 a lane at this occupancy), three of a wave's four blocks of Bu wait in
+// the ring's memory, 12 KB a wave, which the main loop is done with.
+//
+// Measured at 512/2/32768/1638, 3 frequencies (gpp_tile 3.05 ms): 2.74 ms, of
+// it 2.43 the main loop (68 TFLOP/s executed, the matrix clock then at about
+// 2.2 GHz), 0.19 the pole terms, the rest set-up, occupied bands and
+// reductions; with the short pole terms but two workgroups per CU and all of
+// Bu in registers 2.89; with three and Bu in registers (spilled) 2.91.
+//
+// A stage is 8 coefficient rows of 64 columns and 8 aqsn rows of 64 columns,
+// each row one 1 KB direct load; a fragment is four 256-byte row pieces, free
+// of bank conflicts as it is.
+// ---------------------------------------------------------------------------
+constexpr int kRingStages = 3;
+constexpr int kRingWgs = 3;      // workgroups per CU
+constexpr int kRingOcc = 16;
+constexpr int kRingNwc = 4;      // frequencies per epilogue pass of calls with more than three
+
+template <int NWC>
+struct RingLds {
+    union {
+        double2 ring[kRingStages][2][8][64];     // [slot][coefficients, aqsn][k][column]
+        double2 bu[4][3][4][64];                 // [wave][block - 1][register][lane]
+    };
+    double red[4][4 * NWC];
+};
+
+// ALL: nw == NWC, one epilogue pass.
+template <int NWC, bool ALL, bool ACHS, bool TABLE>
+__device__ __forceinline__ void gpp_ring_tile(const GppArgs<double2> &a, int tm, int tn, RingLds<NWC> &sh)
+{
+    constexpr int MB = 2, NB = 2, NWAVES = 4, LPW = 4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave & 1, wn = wave >> 1;
+    const int rowbase = tm * 64 + wm * 32, colbase = tn * 64 + wn * 32;
+    const int nmax = a.C - 1;
+    const int kl = lane >> 4, cl = lane & 15;
+    const int nst = (a.nks * 4 - a.nvpad) / 8;       // stages
+
+    // this wave's rows of a stage: k = 4 (wave % 2) .. + 3 of the coefficients
+    // (waves 0, 1) or of aqsn (2, 3).  Stage s holds coefficient rows nvpad +
+    // 8 s ...; band and column are clamped into aqsn (a zero row of c makes a
+    // clamped band irrelevant, the epilogue drops a clamped column).
+    const bool side_a = wave < 2;
+    const int k0 = 4 * (wave & 1);
+    const double2 *src = side_a ? a.c + tm * 64 + lane : a.aqsn + min(tn * 64 + lane, nmax);
+    const size_t ld = side_a ? (size_t)a.ldc : (size_t)a.C;
+    const int row0 = (side_a ? a.nvpad : a.nv) + k0;
+    const int last = side_a ? a.nks * 4 - 1 : a.nb - 1;
+    const bool direct = side_a || a.aligned;
+    auto issue = [&](int s, int slot) {
+        const int r = row0 + 8 * s;
+        double2 *dst = &sh.ring[slot][side_a ? 0 : 1][k0][0];
+        if (direct) {
+#pragma unroll
+            for (int j = 0; j < LPW; ++j) ring::lds_load16(src + (size_t)min(r + j, last) * ld, dst + 64 * j);
+        } else {
+#pragma unroll
+            for (int j = 0; j < LPW; ++j) dst[64 * j + lane] = ring::load16(src + (size_t)min(r + j, last) * ld);
+        }
+    };
+    auto read = [&](ring::Frags<MB, NB> &f, int, int slot, int q) {
+        const double2 *st = &sh.ring[slot][0][4 * q + kl][cl];
+#pragma unroll
+        for (int i = 0; i < MB; ++i) f.a[i] = st[wm * 32 + 16 * i];
+#pragma unroll
+        for (int j = 0; j < NB; ++j) f.b[j] = st[8 * 64 + wn * 32 + 16 * j];
+    };
+    ring::Acc3<MB, NB> acc;
+    acc.zero();
+    ring::main_loop<MB, NB, kRingStages, LPW>(nst, acc, issue, read);
+    ring::wait_barrier<0>();
+
+    // ---- epilogue ----------------------------------------------------------
+    double2 Bu0[4];
+#pragma unroll
+    for (int k = 0; k < MB * NB; ++k)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const double2 v = acc.value(k / NB, k % NB, r);
+            if (k == 0) Bu0[r] = v;
+            else sh.bu[wave][k - 1][r][lane] = v;
+        }
+    const bool want_ssx = a.nv > 0;
+    const int nko = (a.nv + 3) / 4;
+    unsigned rowok = 0;                       // rows of this lane that are real, kept columns
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = rowbase + i * 16 + 4 * r + kl;
+            const bool ok = row < a.G && gld<TABLE>(a.igp, min(row, a.G - 1)) >= 0;
+            rowok |= (ok ? 1u : 0u) << (i * 4 + r);
+        }
+    const size_t tile = (size_t)tm + (size_t)tn * a.tiles_m;
+    double2 sachs = make_double2(0.0, 0.0);
+    for (int w0 = 0; w0 < (ALL ? 1 : a.nw); w0 += NWC) {
+        double2 sach[NWC], sasx[NWC];
+#pragma unroll
+        for (int q = 0; q < NWC; ++q) { sach[q] = make_double2(0.0, 0.0); sasx[q] = make_double2(0.0, 0.0); }
+        unsigned general = 0;
+#pragma unroll
+        for (int k = 0; k < MB * NB; ++k) {
+            __builtin_amdgcn_sched_barrier(0);
+            const int i = k / NB, j = k % NB, col = colbase + j * 16 + cl;
+            double2 cwt[4], cie[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = rowbase + i * 16 + 4 * r + kl;
+                const size_t e = (size_t)min(row, a.G - 1) * a.C + min(col, nmax);
+                cwt[r] = gld<TABLE>(a.wtilde, e);
+                cie[r] = gld<TABLE>(a.I_eps, e);
+            }
+            // occupied bands of the block, fragments straight from global memory
+            ring::Acc3<1, 1> o;
+            o.zero();
+            for (int ks = 0; ks < nko; ++ks) {
+                ring::Frags<1, 1> f;
+                f.a[0] = gld<TABLE>(a.c, (size_t)(4 * ks + kl) * a.ldc + rowbase + 16 * i + cl);
+                f.b[0] = gld<TABLE>(a.aqsn, (size_t)min(4 * ks + kl, a.nb - 1) * a.C + min(col, nmax));
+                o.mma(f);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (((rowok >> (i * 4 + r)) & 1u) && col <= nmax) {
+                    const double2 Bo = o.value(0, 0, r);
+                    const double2 B = cadd(k == 0 ? Bu0[r] : sh.bu[wave][k > 0 ? k - 1 : 0][r][lane], Bo);
+                    if (!pole_terms<NWC, ALL>(a.pp, w0, cwt[r], cie[r], B, Bo, want_ssx, sach, sasx))
+                        general |= 1u << (k * 4 + r);
+                    if constexpr (ACHS) {
+                        if (w0 == 0) sachs = csub(sachs, cmul(B, cie[r]));
+                    }
+                }
+            }
+        }
+        // the elements pole_terms left out (hardly ever any), one at a time
+        if (__ballot(general != 0)) {
+#pragma unroll 1
+            for (int el = 0; el < MB * NB * 4; ++el) {
+                if ((general >> el) & 1u) {
+                    const int k = el >> 2, r = el & 3;
+                    const int row = rowbase + (k / NB) * 16 + 4 * r + kl, col = colbase + (k % NB) * 16 + cl;
+                    double2 B;
+                    switch (el) {             // constant register indices
+                    case 0: B = Bu0[0]; break;
+                    case 1: B = Bu0[1]; break;
+                    case 2: B = Bu0[2]; break;
+                    case 3: B = Bu0[3]; break;
+                    default: B = sh.bu[wave][k - 1][r][lane];
+                    }
+                    double2 Bo = make_double2(0.0, 0.0);
+                    for (int n1 = 0; n1 < a.nv; ++n1)
+                        Bo = cfma(Bo, gld<TABLE>(a.c, (size_t)n1 * a.ldc + row), gld<TABLE>(a.aqsn, (size_t)n1 * a.C + col));
+                    const size_t e = (size_t)row * a.C + col;
+                    pole_element<NWC>(a.pp, w0, true, gld<TABLE>(a.wtilde, e), gld<TABLE>(a.I_eps, e), cadd(B, Bo), Bo,
+                                      want_ssx, sach, sasx);
+                }
+            }
+        }
+        // wave reduction, then a fixed-order sum over the waves
+        double v[4 * NWC];
+#pragma unroll
+        for (int q = 0; q < NWC; ++q) {
+            v[4 * q + 0] = sach[q].x;
+            v[4 * q + 1] = sach[q].y;
+            v[4 * q + 2] = sasx[q].x;
+            v[4 * q + 3] = sasx[q].y;
+        }
+        if (ALL || w0 + NWC >= a.nw) {
+            const double x = wave_sums_lds(v, lane, reinterpret_cast<double *>(&sh.bu[wave][0][0][0]));
+            if (lane < 4 * NWC) sh.red[wave][lane] = x;
+        } else {          // Bu stays where it is for the next pass
+#pragma unroll
+            for (int q = 0; q < 4 * NWC; ++q) {
+                const double x = wave_sum(v[q]);
+                if (lane == 0) sh.red[wave][q] = x;
+            }
+        }
+        __syncthreads();
+        if (tid < 4 * NWC) {
+            const int iw = w0 + (tid >> 2);
+            if (iw < a.nw) {
+                double sum = sh.red[0][tid];
+#pragma unroll
+                for (int w = 1; w < NWAVES; ++w) sum += sh.red[w][tid];
+                // component 0,1: achtemp re,im; 2,3: asxtemp re,im
+                gst<TABLE>(reinterpret_cast<double *>(a.partials + (tile * a.nw + iw) * 2), tid & 3, sum);
+            }
+        }
+        __syncthreads();
+    }
+    if constexpr (ACHS) {
+        const double v0 = wave_sum(sachs.x), v1 = wave_sum(sachs.y);
+        if (lane == 0) {
+            sh.red[wave][0] = v0;
+            sh.red[wave][1] = v1;
+        }
+        __syncthreads();
+        if (tid < 2) {
+            double sum = sh.red[0][tid];
+#pragma unroll
+            for (int w = 1; w < NWAVES; ++w) sum += sh.red[w][tid];
+            gst<TABLE>(reinterpret_cast<double *>(a.achs_part + tile), tid, sum);
+        }
+        __syncthreads();
+    }
+}
+
+template <int NWC, bool ALL, bool ACHS>
+__global__ __launch_bounds__(256, kRingWgs) void gpp_ring_kernel(GppArgs<double2> a)
+{
+    __shared__ RingLds<NWC> sh;
+    // The second and third workgroup slots of a CU start one and two thirds
+    // of a tile late (see gpp_fused_kernel).
+    if (a.stagger_ticks && (int)blockIdx.x >= a.stagger_lo && (int)blockIdx.x < kRingWgs * a.stagger_lo) {
+        const uint64_t t0 = wall_clock64(), ticks = (uint64_t)a.stagger_ticks * (blockIdx.x / a.stagger_lo);
+        while (wall_clock64() - t0 < ticks) __builtin_amdgcn_s_sleep(32);
+    }
+    int tm, tn;
+    tile_coords(blockIdx.x, a.tiles_m, a.tiles_n, a.group_m, tm, tn);
+    gpp_ring_tile<NWC, ALL, ACHS, false>(a, tm, tn, sh);
+}
+
 // One problem, one tile per workgroup.
 template <class E, int MB, int NB, int P, int WGM, int WGN, int MINW, int NWC, bool ACHS>
 __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gpp_fused_kernel(GppArgs<E> a)
@@ -501,6 +741,26 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gpp_batch_kernel(const G
         const int prob = __builtin_amdgcn_readfirstlane(bt.prob);
         const int tm = __builtin_amdgcn_readfirstlane(bt.tm), tn = __builtin_amdgcn_readfirstlane(bt.tn);
         gpp_tile<E, MB, NB, P, WGM, WGN, NWC, false, true>(probs[prob], tm, tn, sh);
+    }
+}
+
+// The same for gpp_ring_tile (problems with at most kRingOcc occupied bands).
+__global__ __launch_bounds__(256, kRingWgs) void gpp_ring_batch_kernel(const GppArgs<double2> *__restrict__ probs,
+                                                                       const BatchTile *__restrict__ tiles, int ntiles,
+                                                                       int *counter)
+{
+    __shared__ RingLds<kRingNwc> sh;
+    __shared__ int next;
+    for (;;) {
+        if (threadIdx.x == 0) next = atomicAdd(counter, 1);
+        __syncthreads();
+        const int t = __builtin_amdgcn_readfirstlane(next);
+        __syncthreads();
+        if (t >= ntiles) break;
+        const BatchTile bt = tiles[t];
+        const int prob = __builtin_amdgcn_readfirstlane(bt.prob);
+        const int tm = __builtin_amdgcn_readfirstlane(bt.tm), tn = __builtin_amdgcn_readfirstlane(bt.tn);
+        gpp_ring_tile<kRingNwc, false, false, true>(probs[prob], tm, tn, sh);
     }
 }
 
@@ -604,7 +864,8 @@ constexpr int kGroupM = FK_GPP_GROUP_M;
 struct TileCfg { int bm, bn, p, minw; };
 // config ids (fk_options.config = id + 1): wave tile, ring depth, waves, WG/CU
 //   0: 32x64 waves, ring 4, 1x4 waves (32x256 tile), 1 workgroup/CU
-//   1: 32x32 waves, ring 3, 2x2 waves (64x64 tile),  2 workgroups/CU
+//   1: 32x32 waves, ring 3, 2x2 waves (64x64 tile),  2 workgroups/CU; FP64
+//      with at most kRingOcc occupied bands: gpp_ring_tile, 3 workgroups/CU
 //   2: 64x32 waves, ring 3, 2x2 waves (128x64 tile), 2 workgroups/CU
 //   3: 32x64 waves, ring 3, 2x2 waves (64x128 tile), 2 workgroups/CU
 constexpr TileCfg kCfgs[] = {{32, 256, 4, 1}, {64, 64, 3, 2}, {128, 64, 3, 2}, {64, 128, 3, 2}};
@@ -654,6 +915,23 @@ void launch_fused(int cfg, int tiles, hipStream_t s, const GppArgs<E> &a)
     else launch_fused_achs<E, false>(cfg, tiles, s, a);
 }
 
+// gpp_ring_tile runs FP64 calls with the 64 x 64 tiles and at most kRingOcc
+// occupied bands: it contracts those block by block, half the work per loaded
+// fragment, which is lost in the whole while they are few (16 of 512 bands
+// cost nothing that could be measured against 4).
+bool ring_form(int cfg, size_t elem, int nv) { return cfg == 1 && elem == sizeof(double2) && nv <= kRingOcc; }
+
+template <bool ACHS>
+void launch_ring(int tiles, hipStream_t s, const GppArgs<double2> &a)
+{
+    switch (a.nw) {
+    case 1: hipLaunchKernelGGL((gpp_ring_kernel<1, true, ACHS>), dim3(tiles), dim3(256), 0, s, a); break;
+    case 2: hipLaunchKernelGGL((gpp_ring_kernel<2, true, ACHS>), dim3(tiles), dim3(256), 0, s, a); break;
+    case 3: hipLaunchKernelGGL((gpp_ring_kernel<3, true, ACHS>), dim3(tiles), dim3(256), 0, s, a); break;
+    default: hipLaunchKernelGGL((gpp_ring_kernel<kRingNwc, false, ACHS>), dim3(tiles), dim3(256), 0, s, a); break;
+    }
+}
+
 int choose_cfg(const fk_gpp_problem *p, const fk_options *o)
 {
     (void)p;
@@ -664,6 +942,7 @@ int choose_cfg(const fk_gpp_problem *p, const fk_options *o)
 }
 
 struct Layout {
+    bool ring;
     int cfg, Kpad, nvpad, ldc, tiles_m, tiles_n;
     size_t off_c, off_igp, off_part, off_achs;
     size_t off_stop;   // the gppsum = 1 form: the occupied loop's stop per column
@@ -675,9 +954,11 @@ Layout plan_layout(const fk_gpp_problem *p, const fk_options *o, Scratch &ws, si
     const bool sym = p->semantics == FK_GPP_GPPSUM;
     L.cfg = sym ? 1 : choose_cfg(p, o);   // the gppsum = 1 kernel has 64 x 64 tiles
     const TileCfg &t = kCfgs[L.cfg];
+    L.ring = !sym && ring_form(L.cfg, elem, p->nvband);
+    const int kstep = L.ring ? 8 : 4 * t.p;
     L.nvpad = div_up(p->nvband, 4) * 4;
     const int rows = std::max(L.nvpad + p->number_bands - p->nvband, 1);
-    L.Kpad = div_up(rows, 4 * t.p) * 4 * t.p;
+    L.Kpad = L.ring ? L.nvpad + div_up(p->number_bands - p->nvband, kstep) * kstep : div_up(rows, kstep) * kstep;
     L.ldc = div_up(p->ngpown, t.bm) * t.bm;
     L.tiles_m = L.ldc / t.bm;
     L.tiles_n = div_up(p->ncouls, t.bn);
@@ -784,6 +1065,7 @@ int launch_gpp(const fk_gpp_problem *p, const fk_options *o, const Layout &L, Sc
     a.achs_part = d_achs ? static_cast<double2 *>(ws.at(L.off_achs)) : nullptr;
     a.nb = p->number_bands; a.nv = p->nvband; a.C = C; a.G = G; a.nw = p->nfreq; a.ldc = L.ldc; a.Kpad = L.Kpad;
     a.nvpad = L.nvpad; a.nks = L.Kpad / 4;
+    a.aligned = (reinterpret_cast<uintptr_t>(aqsn) & 15) == 0;
     a.tiles_m = L.tiles_m; a.tiles_n = L.tiles_n;
     a.group_m = std::min(L.tiles_m, kGroupM);
     const int tiles = L.tiles_m * L.tiles_n;
@@ -793,7 +1075,14 @@ int launch_gpp(const fk_gpp_problem *p, const fk_options *o, const Layout &L, Sc
         int dev = 0, ncu = 0;
         FK_HIP(hipGetDevice(&dev));
         FK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-        if (tiles > 2 * ncu) {
+        if (L.ring) {
+            // a third of a tile alone on its CU: 6 flops per complex
+            // multiply-add (3M) at 128 flop/cycle, 2.4 GHz
+            if (tiles > kRingWgs * ncu) {
+                a.stagger_lo = ncu;
+                a.stagger_ticks = (int)std::min(6.0 * 64 * 64 * L.Kpad / 128.0 / 24.0, 1.0e6);
+            }
+        } else if (tiles > 2 * ncu) {
             // half a tile of MFMA work at half a CU's rate (two workgroups
             // share it): FP64 MFMA 128 flop/cycle/CU, FP32 256; 2.4 GHz clock,
             // 100 MHz wall clock
@@ -807,7 +1096,13 @@ int launch_gpp(const fk_gpp_problem *p, const fk_options *o, const Layout &L, Sc
     a.pp = make_pole_params(p->wx, p->nfreq, p->limittwo, p->limitone, p->to1, o->mask != 0);
     KernelTimer timer(o->kernel_ms, s);
     FK_TRY(timer.start());
-    launch_fused<E>(L.cfg, tiles, s, a);
+    if constexpr (sizeof(E) == sizeof(double2)) {
+        if (!L.ring) launch_fused<E>(L.cfg, tiles, s, a);
+        else if (a.achs_part) launch_ring<true>(tiles, s, a);
+        else launch_ring<false>(tiles, s, a);
+    } else {
+        launch_fused<E>(L.cfg, tiles, s, a);
+    }
     FK_HIP(hipGetLastError());
     FK_TRY(timer.stop());
     hipLaunchKernelGGL(gpp_reduce_kernel, dim3(2 * p->nfreq), dim3(256), 0, s, part, tiles, p->nfreq,
@@ -1079,12 +1374,14 @@ struct GppBatch {
     size_t bytes = 0, off_args = 0, off_tiles = 0, off_counter = 0, off_out = 0, off_coef = 0, off_red = 0,
            off_nw = 0, off_ptrs = 0;
     int64_t coef_total = 0;
+    bool few_occ = false;      // every problem has at most kRingOcc occupied bands
     hipStream_t cs = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     fk_options opt;
 
     char *at(size_t off) const { return static_cast<char *>(mem) + off; }
+    bool ring(int c) const { return few_occ && ring_form(c, elem(), 0); }
     size_t elem() const { return mixed ? sizeof(float2) : sizeof(double2); }
 
     ~GppBatch()
@@ -1126,8 +1423,10 @@ struct GppBatch {
             // larger padding.  (With the common padding the batch ran 3.5%
             // slower than the single calls.)
             const int kstep = 4 * t.p;
-            a.Kpad = div_up(std::max(b.nvpad + b.nb - b.nv, 1), kstep) * kstep;
+            a.Kpad = ring(c) ? b.nvpad + div_up(b.nb - b.nv, 8) * 8
+                             : div_up(std::max(b.nvpad + b.nb - b.nv, 1), kstep) * kstep;
             a.nks = a.Kpad / 4;
+            a.aligned = (reinterpret_cast<uintptr_t>(a.aqsn) & 15) == 0;
             a.tiles_m = div_up(b.G, t.bm);
             a.tiles_n = div_up(b.C, t.bn);
             a.group_m = a.tiles_m;   // unused: the batch walks its own tile table
@@ -1166,9 +1465,18 @@ struct GppBatch {
         const int cblocks = (int)std::min<int64_t>((coef_total + 255) / 256, 1 << 16);
         hipLaunchKernelGGL(gpp_coef_batch_kernel<E>, dim3(std::max(cblocks, 1)), dim3(256), 0, s,
                            reinterpret_cast<const CoefBatch<E> *>(at(off_coef)), n, coef_total);
-        launch_batch<E>(cfg, ncu * kCfgs[cfg].minw, s, reinterpret_cast<const GppArgs<E> *>(at(off_args)),
-                        reinterpret_cast<const BatchTile *>(at(off_tiles)), ntiles,
-                        reinterpret_cast<int *>(at(off_counter)));
+        const GppArgs<E> *args = reinterpret_cast<const GppArgs<E> *>(at(off_args));
+        const BatchTile *tiles = reinterpret_cast<const BatchTile *>(at(off_tiles));
+        int *counter = reinterpret_cast<int *>(at(off_counter));
+        bool done = false;
+        if constexpr (sizeof(E) == sizeof(double2)) {
+            if (ring(cfg)) {
+                hipLaunchKernelGGL(gpp_ring_batch_kernel, dim3(ncu * kRingWgs), dim3(256), 0, s, args, tiles, ntiles,
+                                   counter);
+                done = true;
+            }
+        }
+        if (!done) launch_batch<E>(cfg, ncu * kCfgs[cfg].minw, s, args, tiles, ntiles, counter);
         hipLaunchKernelGGL(gpp_reduce_batch_kernel, dim3(2 * kMaxFreq, n), dim3(256), 0, s,
                            reinterpret_cast<const ReduceBatch *>(at(off_red)), reinterpret_cast<double2 *>(at(off_out)));
         FK_HIP(hipGetLastError());
@@ -1190,12 +1498,15 @@ struct GppBatch {
         off_counter = plan.plan(sizeof(int));
         max_tiles_total = 0;
         coef_total = 0;
+        few_occ = true;
+        for (const fk_gpp_problem &p : src) few_occ = few_occ && p.nvband <= kRingOcc;
         for (int i = 0; i < n; ++i) {
             BatchProb &b = prob[i];
             const fk_gpp_problem &p = src[i];
             b.nb = p.number_bands; b.nv = p.nvband; b.C = p.ncouls; b.G = p.ngpown; b.nw = p.nfreq;
             b.nvpad = div_up(b.nv, 4) * 4;
-            b.Kpad = div_up(std::max(b.nvpad + b.nb - b.nv, 1), 48) * 48;
+            // at least gpp_ring_tile's rows too: nvpad and the other bands in eights
+            b.Kpad = div_up(std::max(b.nvpad + div_up(b.nb - b.nv, 8) * 8, 1), 48) * 48;
             b.ldc = div_up(b.G, 128) * 128;
             b.max_tiles = 0;
             for (int c = 0; c < kNumCfgs; ++c)
