@@ -1628,7 +1628,7 @@ struct OzBatch {
     std::vector<fk_gpp_problem> src;
     void *mem = nullptr;
     size_t bytes = 0, off_rec = 0, off_first = 0, off_red = 0, off_out = 0, off_nw = 0, off_ptrs = 0;
-    int total_prep = 0, total_gemm = 0, total_pole = 0;
+    int total_prep = 0, total_gemm = 0, total_pole[kOzPoleClasses] = {};
     hipStream_t cs = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -1674,7 +1674,7 @@ struct OzBatch {
         const size_t rec_bytes = gpp_oz_batch_record_bytes();
         Scratch plan;
         off_rec = plan.plan(rec_bytes * n);
-        off_first = plan.plan(sizeof(int) * 3 * (size_t)(n + 1));
+        off_first = plan.plan(sizeof(int) * (2 + kOzPoleClasses) * (size_t)(n + 1));
         off_red = plan.plan(sizeof(ReduceBatch) * n);
         off_out = plan.plan(sizeof(double2) * 2 * kMaxFreq * n);
         off_nw = plan.plan(sizeof(int) * n);
@@ -1695,7 +1695,7 @@ struct OzBatch {
             return FK_ERR_NOMEM;
         }
         std::vector<char> recs(rec_bytes * n);
-        std::vector<int> first(3 * (size_t)(n + 1), 0), nw(n);
+        std::vector<int> first((2 + kOzPoleClasses) * (size_t)(n + 1), 0), nw(n);
         std::vector<ReduceBatch> red(n);
         for (int i = 0; i < n; ++i) {
             const fk_gpp_problem &p = src[i];
@@ -1711,7 +1711,8 @@ struct OzBatch {
                                                      recs.data() + rec_bytes * i);
             first[i + 1] = first[i] + nbk.prep;
             first[(n + 1) + i + 1] = first[(n + 1) + i] + nbk.gemm;
-            first[2 * (n + 1) + i + 1] = first[2 * (n + 1) + i] + nbk.pole;
+            for (int c = 0; c < kOzPoleClasses; ++c)
+                first[(2 + c) * (n + 1) + i + 1] = first[(2 + c) * (n + 1) + i] + (c == nbk.pole_class ? nbk.pole : 0);
             red[i].partials = static_cast<const double2 *>(ws.at(L.off_part));
             red[i].tiles = nbk.pole;
             red[i].nw = p.nfreq;
@@ -1720,7 +1721,7 @@ struct OzBatch {
         }
         total_prep = first[n];
         total_gemm = first[(n + 1) + n];
-        total_pole = first[2 * (n + 1) + n];
+        for (int c = 0; c < kOzPoleClasses; ++c) total_pole[c] = first[(2 + c) * (n + 1) + n];
         FK_HIP(hipMemcpyAsync(at(off_rec), recs.data(), recs.size(), hipMemcpyHostToDevice, cs));
         FK_HIP(hipMemcpyAsync(at(off_first), first.data(), sizeof(int) * first.size(), hipMemcpyHostToDevice, cs));
         FK_HIP(hipMemcpyAsync(at(off_red), red.data(), sizeof(ReduceBatch) * n, hipMemcpyHostToDevice, cs));

@@ -50,25 +50,11 @@ inline PoleParams make_pole_params(const double *wx, int nfreq, double limittwo,
 __device__ __forceinline__ double2 widen(double2 v) { return v; }
 __device__ __forceinline__ double2 widen(float2 v) { return make_double2((double)v.x, (double)v.y); }
 
-// 1/x from v_rcp_f64 refined by STEPS Newton steps.  Measured on MI355X
-// over 4M inputs spanning 2^-40 .. 2^40: v_rcp_f64 alone is within 4.2e8
-// units of 2^-53 (about 2^-24 relative), one step within 20, two steps
-// equal the IEEE quotient.
-template <int STEPS = 2>
-__device__ __forceinline__ double rcp_fast(double x)
-{
-    double r = __builtin_amdgcn_rcp(x);
-#pragma unroll
-    for (int k = 0; k < STEPS; ++k) {
-        const double e = __builtin_fma(-x, r, 1.0);
-        r = __builtin_fma(r, e, r);
-    }
-    return r;
-}
-
-// 1/x from v_rcp_f64 and one step of third order: with e = 1 - x r (about
-// 2^-24), r (1 + e + e^2) is off by e^3, below the last rounding, in three
-// fused operations where two Newton steps take four.
+// 1/x from v_rcp_f64 and one step of third order.  Measured over 4M inputs
+// spanning 2^-40 .. 2^40, v_rcp_f64 alone is within 4.2e8 units of 2^-53
+// (about 2^-24 relative); with e = 1 - x r, r (1 + e + e^2) is off by e^3,
+// below the last rounding, in three fused operations where two Newton steps
+// (equal to the IEEE quotient) take four.
 __device__ __forceinline__ double rcp_cubic(double x)
 {
     const double r = __builtin_amdgcn_rcp(x);
@@ -100,25 +86,27 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
-// Sums of N <= 16 values over the wave through `buf`, 16 * 65 doubles of LDS
-// of its own: lane q < N returns the total of value q.  Lane q + 16 h adds
-// value q of lanes 16 h .. 16 h + 15, then the four quarters meet: N writes,
-// 16 reads and 18 additions where N butterflies take 12 N shuffles and 6 N
-// additions (13312 tiles of 12 values: 0.05 ms less).  A fixed order.
+// Sums of N <= 16 values over the wave through `buf`, 65 P doubles of LDS of
+// its own (P = N rounded up to 8 or 16): lane q < N returns the total of value
+// q.  Lane q + P h adds value q of lanes P h .. P h + P - 1, then the parts
+// meet: for 16 values 16 writes, 16 reads and 18 additions where 16 butterflies
+// take 192 shuffles and 96 additions (13312 tiles of 12 values: 0.05 ms less).
+// A fixed order.
 template <int N>
 __device__ __forceinline__ double wave_sums_lds(const double (&v)[N], int lane, double *buf)
 {
-    static_assert(N <= 16, "one value per lane of a quarter");
+    constexpr int P = N <= 8 ? 8 : 16;
+    static_assert(N <= 16, "one value per lane of a part");
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
     for (int q = 0; q < N; ++q) buf[q * 65 + lane] = v[q];
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    const double *p = buf + (lane & 15) * 65 + (lane & 48);
+    const double *p = buf + (lane & (P - 1)) * 65 + (lane & ~(P - 1));
     double x = 0.0;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) x += p[k];
-    x += __shfl_xor(x, 16, 64);
-    x += __shfl_xor(x, 32, 64);
+    for (int k = 0; k < P; ++k) x += p[k];
+#pragma unroll
+    for (int off = P; off < 64; off <<= 1) x += __shfl_xor(x, off, 64);
     return x;
 }
 
@@ -131,28 +119,13 @@ __device__ __forceinline__ double wave_sums_lds(const double (&v)[N], int lane, 
 // -I_eps delw conj(z) / (4 |z|^2), z = delw + 0.5 (Omega2 conj(cden) /
 // |cden|^2 with cden = 4 wtilde^2 z and Omega2 = wtilde^2 I_eps loses its
 // wtilde^2).
-// HOIST = false evaluates the products per frequency, as the MFMA kernels'
-// epilogues need (fewer live registers); HOIST = true forms B I_eps,
-// Bo Omega2 and Bo I_eps once per element, for the stand-alone pole kernel:
-//   B D = (B I_eps) delw,  Bo ssx = (Bo Omega2) / wx^2  or
-//   -(Bo I_eps) delw conj(z) / (4 |z|^2).
-// Both equal the reference's expressions up to rounding.
-template <int NWC, bool HOIST = false>
+template <int NWC>
 __device__ __forceinline__ void pole_element(const PoleParams &pp, int w0, bool ok, double2 wt, double2 ie,
                                              double2 B, double2 Bo, bool want_ssx, double2 (&sach)[NWC],
                                              double2 (&sasx)[NWC])
 {
-    // HOIST (the mixed-precision pole kernel): one Newton step, 2e-15
-    // relative, far inside the 1e-13 band that takes the IEEE quotient
-    constexpr int kSteps = HOIST ? 1 : 2;
     const double tol1 = 1e-13 * pp.limitone, tol2 = 1e-13 * pp.to1;
     const double2 Om = cmul(cmul(wt, wt), ie);
-    double2 Bie = B, BoOm = Om, Boie = ie;
-    if constexpr (HOIST) {
-        Bie = cmul(B, ie);
-        BoOm = cmul(Bo, Om);
-        Boie = cmul(Bo, ie);
-    }
 #pragma unroll
     for (int q = 0; q < NWC; ++q) {
         const int iw = min(w0 + q, pp.nw - 1);
@@ -161,7 +134,7 @@ __device__ __forceinline__ void pole_element(const PoleParams &pp, int w0, bool 
         const double wdiffr = pole_wdiffr(wdr, -wt.y);
         double2 delw;
         double delwr;
-        pole_delw(wt, wdr, rcp_fast<kSteps>(wdiffr), delw, delwr);
+        pole_delw(wt, wdr, rcp_cubic(wdiffr), delw, delwr);
         // points within 1e-13 of a branch threshold take the IEEE quotient,
         // so every branch decision is the reference's
         const bool near = fabs(delwr - pp.limitone) <= tol1 || fabs(delwr - pp.to1) <= tol2;
@@ -169,31 +142,22 @@ __device__ __forceinline__ void pole_element(const PoleParams &pp, int w0, bool 
             if (near) pole_delw(wt, wdr, 1.0 / wdiffr, delw, delwr);
         }
         const bool m = (wdiffr > pp.limittwo) && (delwr < pp.limitone);
-        if constexpr (HOIST) {
-            const double2 t = (live && (m || !pp.mask_on)) ? cmul(Bie, delw) : make_double2(0.0, 0.0);
-            sach[q] = cadd(sach[q], t);
-        } else {
-            const double2 D = (m || !pp.mask_on) ? cmul(delw, ie) : make_double2(0.0, 0.0);
-            const double2 t = cmul(B, D);
-            if (live) sach[q] = cadd(sach[q], t);
-        }
+        const double2 D = (m || !pp.mask_on) ? cmul(delw, ie) : make_double2(0.0, 0.0);
+        const double2 t = cmul(B, D);
+        if (live) sach[q] = cadd(sach[q], t);
         if (want_ssx) {
-            double2 S = m ? make_double2(BoOm.x * pp.pc.iwx2[iw], BoOm.y * pp.pc.iwx2[iw]) : make_double2(0.0, 0.0);
+            double2 S = m ? make_double2(Om.x * pp.pc.iwx2[iw], Om.y * pp.pc.iwx2[iw]) : make_double2(0.0, 0.0);
             const bool need2 = !m && delwr > pp.to1;
             if (__ballot(need2)) {
                 if (need2) {
                     const double2 z = make_double2(delw.x + 0.5, delw.y);
-                    const double sc = -0.25 * rcp_fast<kSteps>(z.x * z.x + z.y * z.y);
-                    const double2 v = cmul(Boie, cmul(delw, cconj(z)));
+                    const double sc = -0.25 * rcp_cubic(z.x * z.x + z.y * z.y);
+                    const double2 v = cmul(ie, cmul(delw, cconj(z)));
                     S = make_double2(sc * v.x, sc * v.y);
                 }
             }
-            if constexpr (HOIST) {
-                if (live) sasx[q] = cadd(sasx[q], S);
-            } else {
-                const double2 u = cmul(Bo, S);
-                if (live) sasx[q] = cadd(sasx[q], u);
-            }
+            const double2 u = cmul(Bo, S);
+            if (live) sasx[q] = cadd(sasx[q], u);
         }
     }
 }

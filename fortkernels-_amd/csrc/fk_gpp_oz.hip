@@ -530,387 +530,170 @@ __global__ __launch_bounds__(768, 1) void gpp_oz_gemm_kernel(GemmArgs a, int til
 
 // ---------------------------------------------------------------------------
 // Pole/SX epilogue over every (my_igp, ig): B from bmat, Bo = sum over the
-// occupied bands in FP64, then the FP64 pole and SX factors.  Workgroup b
-// takes row my_igp = b / chunks and the (b % chunks)-th of its columns, in
-// blocks of kPoleCols, kPoleK columns per thread (tid, tid + 256, ...).  For
-// each block it loads the elements once, forms the per-element products
-// (B I_eps, Bo Omega2, Bo I_eps) once, and keeps them in registers across
-// the frequency passes;
-// a pass takes up to 4 frequencies (nw split into ceil(nw / 4) passes of
-// near-equal width, so no frequency slot is evaluated for nothing).  The
-// occupied coefficients of the row are staged in LDS.  One partial per
-// workgroup and frequency, summed in a fixed order (over the threads per
-// block, then over the blocks).
+// occupied bands in FP64, then the pole and SX factors in FP64 (pole_terms).
+// A workgroup takes R rows my_igp and a run of their columns, one column of
+// all R rows per thread and iteration: the R rows' loads are independent (R
+// times the bytes in flight of a wave that takes one row), the occupied bands'
+// aqsn values are loaded and widened once for R rows, and the rows'
+// coefficients are uniform loads.  All W >= nw frequencies of a thread's
+// elements are summed in registers, over the workgroup once at the end: one
+// partial per workgroup and frequency, a fixed order.
+//
+// W is the kernel's class, 4, 8, 12 or 16 frequencies (exact for a single call
+// of up to 4): 8 W registers of sums decide how many waves fit, so a kernel
+// for every nw would run all at the occupancy of 16.
 // ---------------------------------------------------------------------------
-#ifndef FK_POLE_K
-#define FK_POLE_K 2
-#endif
-constexpr int kPoleK = FK_POLE_K;             // columns per thread
-constexpr int kPoleCols = 256 * kPoleK;       // columns per workgroup
-constexpr int kOccLds = 64;                   // occupied coefficients staged in LDS
+constexpr int oz_class(int nw) { return (nw - 1) / 4; }
+constexpr int pole_rows(int W) { return W <= 8 ? 4 : 2; }
+// waves per SIMD that the kernels are held to: 128, 168 and 256 registers
+constexpr int pole_waves(int W) { return W <= 4 ? 4 : W <= 8 ? 3 : 2; }
 
 struct PoleArgs {
     const double2 *bmat;     // [ldm][ldn] B
     const double2 *c_occ;    // [nv][ldm]
     const float2 *aqsn, *I_eps, *wtilde;
     const int *igp;
-    double2 *partials;       // [G * chunks][nw][2]
-    double2 *achs_part;      // [G * chunks] static-CH remainder, or NULL
+    double2 *partials;       // [blocks][nw][2]
+    double2 *achs_part;      // [blocks] static-CH remainder, or NULL
     int nv, C, G, ldm, ldn, chunks;
     PoleParams pp;
 };
 
-// LDS of the STREAM form (occupied coefficients, per-wave sums) and of a
-// kernel with the BLOCKS form as well (plus the per-block sums)
-struct StreamLds {
-    double2 occ[kOccLds];
-    double red[4][16];
-};
+// Workgroups per group of rows: runs of at most 16 iterations of 256 columns,
+// shorter where the rows alone give fewer than about 8 workgroups per CU.
+inline int pole_chunks(int G, int C, int nw)
+{
+    const int iters = div_up(C, 256), groups = div_up(G, pole_rows(4 * oz_class(nw) + 4));
+    return std::min(iters, std::max(div_up(iters, 16), div_up(2048, groups)));
+}
+inline int pole_blocks(int G, int C, int nw)
+{
+    return div_up(G, pole_rows(4 * oz_class(nw) + 4)) * pole_chunks(G, C, nw);
+}
+
+template <int W>
 struct PoleLds {
-    double2 occ[kOccLds];
-    double red[4][16];
-    double val[16][256];     // [value][thread] of a workgroup sum
-    double part[16][16];
+    double buf[4][8 * 65];
+    double red[4][4 * W + 2];
 };
 
-// Workgroup sum of V <= 16 values per thread, once per workgroup: each
-// wave's sum (fixed butterfly), then the four waves in order.  Thread q < V
-// returns the total of value q.
-template <int V>
-__device__ __forceinline__ double wave_block_sum(const double (&v)[V], double (&red)[4][16])
+template <int W, bool ALL, bool ACHS>
+__device__ __forceinline__ void oz_pole_block(const PoleArgs &a, int b, PoleLds<W> &L)
 {
+    constexpr int R = pole_rows(W);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-#pragma unroll
-    for (int q = 0; q < V; ++q) {
-        const double x = wave_sum(v[q]);
-        if (lane == 0) red[wave][q] = x;
-    }
-    __syncthreads();
-    double x = 0.0;
-    if (tid < V) x = ((red[0][tid] + red[1][tid]) + red[2][tid]) + red[3][tid];
-    return x;
-}
-
-// Fixed-order workgroup sum of V values per thread: 16 partial sums per
-// value over threads s, s + 16, ..., s + 240, then their sum.  Thread q < V
-// returns the total of value q.  Two barriers; L.val and L.part may be
-// reused after the call.
-template <int V>
-__device__ __forceinline__ double block_sum(const double (&v)[V], PoleLds &L)
-{
-    const int tid = threadIdx.x;
-#pragma unroll
-    for (int q = 0; q < V; ++q) L.val[q][tid] = v[q];
-    __syncthreads();
-    if (tid < 16 * V) {
-        const int q = tid >> 4, s = tid & 15;
-        double x = 0.0;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) x += L.val[q][s + 16 * j];
-        L.part[q][s] = x;
-    }
-    __syncthreads();
-    double x = 0.0;
-    if (tid < V) {
-#pragma unroll
-        for (int s = 0; s < 16; ++s) x += L.part[tid][s];
-    }
-    return x;
-}
-
-// The W frequencies wq[0..W-1] of one element: the per-frequency steps of
-// pole_element's hoisted form, every frequency live.
-//
-// The fast path forms delw with shorter numerators and |delw|^2 as
-// |wtilde|^2 / |wdiff|^2 (equal to the reference's delw.x^2 + delw.y^2 up to
-// rounding, a few 1e-15 relative with the one-step reciprocal).  Every point
-// whose |delw|^2 falls within 1e-13 of a branch threshold is evaluated again
-// in the reference's order with the IEEE quotient, so every branch decision
-// is the reference's; |wdiff|^2, which the mask compares with limittwo, is
-// always the reference's (contraction off).  Both conditional blocks are
-// plain divergent branches, skipped when no lane of the wave takes them (a
-// ballot in front of them adds two vector instructions per frequency).
-template <int W>
-__device__ __forceinline__ void pole_freqs(const PoleParams &pp, const double (&wq)[W], const double (&iq)[W],
-                                           double2 wt, double2 Bie, double2 BoOm, double2 Boie, bool want_ssx,
-                                           double2 (&sach)[W], double2 (&sasx)[W])
-{
-    const double tol1 = 1e-13 * pp.limitone, tol2 = 1e-13 * pp.to1;
-    double wy2;
-    {
-#pragma clang fp contract(off)
-        wy2 = wt.y * wt.y;                   // wdi^2, as the reference rounds it
-    }
-    const double wt2 = __builtin_fma(wt.x, wt.x, wy2);
-#pragma unroll
-    for (int q = 0; q < W; ++q) {
-        const double wdr = wq[q] - wt.x;
-        double wdiffr;
-        {
-#pragma clang fp contract(off)
-            wdiffr = wdr * wdr + wy2;        // = pole_wdiffr(wdr, -wt.y)
-        }
-        const double rden = rcp_fast<1>(wdiffr);
-        // numerators wt.x wdr - wdi^2 and wt.y (wt.x + wdr) = wt.y wx
-        double2 delw = make_double2(__builtin_fma(wt.x, wdr, -wy2) * rden, wt.y * wq[q] * rden);
-        double delwr = wt2 * rden;
-        const bool near = (int)(fabs(delwr - pp.limitone) <= tol1) | (int)(fabs(delwr - pp.to1) <= tol2);
-        if (near) pole_delw(wt, wdr, 1.0 / wdiffr, delw, delwr);
-        const bool m = (wdiffr > pp.limittwo) && (delwr < pp.limitone);
-        const double2 t = (m || !pp.mask_on) ? cmul(Bie, delw) : make_double2(0.0, 0.0);
-        sach[q] = cadd(sach[q], t);
-        if (want_ssx) {
-            // mask branch: Bo Omega2 / wx^2, added through a selected factor
-            // (Bo Omega2 is finite, so a zero factor adds an exact zero)
-            const double f = m ? iq[q] : 0.0;
-            sasx[q].x = __builtin_fma(BoOm.x, f, sasx[q].x);
-            sasx[q].y = __builtin_fma(BoOm.y, f, sasx[q].y);
-            if (!m && delwr > pp.to1) {
-                const double2 z = make_double2(delw.x + 0.5, delw.y);
-                const double sc = -0.25 * rcp_fast<1>(z.x * z.x + z.y * z.y);
-                const double2 v = cmul(Boie, cmul(delw, cconj(z)));
-                sasx[q].x = __builtin_fma(sc, v.x, sasx[q].x);
-                sasx[q].y = __builtin_fma(sc, v.y, sasx[q].y);
-            }
-        }
-    }
-}
-
-struct PoleElems {
-    double2 wt[kPoleK], Bie[kPoleK], BoOm[kPoleK], Boie[kPoleK];
-};
-
-// The W frequencies w0 .. w0 + W - 1 of the current column block's
-// elements, added to this thread's sums
-template <int W>
-__device__ __forceinline__ void oz_pole_freqs(const PoleArgs &a, int w0, bool want_ssx, const PoleElems &E,
-                                              double2 (&sach)[W], double2 (&sasx)[W])
-{
-    double wq[W], iq[W];
-#pragma unroll
-    for (int q = 0; q < W; ++q) {
-        wq[q] = a.pp.pc.wx[w0 + q];
-        iq[q] = a.pp.pc.iwx2[w0 + q];
-    }
-#pragma unroll
-    for (int e = 0; e < kPoleK; ++e)
-        pole_freqs<W>(a.pp, wq, iq, E.wt[e], E.Bie[e], E.BoOm[e], E.Boie[e], want_ssx, sach, sasx);
-}
-
-// workgroup total of the thread sums; thread q < 4 W returns value q
-// (frequency q / 4; component q % 4: achtemp re, im, asxtemp re, im)
-template <int W>
-__device__ __forceinline__ double oz_pole_total(const double2 (&sach)[W], const double2 (&sasx)[W], PoleLds &L)
-{
-    double v[4 * W];
-#pragma unroll
-    for (int q = 0; q < W; ++q) {
-        v[4 * q + 0] = sach[q].x;
-        v[4 * q + 1] = sach[q].y;
-        v[4 * q + 2] = sasx[q].x;
-        v[4 * q + 3] = sasx[q].y;
-    }
-    return block_sum<4 * W>(v, L);
-}
-
-// One column block of row m: loads first (all independent), then Bo, then
-// the products every pass uses.  Columns past c_hi and skipped rows are
-// dead elements: B = Bo = 0 with wtilde = i, so every quotient is finite
-// (|wdiff|^2 >= 1) and every term they add is zero.
-template <bool ACHS>
-__device__ __forceinline__ void oz_pole_elems(const PoleArgs &a, const PoleLds &L, int m, bool ok, bool want_ssx,
-                                              int c0, int c_hi, PoleElems &E, double2 &sachs)
-{
-    const int tid = threadIdx.x;
-    const double2 *brow = a.bmat + (size_t)m * a.ldn;
-    const float2 *wrow = a.wtilde + (size_t)m * a.C, *erow = a.I_eps + (size_t)m * a.C;
-    bool live[kPoleK];
-    double2 B[kPoleK], wt[kPoleK], ie[kPoleK], Bo[kPoleK];
-#pragma unroll
-    for (int e = 0; e < kPoleK; ++e) {
-        const int ig = c0 + e * 256 + tid;
-        live[e] = ok && ig < c_hi;
-        B[e] = live[e] ? brow[ig] : make_double2(0.0, 0.0);
-        wt[e] = live[e] ? widen(wrow[ig]) : make_double2(0.0, 1.0);
-        ie[e] = live[e] ? widen(erow[ig]) : make_double2(0.0, 0.0);
-        Bo[e] = make_double2(0.0, 0.0);
-    }
-    if (ok && want_ssx) {
-        for (int n1 = 0; n1 < a.nv; ++n1) {
-            const double2 co = n1 < kOccLds ? L.occ[n1] : a.c_occ[(size_t)n1 * a.ldm + m];
-            const float2 *arow = a.aqsn + (size_t)n1 * a.C;
-#pragma unroll
-            for (int e = 0; e < kPoleK; ++e) {
-                const int ig = c0 + e * 256 + tid;
-                const double2 x = live[e] ? widen(arow[ig]) : make_double2(0.0, 0.0);
-                Bo[e] = cadd(Bo[e], cmul(co, x));
-            }
-        }
-    }
-#pragma unroll
-    for (int e = 0; e < kPoleK; ++e) {
-        const double2 Om = cmul(cmul(wt[e], wt[e]), ie[e]);
-        E.wt[e] = wt[e];
-        E.Bie[e] = cmul(B[e], ie[e]);
-        E.BoOm[e] = cmul(Bo[e], Om);
-        E.Boie[e] = cmul(Bo[e], ie[e]);
-        // static-CH remainder -sum B I_eps (gppkernel.deslippe.09.30.2014.f90:192-230)
-        if constexpr (ACHS) sachs = csub(sachs, E.Bie[e]);
-    }
-}
-
-// nw <= 4 (one pass): the chunk's columns one element per thread and
-// iteration, each element's products formed and used at once (few live
-// registers, so many waves hide the loads); the thread sums are summed
-// over the workgroup once
-template <int W, bool ACHS, class LDS>
-__device__ __forceinline__ void oz_pole_stream(const PoleArgs &a, LDS &L, int b, int m, bool ok,
-                                               bool want_ssx, int c_lo, int c_hi, double2 &sachs)
-{
-    double wq[W], iq[W];
-#pragma unroll
-    for (int q = 0; q < W; ++q) {
-        wq[q] = a.pp.pc.wx[q];
-        iq[q] = a.pp.pc.iwx2[q];
-    }
-    double2 sach[W], sasx[W];
-#pragma unroll
-    for (int q = 0; q < W; ++q) { sach[q] = make_double2(0.0, 0.0); sasx[q] = make_double2(0.0, 0.0); }
-    const int tid = threadIdx.x;
-    if (ok) {
-        const double2 *brow = a.bmat + (size_t)m * a.ldn;
-        const float2 *wrow = a.wtilde + (size_t)m * a.C, *erow = a.I_eps + (size_t)m * a.C;
-        const int nvl = min(a.nv, kOccLds);
-        for (int ig = c_lo + tid; ig < c_hi; ig += 256) {
-            const double2 B = brow[ig];
-            const double2 wt = widen(wrow[ig]), ie = widen(erow[ig]);
-            double2 Bo = make_double2(0.0, 0.0);
-            for (int n1 = 0; n1 < nvl; ++n1) Bo = cadd(Bo, cmul(L.occ[n1], widen(a.aqsn[(size_t)n1 * a.C + ig])));
-            for (int n1 = nvl; n1 < a.nv; ++n1)
-                Bo = cadd(Bo, cmul(a.c_occ[(size_t)n1 * a.ldm + m], widen(a.aqsn[(size_t)n1 * a.C + ig])));
-            const double2 Om = cmul(cmul(wt, wt), ie);
-            const double2 Bie = cmul(B, ie);
-            pole_freqs<W>(a.pp, wq, iq, wt, Bie, cmul(Bo, Om), cmul(Bo, ie), want_ssx, sach, sasx);
-            // static-CH remainder -sum B I_eps (gppkernel.deslippe.09.30.2014.f90:192-230)
-            if constexpr (ACHS) sachs = csub(sachs, Bie);
-        }
-    }
-    double v[4 * W];
-#pragma unroll
-    for (int q = 0; q < W; ++q) {
-        v[4 * q + 0] = sach[q].x;
-        v[4 * q + 1] = sach[q].y;
-        v[4 * q + 2] = sasx[q].x;
-        v[4 * q + 3] = sasx[q].y;
-    }
-    const double x = wave_block_sum<4 * W>(v, L.red);
-    if (tid < 4 * W) reinterpret_cast<double *>(a.partials + ((size_t)b * W + (tid >> 2)) * 2)[tid & 3] = x;
-}
-
-// nw > 4: per block, each pass's sums are summed over the workgroup and
-// added to the thread that owns them (thread q < 4 W of pass p: own[p])
-template <int W>
-__device__ __forceinline__ void oz_pole_pass(const PoleArgs &a, int w0, bool want_ssx, const PoleElems &E,
-                                             PoleLds &L, double &own)
-{
-    double2 sach[W], sasx[W];
-#pragma unroll
-    for (int q = 0; q < W; ++q) { sach[q] = make_double2(0.0, 0.0); sasx[q] = make_double2(0.0, 0.0); }
-    oz_pole_freqs<W>(a, w0, want_ssx, E, sach, sasx);
-    own += oz_pole_total<W>(sach, sasx, L);
-}
-
-// workgroup b of the problem's launch: row b / chunks, the (b % chunks)-th
-// of the row's columns.  Forms: STREAM for nw <= 4, BLOCKS (blocks of
-// kPoleCols, near-equal passes) for nw > 4; a kernel built with both picks
-// by nw.
-constexpr int kPoleStream = 1, kPoleBlocks = 2;
-template <bool ACHS, int FORMS, class LDS>
-__device__ __forceinline__ void oz_pole_body(const PoleArgs &a, int b, LDS &L)
-{
-    const int tid = threadIdx.x;
-    const int m = __builtin_amdgcn_readfirstlane(b / a.chunks);
-    const int ch = __builtin_amdgcn_readfirstlane(b - m * a.chunks);
-    const int c_lo = (int)((int64_t)ch * a.C / a.chunks), c_hi = (int)((int64_t)(ch + 1) * a.C / a.chunks);
-    const bool ok = a.igp[m] >= 0;
+    const int mg = __builtin_amdgcn_readfirstlane(b / a.chunks);
+    const int ch = __builtin_amdgcn_readfirstlane(b - mg * a.chunks);
+    const int iters = (a.C + 255) / 256, m0 = mg * R;
+    const int c_lo = 256 * (int)((int64_t)ch * iters / a.chunks);
+    const int c_hi = min(256 * (int)((int64_t)(ch + 1) * iters / a.chunks), a.C);
     const bool want_ssx = a.nv > 0;
-    const int nvl = min(a.nv, kOccLds);
-    for (int n1 = tid; n1 < nvl; n1 += 256) L.occ[n1] = a.c_occ[(size_t)n1 * a.ldm + m];
-    __syncthreads();
-    const int nw = a.pp.nw, passes = (nw + 3) / 4;
-    double2 sachs = make_double2(0.0, 0.0);
-
-    if ((FORMS & kPoleStream) && ((FORMS & kPoleBlocks) == 0 || nw <= 4)) {
-        switch (nw) {
-        case 1: oz_pole_stream<1, ACHS>(a, L, b, m, ok, want_ssx, c_lo, c_hi, sachs); break;
-        case 2: oz_pole_stream<2, ACHS>(a, L, b, m, ok, want_ssx, c_lo, c_hi, sachs); break;
-        case 3: oz_pole_stream<3, ACHS>(a, L, b, m, ok, want_ssx, c_lo, c_hi, sachs); break;
-        default: oz_pole_stream<4, ACHS>(a, L, b, m, ok, want_ssx, c_lo, c_hi, sachs); break;
+    // coefficients of the rows' occupied bands: uniform, read-only here (the
+    // rows of c_occ are padded to ldm, a multiple of R)
+    typedef const __attribute__((address_space(4))) double cdbl;
+    cdbl *occ = (cdbl *)(const double *)(a.c_occ + m0);
+    bool ok[R];
+    size_t row[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        row[r] = (size_t)min(m0 + r, a.G - 1);
+        ok[r] = m0 + r < a.G && __builtin_amdgcn_readfirstlane(a.igp[row[r]]) >= 0;
+    }
+    double2 sach[W], sasx[W], sachs = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int q = 0; q < W; ++q) { sach[q] = make_double2(0.0, 0.0); sasx[q] = make_double2(0.0, 0.0); }
+    for (int ig = c_lo + tid; ig < c_hi; ig += 256) {
+        double2 B[R], Bo[R];
+        float2 wt[R], ie[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            B[r] = a.bmat[row[r] * a.ldn + ig];
+            wt[r] = a.wtilde[row[r] * a.C + ig];
+            ie[r] = a.I_eps[row[r] * a.C + ig];
+            Bo[r] = make_double2(0.0, 0.0);
         }
-    } else if constexpr ((FORMS & kPoleBlocks) != 0) {
-        double own[4] = {0.0, 0.0, 0.0, 0.0};     // this thread's totals, one per pass
-        for (int c0 = c_lo; c0 < c_hi; c0 += kPoleCols) {
-            PoleElems E;
-            oz_pole_elems<ACHS>(a, L, m, ok, want_ssx, c0, c_hi, E, sachs);
-            for (int p = 0, w0 = 0; p < passes; ++p) {
-                const int W = (nw - w0 + (passes - p) - 1) / (passes - p);
-                switch (W) {
-                case 1: oz_pole_pass<1>(a, w0, want_ssx, E, L, own[p]); break;
-                case 2: oz_pole_pass<2>(a, w0, want_ssx, E, L, own[p]); break;
-                case 3: oz_pole_pass<3>(a, w0, want_ssx, E, L, own[p]); break;
-                default: oz_pole_pass<4>(a, w0, want_ssx, E, L, own[p]); break;
-                }
-                w0 += W;
+        for (int n1 = 0; n1 < a.nv; ++n1) {
+            const double2 x = widen(a.aqsn[(size_t)n1 * a.C + ig]);
+            cdbl *co = occ + (size_t)n1 * a.ldm * 2;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                Bo[r].x = __builtin_fma(co[2 * r], x.x, __builtin_fma(-co[2 * r + 1], x.y, Bo[r].x));
+                Bo[r].y = __builtin_fma(co[2 * r], x.y, __builtin_fma(co[2 * r + 1], x.x, Bo[r].y));
             }
         }
-        for (int p = 0, w0 = 0; p < passes; ++p) {
-            const int W = (nw - w0 + (passes - p) - 1) / (passes - p);
-            if (tid < 4 * W) {
-                const int q = tid >> 2, comp = tid & 3;
-                reinterpret_cast<double *>(a.partials + ((size_t)b * nw + w0 + q) * 2)[comp] = own[p];
-            }
-            w0 += W;
+        unsigned general = 0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (!ok[r]) continue;
+            if (!pole_terms<W, ALL>(a.pp, 0, widen(wt[r]), widen(ie[r]), B[r], Bo[r], want_ssx, sach, sasx))
+                general |= 1u << r;
+            // static-CH remainder -sum B I_eps (gppkernel.deslippe.09.30.2014.f90:192-230)
+            if constexpr (ACHS) sachs = csub(sachs, cmul(B[r], widen(ie[r])));
         }
+        // the elements pole_terms left out (hardly ever any), one at a time
+        if (__ballot(general != 0)) {
+#pragma unroll 1
+            for (int r = 0; r < R; ++r) {
+                if (!((general >> r) & 1u)) continue;
+                const size_t m = (size_t)(m0 + r);
+                double2 o = make_double2(0.0, 0.0);
+                for (int n1 = 0; n1 < a.nv; ++n1)
+                    o = cfma(o, a.c_occ[(size_t)n1 * a.ldm + m], widen(a.aqsn[(size_t)n1 * a.C + ig]));
+                pole_element<W>(a.pp, 0, true, widen(a.wtilde[m * a.C + ig]), widen(a.I_eps[m * a.C + ig]),
+                                a.bmat[m * a.ldn + ig], o, want_ssx, sach, sasx);
+            }
+        }
+    }
+    // sums over the wave, two frequencies at a time, then over the waves
+#pragma unroll
+    for (int q = 0; q < W; q += 2) {
+        constexpr int kNone = W - 1;
+        const int q1 = q + 1 < W ? q + 1 : kNone;
+        const double v[8] = {sach[q].x, sach[q].y, sasx[q].x, sasx[q].y, sach[q1].x, sach[q1].y, sasx[q1].x, sasx[q1].y};
+        const double x = wave_sums_lds(v, lane, L.buf[wave]);
+        if (lane < (q + 1 < W ? 8 : 4)) L.red[wave][4 * q + lane] = x;
     }
     if constexpr (ACHS) {
-        __syncthreads();     // L.red is free again
-        const double v[2] = {sachs.x, sachs.y};
-        const double x = wave_block_sum<2>(v, L.red);
-        if (tid < 2) reinterpret_cast<double *>(a.achs_part + b)[tid] = x;
+        const double v0 = wave_sum(sachs.x), v1 = wave_sum(sachs.y);
+        if (lane == 0) {
+            L.red[wave][4 * W] = v0;
+            L.red[wave][4 * W + 1] = v1;
+        }
+    }
+    __syncthreads();
+    const int nw = ALL ? W : a.pp.nw;
+    if (tid < 4 * nw)
+        reinterpret_cast<double *>(a.partials + (size_t)b * nw * 2)[tid] =
+            ((L.red[0][tid] + L.red[1][tid]) + L.red[2][tid]) + L.red[3][tid];
+    if (ACHS && tid >= 128 && tid < 130) {
+        const int k = 4 * W + tid - 128;
+        reinterpret_cast<double *>(a.achs_part + b)[tid - 128] = ((L.red[0][k] + L.red[1][k]) + L.red[2][k]) + L.red[3][k];
     }
 }
 
-template <bool ACHS, int FORMS>
-__device__ __forceinline__ void oz_pole_block(const PoleArgs &a, int b)
+template <int W, bool ALL, bool ACHS>
+__global__ __launch_bounds__(256, pole_waves(W)) void gpp_oz_pole_kernel(PoleArgs a)
 {
-    if constexpr (FORMS == kPoleStream) {
-        __shared__ StreamLds L;
-        oz_pole_body<ACHS, FORMS>(a, b, L);
-    } else {
-        __shared__ PoleLds L;
-        oz_pole_body<ACHS, FORMS>(a, b, L);
+    __shared__ PoleLds<W> L;
+    oz_pole_block<W, ALL, ACHS>(a, blockIdx.x, L);
+}
+
+template <bool ACHS>
+void launch_pole(int blocks, hipStream_t s, const PoleArgs &a)
+{
+    switch (a.pp.nw) {
+    case 1: hipLaunchKernelGGL((gpp_oz_pole_kernel<1, true, ACHS>), dim3(blocks), dim3(256), 0, s, a); break;
+    case 2: hipLaunchKernelGGL((gpp_oz_pole_kernel<2, true, ACHS>), dim3(blocks), dim3(256), 0, s, a); break;
+    case 3: hipLaunchKernelGGL((gpp_oz_pole_kernel<3, true, ACHS>), dim3(blocks), dim3(256), 0, s, a); break;
+    case 4: hipLaunchKernelGGL((gpp_oz_pole_kernel<4, true, ACHS>), dim3(blocks), dim3(256), 0, s, a); break;
+    default:
+        switch (oz_class(a.pp.nw)) {
+        case 1: hipLaunchKernelGGL((gpp_oz_pole_kernel<8, false, ACHS>), dim3(blocks), dim3(256), 0, s, a); break;
+        case 2: hipLaunchKernelGGL((gpp_oz_pole_kernel<12, false, ACHS>), dim3(blocks), dim3(256), 0, s, a); break;
+        default: hipLaunchKernelGGL((gpp_oz_pole_kernel<16, false, ACHS>), dim3(blocks), dim3(256), 0, s, a); break;
+        }
     }
 }
-
-// Occupancy the pole kernels are held to: 5 waves per SIMD (<= 96 VGPRs)
-// for the stream form, 4 (<= 128) for a kernel with the blocks form.  To fit,
-// the compiler spills a few registers (1 to 12 a lane) in the set-up and at
-// block boundaries, outside the frequency loop; left free, it takes a few
-// registers more and loses a wave, which measured slower.
-constexpr int pole_waves(int forms) { return forms == kPoleStream ? 5 : 4; }
-
-template <bool ACHS, int FORMS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(pole_waves(FORMS))))
-void gpp_oz_pole_kernel(PoleArgs a)
-{
-    oz_pole_block<ACHS, FORMS>(a, blockIdx.x);
-}
-
-// column chunks of a row in the pole kernel (one workgroup each)
-#ifndef FK_POLE_CHUNKS
-#define FK_POLE_CHUNKS 4
-#endif
-inline int pole_chunks(int C) { return std::min(FK_POLE_CHUNKS, div_up(C, kPoleCols)); }
 
 // ---------------------------------------------------------------------------
 // Batches: one launch of each kernel above for many problems.  Every
@@ -970,13 +753,16 @@ __global__ __launch_bounds__(768, 1) void gpp_oz_gemm_batch_kernel(const OzRecor
     }
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(pole_waves(kPoleStream | kPoleBlocks))))
-void gpp_oz_pole_batch_kernel(const OzRecord *rec, const int *first, int n)
+// The problems of one frequency class (first: no blocks for the others).  The
+// arguments by reference: a register copy of them (with the pole parameters of
+// up to 16 frequencies) made this kernel 1.7x slower.
+template <int W>
+__global__ __launch_bounds__(256, pole_waves(W)) void gpp_oz_pole_batch_kernel(const OzRecord *__restrict__ rec,
+                                                                               const int *first, int n)
 {
+    __shared__ PoleLds<W> L;
     const int b = (int)blockIdx.x, p = batch_problem(first, n, b);
-    // by reference: a register copy of the arguments (with the pole
-    // parameters of up to 16 frequencies) made this kernel 1.7x slower
-    oz_pole_block<false, kPoleStream | kPoleBlocks>(rec[p].pa, b - first[p]);
+    oz_pole_block<W, false, false>(rec[p].pa, b - first[p], L);
 }
 
 }  // namespace
@@ -1009,7 +795,7 @@ OzBlocks gpp_oz_batch_record(const fk_gpp_problem *p, const fk_options *o, const
     pa.partials = static_cast<double2 *>(ws.at(L.off_part));
     pa.achs_part = nullptr;
     pa.nv = p->nvband; pa.C = p->ncouls; pa.G = p->ngpown; pa.ldm = L.ldm; pa.ldn = L.ldn;
-    pa.chunks = pole_chunks(p->ncouls);
+    pa.chunks = pole_chunks(p->ngpown, p->ncouls, p->nfreq);
     pa.pp = make_pole_params(p->wx, p->nfreq, p->limittwo, p->limitone, p->to1, o->mask != 0);
     r.gemm_tiles = L.tiles_m * L.tiles_n;
     std::memcpy(record, &r, sizeof(r));
@@ -1017,12 +803,13 @@ OzBlocks gpp_oz_batch_record(const fk_gpp_problem *p, const fk_options *o, const
     const bool any = p->number_bands > 0;
     nb.prep = any ? L.ldm / kPrepRowsA + L.ldn / kPrepColsB : 0;
     nb.gemm = any ? div_up(r.gemm_tiles, kXcds) * kXcds : 0;
-    nb.pole = any ? p->ngpown * pa.chunks : 0;
+    nb.pole = any ? pole_blocks(p->ngpown, p->ncouls, p->nfreq) : 0;
+    nb.pole_class = oz_class(p->nfreq);
     return nb;
 }
 
 int gpp_oz_batch_launch(const void *records, const int *first_prep, const int *first_gemm, const int *first_pole,
-                        int n, int total_prep, int total_gemm, int total_pole, hipStream_t s)
+                        int n, int total_prep, int total_gemm, const int *total_pole, hipStream_t s)
 {
     const OzRecord *rec = static_cast<const OzRecord *>(records);
     if (total_prep > 0)
@@ -1034,8 +821,17 @@ int gpp_oz_batch_launch(const void *records, const int *first_prep, const int *f
         const int grid = std::max(1, std::min(total_gemm, ncu));
         hipLaunchKernelGGL(gpp_oz_gemm_batch_kernel, dim3(grid), dim3(kWaves12 * 64), 0, s, rec, first_gemm, n);
     }
-    if (total_pole > 0)
-        hipLaunchKernelGGL(gpp_oz_pole_batch_kernel, dim3(total_pole), dim3(256), 0, s, rec, first_pole, n);
+    for (int c = 0; c < kOzPoleClasses; ++c) {
+        if (total_pole[c] <= 0) continue;
+        const dim3 grid(total_pole[c]), block(256);
+        const int *first = first_pole + c * (n + 1);
+        switch (c) {
+        case 0: hipLaunchKernelGGL(gpp_oz_pole_batch_kernel<4>, grid, block, 0, s, rec, first, n); break;
+        case 1: hipLaunchKernelGGL(gpp_oz_pole_batch_kernel<8>, grid, block, 0, s, rec, first, n); break;
+        case 2: hipLaunchKernelGGL(gpp_oz_pole_batch_kernel<12>, grid, block, 0, s, rec, first, n); break;
+        default: hipLaunchKernelGGL(gpp_oz_pole_batch_kernel<16>, grid, block, 0, s, rec, first, n); break;
+        }
+    }
     FK_HIP(hipGetLastError());
     return FK_OK;
 }
@@ -1054,8 +850,9 @@ void gpp_oz_plan(const fk_gpp_problem *p, Scratch &ws, OzLayout &L)
     L.off_eb = ws.plan(sizeof(double) * kProds * (size_t)L.ldn);
     L.off_cocc = ws.plan(sizeof(double2) * (size_t)std::max(p->nvband, 1) * L.ldm);
     L.off_bmat = ws.plan(sizeof(double2) * (size_t)L.ldm * L.ldn);
-    L.off_part = ws.plan(sizeof(double2) * 2 * (size_t)p->nfreq * p->ngpown * pole_chunks(p->ncouls));
-    L.off_achs = ws.plan(sizeof(double2) * (size_t)p->ngpown * pole_chunks(p->ncouls));
+    const size_t blocks = (size_t)pole_blocks(p->ngpown, p->ncouls, p->nfreq);
+    L.off_part = ws.plan(sizeof(double2) * 2 * (size_t)p->nfreq * blocks);
+    L.off_achs = ws.plan(sizeof(double2) * blocks);
 }
 
 int gpp_oz_check(const fk_gpp_problem *p)
@@ -1106,16 +903,11 @@ int gpp_oz_launch(const fk_gpp_problem *p, const fk_options *o, const OzLayout &
     pa.partials = static_cast<double2 *>(ws.at(L.off_part));
     pa.achs_part = d_achs ? static_cast<double2 *>(ws.at(L.off_achs)) : nullptr;
     pa.nv = p->nvband; pa.C = p->ncouls; pa.G = p->ngpown; pa.ldm = L.ldm; pa.ldn = L.ldn;
-    pa.chunks = pole_chunks(p->ncouls);
+    pa.chunks = pole_chunks(p->ngpown, p->ncouls, p->nfreq);
     pa.pp = make_pole_params(p->wx, p->nfreq, p->limittwo, p->limitone, p->to1, o->mask != 0);
-    const int blocks = p->ngpown * pa.chunks;
-    if (p->nfreq <= 4) {
-        if (pa.achs_part) hipLaunchKernelGGL((gpp_oz_pole_kernel<true, kPoleStream>), dim3(blocks), dim3(256), 0, s, pa);
-        else hipLaunchKernelGGL((gpp_oz_pole_kernel<false, kPoleStream>), dim3(blocks), dim3(256), 0, s, pa);
-    } else {
-        if (pa.achs_part) hipLaunchKernelGGL((gpp_oz_pole_kernel<true, kPoleBlocks>), dim3(blocks), dim3(256), 0, s, pa);
-        else hipLaunchKernelGGL((gpp_oz_pole_kernel<false, kPoleBlocks>), dim3(blocks), dim3(256), 0, s, pa);
-    }
+    const int blocks = pole_blocks(p->ngpown, p->ncouls, p->nfreq);
+    if (pa.achs_part) launch_pole<true>(blocks, s, pa);
+    else launch_pole<false>(blocks, s, pa);
     FK_HIP(hipGetLastError());
     FK_TRY(gpp_reduce_launch(pa.partials, blocks, p->nfreq, 2.0 * p->occ, d_ach, d_asx, s));
     if (d_achs) FK_TRY(gpp_sum_launch(pa.achs_part, blocks, d_achs, s));
