@@ -599,7 +599,7 @@ __device__ __forceinline__ void gpp_ring_tile(const GppArgs<double2> &a, int tm,
                 if (((rowok >> (i * 4 + r)) & 1u) && col <= nmax) {
                     const double2 Bo = o.value(0, 0, r);
                     const double2 B = cadd(k == 0 ? Bu0[r] : sh.bu[wave][k > 0 ? k - 1 : 0][r][lane], Bo);
-                    if (!pole_terms<NWC, ALL>(a.pp, w0, cwt[r], cie[r], B, Bo, want_ssx, sach, sasx))
+                    if (!pole_terms<NWC, ALL>(a.pp, a.pp.pc.wx, a.pp.pc.iwx2, w0, cwt[r], cie[r], B, Bo, sach, sasx))
                         general |= 1u << (k * 4 + r);
                     if constexpr (ACHS) {
                         if (w0 == 0) sachs = csub(sachs, cmul(B, cie[r]));
@@ -637,8 +637,8 @@ __device__ __forceinline__ void gpp_ring_tile(const GppArgs<double2> &a, int tm,
         for (int q = 0; q < NWC; ++q) {
             v[4 * q + 0] = sach[q].x;
             v[4 * q + 1] = sach[q].y;
-            v[4 * q + 2] = sasx[q].x;
-            v[4 * q + 3] = sasx[q].y;
+            v[4 * q + 2] = want_ssx ? sasx[q].x : 0.0;
+            v[4 * q + 3] = want_ssx ? sasx[q].y : 0.0;
         }
         if (ALL || w0 + NWC >= a.nw) {
             const double x = wave_sums_lds(v, lane, reinterpret_cast<double *>(&sh.bu[wave][0][0][0]));

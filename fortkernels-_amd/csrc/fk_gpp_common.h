@@ -170,11 +170,11 @@ __device__ __forceinline__ double2 cmul_fused(double2 a, double2 b)
 
 // One kept (my_igp, ig) element for the frequencies w0 .. w0+NWC-1 that
 // exist: adds B D to sach[q] and Bo ssx to sasx[q], what pole_element adds, in
-// a third of its operations (25 per frequency).  FP64 vector operations and
+// less than half its operations (27 per frequency).  FP64 vector operations and
 // FP64 MFMAs take turns on the same units here, so the epilogue adds to the
 // MFMA time however well the two are interleaved, and its length is what it
-// costs (512/2/32768/1638, 3 frequencies, same tiles: 3.00 ms with pole_element's
-// operations, 2.89 with these).
+// costs (512/2/32768/1638, 3 frequencies, an earlier form of the ring tiles: 3.00
+// ms with pole_element's operations, 2.89 with these).
 //
 // With u = wx - wtilde and s = wx + wtilde,
 //     D   = I_eps wtilde / u                     where the mask is on,
@@ -191,9 +191,17 @@ __device__ __forceinline__ double2 cmul_fused(double2 a, double2 b)
 // 1.01 to1 limittwo (u = 0, where |delw|^2 is a NaN, adds nothing).  Other
 // elements (|wtilde| outside 5e-4 .. 249 with the default limits, NaNs), and
 // all with the mask off, return false and are left to pole_element.
-template <int NWC, bool ALL>
-__device__ __forceinline__ bool pole_terms(const PoleParams &pp, int w0, double2 wt, double2 ie, double2 B, double2 Bo,
-                                           bool want_ssx, double2 (&sach)[NWC], double2 (&sasx)[NWC])
+//
+// The branches are taken under the execution mask: with selected factors instead
+// (five more operations, no branch) every kernel that uses this is slower, by 7%
+// at 3 frequencies and 20% at 7.
+//
+// Without occupied bands (Bo = 0) the sums of sasx are to be dropped: a 0 / wx^2
+// at wx = 0 leaves a NaN there.
+// wx, iwx2: the frequencies' tables (PoleConst).
+template <int NWC, bool ALL, class Table>
+__device__ __forceinline__ bool pole_terms(const PoleParams &pp, Table wx, Table iwx2, int w0, double2 wt, double2 ie, double2 B,
+                                           double2 Bo, double2 (&sach)[NWC], double2 (&sasx)[NWC])
 {
     // fused operations only where written, so every kernel rounds alike
 #pragma clang fp contract(off)
@@ -202,33 +210,25 @@ __device__ __forceinline__ bool pole_terms(const PoleParams &pp, int w0, double2
     if (!(wt2 > pp.lo && wt2 < pp.hi)) return false;
     const double2 T = cmul_fused(ie, wt), P = cmul_fused(B, T);
     const double2 PQ = make_double2(P.y * wt.y, P.x * wt.y);
-    double2 BoOm = make_double2(0.0, 0.0), R = BoOm, RQ = BoOm;
-    if (want_ssx) {
-        BoOm = cmul_fused(Bo, cmul_fused(T, wt));
-        R = cmul_fused(Bo, make_double2(-0.5 * T.x, -0.5 * T.y));
-        RQ = make_double2(R.y * wt.y, R.x * wt.y);
-    }
+    const double2 BoOm = cmul_fused(Bo, cmul_fused(T, wt));
+    const double2 R = cmul_fused(Bo, make_double2(-0.5 * T.x, -0.5 * T.y));
+    const double2 RQ = make_double2(R.y * wt.y, R.x * wt.y);
 #pragma unroll
     for (int q = 0; q < NWC; ++q) {
         if (!ALL && q > 0 && w0 + q >= pp.nw) break;
-        const double wx = pp.pc.wx[w0 + q];
-        double y = wx - wt.x, d = y * y + wy2;
-        const bool m = d > pp.limittwo, pole = !m && d > 0.0;
-        if (!m) {
-            y = wx + wt.x;
-            d = __builtin_fma(y, y, wy2);
-        }
-        const double r = rcp_cubic(d);
+        const double yu = wx[w0 + q] - wt.x, du = yu * yu + wy2;
+        const double ys = wx[w0 + q] + wt.x, ds = __builtin_fma(ys, ys, wy2);
+        const bool m = du > pp.limittwo;
+        const double r = rcp_cubic(m ? du : ds);
         if (m) {
-            sach[q].x = __builtin_fma(__builtin_fma(P.x, y, -PQ.x), r, sach[q].x);
-            sach[q].y = __builtin_fma(__builtin_fma(P.y, y, PQ.y), r, sach[q].y);
-            if (want_ssx) {
-                sasx[q].x = __builtin_fma(BoOm.x, pp.pc.iwx2[w0 + q], sasx[q].x);
-                sasx[q].y = __builtin_fma(BoOm.y, pp.pc.iwx2[w0 + q], sasx[q].y);
-            }
-        } else if (want_ssx && pole) {
-            sasx[q].x = __builtin_fma(__builtin_fma(R.x, y, RQ.x), r, sasx[q].x);
-            sasx[q].y = __builtin_fma(__builtin_fma(R.y, y, -RQ.y), r, sasx[q].y);
+            sach[q].x = __builtin_fma(__builtin_fma(P.x, yu, -PQ.x), r, sach[q].x);
+            sach[q].y = __builtin_fma(__builtin_fma(P.y, yu, PQ.y), r, sach[q].y);
+            sasx[q].x = __builtin_fma(BoOm.x, iwx2[w0 + q], sasx[q].x);
+            sasx[q].y = __builtin_fma(BoOm.y, iwx2[w0 + q], sasx[q].y);
+        } else {
+            const double rs = du > 0.0 ? r : 0.0;
+            sasx[q].x = __builtin_fma(__builtin_fma(R.x, ys, RQ.x), rs, sasx[q].x);
+            sasx[q].y = __builtin_fma(__builtin_fma(R.y, ys, -RQ.y), rs, sasx[q].y);
         }
     }
     return true;

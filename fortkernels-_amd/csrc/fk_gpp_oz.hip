@@ -44,6 +44,7 @@
 #include "fk_internal.h"
 
 #include <algorithm>
+#include <cstddef>
 #include <cstring>
 #include <type_traits>
 
@@ -539,6 +540,11 @@ __global__ __launch_bounds__(768, 1) void gpp_oz_gemm_kernel(GemmArgs a, int til
 // elements are summed in registers, over the workgroup once at the end: one
 // partial per workgroup and frequency, a fixed order.
 //
+// Measured: 512/2/32768/1638, 3 frequencies 367 us (4.7 TB/s; without the pole
+// terms 300 us, 5.7 TB/s), the form of one row and two quotients 558; a batch of
+// 12 problems of 3 to 11 frequencies 1.50 ms, before 2.65.  Two rows cost the
+// same at 3 frequencies and 8% more at 7, loading one iteration ahead 5% more.
+//
 // W is the kernel's class, 4, 8, 12 or 16 frequencies (exact for a single call
 // of up to 4): 8 W registers of sums decide how many waves fit, so a kernel
 // for every nw would run all at the occupancy of 16.
@@ -577,8 +583,12 @@ struct PoleLds {
     double red[4][4 * W + 2];
 };
 
+// tab: the wx and iwx2 tables of a.pp, read through scalar loads
+typedef const __attribute__((address_space(4))) double cdbl;
+static_assert(offsetof(PoleConst, iwx2) == sizeof(double) * kMaxFreq, "tab + kMaxFreq is iwx2");
+
 template <int W, bool ALL, bool ACHS>
-__device__ __forceinline__ void oz_pole_block(const PoleArgs &a, int b, PoleLds<W> &L)
+__device__ __forceinline__ void oz_pole_block(const PoleArgs &a, cdbl *tab, int b, PoleLds<W> &L)
 {
     constexpr int R = pole_rows(W);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -590,7 +600,6 @@ __device__ __forceinline__ void oz_pole_block(const PoleArgs &a, int b, PoleLds<
     const bool want_ssx = a.nv > 0;
     // coefficients of the rows' occupied bands: uniform, read-only here (the
     // rows of c_occ are padded to ldm, a multiple of R)
-    typedef const __attribute__((address_space(4))) double cdbl;
     cdbl *occ = (cdbl *)(const double *)(a.c_occ + m0);
     bool ok[R];
     size_t row[R];
@@ -625,7 +634,11 @@ __device__ __forceinline__ void oz_pole_block(const PoleArgs &a, int b, PoleLds<
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             if (!ok[r]) continue;
-            if (!pole_terms<W, ALL>(a.pp, 0, widen(wt[r]), widen(ie[r]), B[r], Bo[r], want_ssx, sach, sasx))
+            // past four frequencies the tables are read again for each row:
+            // kept in scalar registers all along they push others out of them
+            // (nw 7: 119 to 150 us at 12000 x 600)
+            if constexpr (W > 4) asm volatile("" : "+s"(tab));
+            if (!pole_terms<W, ALL>(a.pp, tab, tab + kMaxFreq, 0, widen(wt[r]), widen(ie[r]), B[r], Bo[r], sach, sasx))
                 general |= 1u << r;
             // static-CH remainder -sum B I_eps (gppkernel.deslippe.09.30.2014.f90:192-230)
             if constexpr (ACHS) sachs = csub(sachs, cmul(B[r], widen(ie[r])));
@@ -649,7 +662,8 @@ __device__ __forceinline__ void oz_pole_block(const PoleArgs &a, int b, PoleLds<
     for (int q = 0; q < W; q += 2) {
         constexpr int kNone = W - 1;
         const int q1 = q + 1 < W ? q + 1 : kNone;
-        const double v[8] = {sach[q].x, sach[q].y, sasx[q].x, sasx[q].y, sach[q1].x, sach[q1].y, sasx[q1].x, sasx[q1].y};
+        double v[8] = {sach[q].x, sach[q].y, sasx[q].x, sasx[q].y, sach[q1].x, sach[q1].y, sasx[q1].x, sasx[q1].y};
+        if (!want_ssx) v[2] = v[3] = v[6] = v[7] = 0.0;
         const double x = wave_sums_lds(v, lane, L.buf[wave]);
         if (lane < (q + 1 < W ? 8 : 4)) L.red[wave][4 * q + lane] = x;
     }
@@ -675,7 +689,8 @@ template <int W, bool ALL, bool ACHS>
 __global__ __launch_bounds__(256, pole_waves(W)) void gpp_oz_pole_kernel(PoleArgs a)
 {
     __shared__ PoleLds<W> L;
-    oz_pole_block<W, ALL, ACHS>(a, blockIdx.x, L);
+    cdbl *args = (cdbl *)__builtin_amdgcn_kernarg_segment_ptr();   // a is the first argument
+    oz_pole_block<W, ALL, ACHS>(a, args + (offsetof(PoleArgs, pp) + offsetof(PoleParams, pc)) / sizeof(double), blockIdx.x, L);
 }
 
 template <bool ACHS>
@@ -762,7 +777,7 @@ __global__ __launch_bounds__(256, pole_waves(W)) void gpp_oz_pole_batch_kernel(c
 {
     __shared__ PoleLds<W> L;
     const int b = (int)blockIdx.x, p = batch_problem(first, n, b);
-    oz_pole_block<W, false, false>(rec[p].pa, b - first[p], L);
+    oz_pole_block<W, false, false>(rec[p].pa, (cdbl *)&rec[p].pa.pp.pc, b - first[p], L);
 }
 
 }  // namespace
