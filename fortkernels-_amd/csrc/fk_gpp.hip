@@ -486,26 +486,34 @@ __device__ __forceinline__ void gpp_tile(const GppArgs<E> &a, int tm, int tn, Ti
 // ---------------------------------------------------------------------------
 constexpr int kRingStages = 3;
 constexpr int kRingWgs = 3;      // workgroups per CU
+constexpr int kRingSmallWgs = 3; // of the 32 x 32 tiles, at least
 constexpr int kRingOcc = 16;
-constexpr int kRingNwc = 4;      // frequencies per epilogue pass of calls with more than three
+// Frequencies per epilogue pass of calls with more than three: what the registers
+// hold (a batch of 12 problems of 3 to 11 frequencies takes 6.58 ms with 3, 6.42
+// with 4, 6.24 with 5, 6.17 with 6; with the static-CH remainder, 7 frequencies of
+// 333/11/10007/1001, the whole call 978 us with 4, 988 with 5, 1013 with 6).
+constexpr int ring_nwc(int mb, bool achs) { return mb == 2 && achs ? 4 : 6; }
 
-template <int NWC>
+template <int MB, int NWC>
 struct RingLds {
     union {
-        double2 ring[kRingStages][2][8][64];     // [slot][coefficients, aqsn][k][column]
-        double2 bu[4][3][4][64];                 // [wave][block - 1][register][lane]
+        double2 ring[kRingStages][2][8][32 * MB];    // [slot][coefficients, aqsn][k][column]
+        double2 bu[4][MB == 2 ? 3 : 1][4][64];       // [wave][block - 1][register][lane]
+        double sums[4][8 * 65];                      // wave_sums_lds
     };
     double red[4][4 * NWC];
 };
 
-// ALL: nw == NWC, one epilogue pass.
-template <int NWC, bool ALL, bool ACHS, bool TABLE>
-__device__ __forceinline__ void gpp_ring_tile(const GppArgs<double2> &a, int tm, int tn, RingLds<NWC> &sh)
+// MB x MB blocks per wave: 64 x 64 tiles (MB = 2) or 32 x 32.  ALL: nw == NWC,
+// one epilogue pass.
+template <int MB, int NWC, bool ALL, bool ACHS, bool TABLE>
+__device__ __forceinline__ void gpp_ring_tile(const GppArgs<double2> &a, int tm, int tn, RingLds<MB, NWC> &sh)
 {
-    constexpr int MB = 2, NB = 2, NWAVES = 4, LPW = 4;
+    constexpr int NB = MB, T = 32 * MB, NWAVES = 4;
+    constexpr int RPL = 64 / T, LPW = 4 / RPL;       // rows of a direct load, loads of a wave per stage
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave & 1, wn = wave >> 1;
-    const int rowbase = tm * 64 + wm * 32, colbase = tn * 64 + wn * 32;
+    const int rowbase = tm * T + wm * 16 * MB, colbase = tn * T + wn * 16 * NB;
     const int nmax = a.C - 1;
     const int kl = lane >> 4, cl = lane & 15;
     const int nst = (a.nks * 4 - a.nvpad) / 8;       // stages
@@ -516,28 +524,29 @@ __device__ __forceinline__ void gpp_ring_tile(const GppArgs<double2> &a, int tm,
     // clamped band irrelevant, the epilogue drops a clamped column).
     const bool side_a = wave < 2;
     const int k0 = 4 * (wave & 1);
-    const double2 *src = side_a ? a.c + tm * 64 + lane : a.aqsn + min(tn * 64 + lane, nmax);
+    const double2 *src = side_a ? a.c + tm * T + lane % T : a.aqsn + min(tn * T + lane % T, nmax);
     const size_t ld = side_a ? (size_t)a.ldc : (size_t)a.C;
     const int row0 = (side_a ? a.nvpad : a.nv) + k0;
     const int last = side_a ? a.nks * 4 - 1 : a.nb - 1;
     const bool direct = side_a || a.aligned;
     auto issue = [&](int s, int slot) {
-        const int r = row0 + 8 * s;
+        const int r = row0 + 8 * s + lane / T;
         double2 *dst = &sh.ring[slot][side_a ? 0 : 1][k0][0];
+        auto at = [&](int j) { return src + (size_t)min(r + RPL * j, last) * ld; };
         if (direct) {
 #pragma unroll
-            for (int j = 0; j < LPW; ++j) ring::lds_load16(src + (size_t)min(r + j, last) * ld, dst + 64 * j);
+            for (int j = 0; j < LPW; ++j) ring::lds_load16(at(j), dst + 64 * j);
         } else {
 #pragma unroll
-            for (int j = 0; j < LPW; ++j) dst[64 * j + lane] = ring::load16(src + (size_t)min(r + j, last) * ld);
+            for (int j = 0; j < LPW; ++j) dst[64 * j + lane] = ring::load16(at(j));
         }
     };
     auto read = [&](ring::Frags<MB, NB> &f, int, int slot, int q) {
         const double2 *st = &sh.ring[slot][0][4 * q + kl][cl];
 #pragma unroll
-        for (int i = 0; i < MB; ++i) f.a[i] = st[wm * 32 + 16 * i];
+        for (int i = 0; i < MB; ++i) f.a[i] = st[wm * 16 * MB + 16 * i];
 #pragma unroll
-        for (int j = 0; j < NB; ++j) f.b[j] = st[8 * 64 + wn * 32 + 16 * j];
+        for (int j = 0; j < NB; ++j) f.b[j] = st[8 * T + wn * 16 * NB + 16 * j];
     };
     ring::Acc3<MB, NB> acc;
     acc.zero();
@@ -572,14 +581,19 @@ __device__ __forceinline__ void gpp_ring_tile(const GppArgs<double2> &a, int tm,
 #pragma unroll
         for (int q = 0; q < NWC; ++q) { sach[q] = make_double2(0.0, 0.0); sasx[q] = make_double2(0.0, 0.0); }
         unsigned general = 0;
+        // the lane's row and column, opaque in each pass: otherwise the addresses
+        // of its 16 elements are kept in registers across the passes, which
+        // spills 60 others
+        int kp = kl, cp = cl;
+        if constexpr (!ALL) asm volatile("" : "+v"(kp), "+v"(cp));
 #pragma unroll
         for (int k = 0; k < MB * NB; ++k) {
             __builtin_amdgcn_sched_barrier(0);
-            const int i = k / NB, j = k % NB, col = colbase + j * 16 + cl;
+            const int i = k / NB, j = k % NB, col = colbase + j * 16 + cp;
             double2 cwt[4], cie[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int row = rowbase + i * 16 + 4 * r + kl;
+                const int row = rowbase + i * 16 + 4 * r + kp;
                 const size_t e = (size_t)min(row, a.G - 1) * a.C + min(col, nmax);
                 cwt[r] = gld<TABLE>(a.wtilde, e);
                 cie[r] = gld<TABLE>(a.I_eps, e);
@@ -589,8 +603,8 @@ __device__ __forceinline__ void gpp_ring_tile(const GppArgs<double2> &a, int tm,
             o.zero();
             for (int ks = 0; ks < nko; ++ks) {
                 ring::Frags<1, 1> f;
-                f.a[0] = gld<TABLE>(a.c, (size_t)(4 * ks + kl) * a.ldc + rowbase + 16 * i + cl);
-                f.b[0] = gld<TABLE>(a.aqsn, (size_t)min(4 * ks + kl, a.nb - 1) * a.C + min(col, nmax));
+                f.a[0] = gld<TABLE>(a.c, (size_t)(4 * ks + kp) * a.ldc + rowbase + 16 * i + cp);
+                f.b[0] = gld<TABLE>(a.aqsn, (size_t)min(4 * ks + kp, a.nb - 1) * a.C + min(col, nmax));
                 o.mma(f);
             }
 #pragma unroll
@@ -640,9 +654,17 @@ __device__ __forceinline__ void gpp_ring_tile(const GppArgs<double2> &a, int tm,
             v[4 * q + 2] = want_ssx ? sasx[q].x : 0.0;
             v[4 * q + 3] = want_ssx ? sasx[q].y : 0.0;
         }
-        if (ALL || w0 + NWC >= a.nw) {
-            const double x = wave_sums_lds(v, lane, reinterpret_cast<double *>(&sh.bu[wave][0][0][0]));
-            if (lane < 4 * NWC) sh.red[wave][lane] = x;
+        if (MB == 1 || ALL || w0 + NWC >= a.nw) {
+            // each wave in its own part of the ring's memory, eight values at a time
+            double *buf = MB == 1 ? sh.sums[wave] : reinterpret_cast<double *>(&sh.bu[wave][0][0][0]);
+#pragma unroll
+            for (int q = 0; q < 4 * NWC; q += 8) {
+                double u[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) u[k] = q + k < 4 * NWC ? v[q + k < 4 * NWC ? q + k : 0] : 0.0;
+                const double x = wave_sums_lds(u, lane, buf);
+                if (lane < 8 && q + lane < 4 * NWC) sh.red[wave][q + lane] = x;
+            }
         } else {          // Bu stays where it is for the next pass
 #pragma unroll
             for (int q = 0; q < 4 * NWC; ++q) {
@@ -680,10 +702,10 @@ __device__ __forceinline__ void gpp_ring_tile(const GppArgs<double2> &a, int tm,
     }
 }
 
-template <int NWC, bool ALL, bool ACHS>
-__global__ __launch_bounds__(256, kRingWgs) void gpp_ring_kernel(GppArgs<double2> a)
+template <int MB, int NWC, bool ALL, bool ACHS>
+__global__ __launch_bounds__(256, MB == 2 ? kRingWgs : kRingSmallWgs) void gpp_ring_kernel(GppArgs<double2> a)
 {
-    __shared__ RingLds<NWC> sh;
+    __shared__ RingLds<MB, NWC> sh;
     // The second and third workgroup slots of a CU start one and two thirds
     // of a tile late (see gpp_fused_kernel).
     if (a.stagger_ticks && (int)blockIdx.x >= a.stagger_lo && (int)blockIdx.x < kRingWgs * a.stagger_lo) {
@@ -692,7 +714,7 @@ __global__ __launch_bounds__(256, kRingWgs) void gpp_ring_kernel(GppArgs<double2
     }
     int tm, tn;
     tile_coords(blockIdx.x, a.tiles_m, a.tiles_n, a.group_m, tm, tn);
-    gpp_ring_tile<NWC, ALL, ACHS, false>(a, tm, tn, sh);
+    gpp_ring_tile<MB, NWC, ALL, ACHS, false>(a, tm, tn, sh);
 }
 
 // One problem, one tile per workgroup.
@@ -749,7 +771,7 @@ __global__ __launch_bounds__(256, kRingWgs) void gpp_ring_batch_kernel(const Gpp
                                                                        const BatchTile *__restrict__ tiles, int ntiles,
                                                                        int *counter)
 {
-    __shared__ RingLds<kRingNwc> sh;
+    __shared__ RingLds<2, ring_nwc(2, false)> sh;
     __shared__ int next;
     for (;;) {
         if (threadIdx.x == 0) next = atomicAdd(counter, 1);
@@ -760,7 +782,7 @@ __global__ __launch_bounds__(256, kRingWgs) void gpp_ring_batch_kernel(const Gpp
         const BatchTile bt = tiles[t];
         const int prob = __builtin_amdgcn_readfirstlane(bt.prob);
         const int tm = __builtin_amdgcn_readfirstlane(bt.tm), tn = __builtin_amdgcn_readfirstlane(bt.tn);
-        gpp_ring_tile<kRingNwc, false, false, true>(probs[prob], tm, tn, sh);
+        gpp_ring_tile<2, ring_nwc(2, false), false, false, true>(probs[prob], tm, tn, sh);
     }
 }
 
@@ -921,14 +943,36 @@ void launch_fused(int cfg, int tiles, hipStream_t s, const GppArgs<E> &a)
 // cost nothing that could be measured against 4).
 bool ring_form(int cfg, size_t elem, int nv) { return cfg == 1 && elem == sizeof(double2) && nv <= kRingOcc; }
 
-template <bool ACHS>
-void launch_ring(int tiles, hipStream_t s, const GppArgs<double2> &a)
+// 32 x 32 tiles, for calls of few 64 x 64 tiles: four times the workgroups, a
+// quarter of the epilogue in each, at about 0.8 of the larger tiles' rate once the
+// GPU is full.  Time of the 64 x 64 tiles over that of these, by tiles (64 x 64)
+// and bands: 128 tiles 1.8 at 32 bands to 1.53 at 1000; 256 tiles 1.37, 1.16 (130
+// bands), 0.99 (400), 0.93; 384 tiles 1.23, 1.13, 1.08, 0.99; 512 tiles 1.13, 0.97,
+// 0.86; 640 tiles 1.06, 0.98, 0.93; 768 tiles 0.98, 0.87.
+bool ring_small(int tiles64, int nb) { return tiles64 <= (nb <= 48 ? 640 : nb <= 160 ? 384 : 255); }
+
+template <int MB, bool ACHS>
+void launch_ring_mb(int tiles, hipStream_t s, const GppArgs<double2> &a)
 {
     switch (a.nw) {
-    case 1: hipLaunchKernelGGL((gpp_ring_kernel<1, true, ACHS>), dim3(tiles), dim3(256), 0, s, a); break;
-    case 2: hipLaunchKernelGGL((gpp_ring_kernel<2, true, ACHS>), dim3(tiles), dim3(256), 0, s, a); break;
-    case 3: hipLaunchKernelGGL((gpp_ring_kernel<3, true, ACHS>), dim3(tiles), dim3(256), 0, s, a); break;
-    default: hipLaunchKernelGGL((gpp_ring_kernel<kRingNwc, false, ACHS>), dim3(tiles), dim3(256), 0, s, a); break;
+    case 1: hipLaunchKernelGGL((gpp_ring_kernel<MB, 1, true, ACHS>), dim3(tiles), dim3(256), 0, s, a); break;
+    case 2: hipLaunchKernelGGL((gpp_ring_kernel<MB, 2, true, ACHS>), dim3(tiles), dim3(256), 0, s, a); break;
+    case 3: hipLaunchKernelGGL((gpp_ring_kernel<MB, 3, true, ACHS>), dim3(tiles), dim3(256), 0, s, a); break;
+    default:
+        hipLaunchKernelGGL((gpp_ring_kernel<MB, ring_nwc(MB, ACHS), false, ACHS>), dim3(tiles), dim3(256),
+                           0, s, a);
+        break;
+    }
+}
+
+void launch_ring(int tile, int tiles, hipStream_t s, const GppArgs<double2> &a)
+{
+    if (tile == 32) {
+        if (a.achs_part) launch_ring_mb<1, true>(tiles, s, a);
+        else launch_ring_mb<1, false>(tiles, s, a);
+    } else {
+        if (a.achs_part) launch_ring_mb<2, true>(tiles, s, a);
+        else launch_ring_mb<2, false>(tiles, s, a);
     }
 }
 
@@ -942,7 +986,7 @@ int choose_cfg(const fk_gpp_problem *p, const fk_options *o)
 }
 
 struct Layout {
-    bool ring;
+    int ring;                // gpp_ring_tile's tile size, 32 or 64, or 0
     int cfg, Kpad, nvpad, ldc, tiles_m, tiles_n;
     size_t off_c, off_igp, off_part, off_achs;
     size_t off_stop;   // the gppsum = 1 form: the occupied loop's stop per column
@@ -954,18 +998,29 @@ Layout plan_layout(const fk_gpp_problem *p, const fk_options *o, Scratch &ws, si
     const bool sym = p->semantics == FK_GPP_GPPSUM;
     L.cfg = sym ? 1 : choose_cfg(p, o);   // the gppsum = 1 kernel has 64 x 64 tiles
     const TileCfg &t = kCfgs[L.cfg];
-    L.ring = !sym && ring_form(L.cfg, elem, p->nvband);
+    L.ring = 0;
+    if (!sym && ring_form(L.cfg, elem, p->nvband)) {
+        const int64_t tiles64 = (int64_t)div_up(p->ngpown, 64) * div_up(p->ncouls, 64);
+        L.ring = o->config == 0 && tiles64 <= 1024 && ring_small((int)tiles64, p->number_bands) ? 32 : 64;
+    }
+    const int bm = L.ring ? L.ring : t.bm, bn = L.ring ? L.ring : t.bn;
     const int kstep = L.ring ? 8 : 4 * t.p;
     L.nvpad = div_up(p->nvband, 4) * 4;
     const int rows = std::max(L.nvpad + p->number_bands - p->nvband, 1);
     L.Kpad = L.ring ? L.nvpad + div_up(p->number_bands - p->nvband, kstep) * kstep : div_up(rows, kstep) * kstep;
-    L.ldc = div_up(p->ngpown, t.bm) * t.bm;
-    L.tiles_m = L.ldc / t.bm;
-    L.tiles_n = div_up(p->ncouls, t.bn);
-    L.off_c = ws.plan((size_t)L.Kpad * L.ldc * elem);
+    L.ldc = div_up(p->ngpown, bm) * bm;
+    L.tiles_m = L.ldc / bm;
+    L.tiles_n = div_up(p->ncouls, bn);
+    // never less than the 64 x 64 tiles of gpp_tile and of the gppsum = 1 form
+    // take (bands to 12, columns to 64): callers size the workspace of either
+    // form by the canonical one's
+    const size_t c_elems = std::max((size_t)L.Kpad * L.ldc, (size_t)(div_up(rows, 12) * 12) * (div_up(p->ngpown, 64) * 64));
+    const size_t tiles = std::max((size_t)L.tiles_m * L.tiles_n,
+                                  L.ring ? (size_t)div_up(p->ngpown, 64) * div_up(p->ncouls, 64) : 0);
+    L.off_c = ws.plan((L.ring ? c_elems : (size_t)L.Kpad * L.ldc) * elem);
     L.off_igp = ws.plan(sizeof(int) * (size_t)p->ngpown);
-    L.off_part = ws.plan(sizeof(double2) * 2 * (size_t)p->nfreq * L.tiles_m * L.tiles_n);
-    L.off_achs = ws.plan(sizeof(double2) * (size_t)L.tiles_m * L.tiles_n);   // used when achstemp is asked for
+    L.off_part = ws.plan(sizeof(double2) * 2 * (size_t)p->nfreq * tiles);
+    L.off_achs = ws.plan(sizeof(double2) * tiles);   // used when achstemp is asked for
     L.off_stop = sym ? ws.plan(sizeof(int) * (size_t)p->ngpown) : 0;
     return L;
 }
@@ -1078,7 +1133,7 @@ int launch_gpp(const fk_gpp_problem *p, const fk_options *o, const Layout &L, Sc
         if (L.ring) {
             // a third of a tile alone on its CU: 6 flops per complex
             // multiply-add (3M) at 128 flop/cycle, 2.4 GHz
-            if (tiles > kRingWgs * ncu) {
+            if (L.ring == 64 && tiles > kRingWgs * ncu) {
                 a.stagger_lo = ncu;
                 a.stagger_ticks = (int)std::min(6.0 * 64 * 64 * L.Kpad / 128.0 / 24.0, 1.0e6);
             }
@@ -1097,9 +1152,8 @@ int launch_gpp(const fk_gpp_problem *p, const fk_options *o, const Layout &L, Sc
     KernelTimer timer(o->kernel_ms, s);
     FK_TRY(timer.start());
     if constexpr (sizeof(E) == sizeof(double2)) {
-        if (!L.ring) launch_fused<E>(L.cfg, tiles, s, a);
-        else if (a.achs_part) launch_ring<true>(tiles, s, a);
-        else launch_ring<false>(tiles, s, a);
+        if (L.ring) launch_ring(L.ring, tiles, s, a);
+        else launch_fused<E>(L.cfg, tiles, s, a);
     } else {
         launch_fused<E>(L.cfg, tiles, s, a);
     }

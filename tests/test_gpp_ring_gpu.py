@@ -33,17 +33,20 @@ def _check(fk, fko, p, **kw):
         assert _rel(asx, ref_asx) <= RTOL
 
 
+@pytest.mark.parametrize("config", [0, 2])     # 0: 32 x 32 tiles at these sizes, 2: 64 x 64
 @pytest.mark.parametrize("nb,nv,C,G,nw", [
-    (1, 0, 1, 1, 1), (1, 1, 1, 1, 2), (8, 0, 63, 7, 3), (9, 1, 64, 64, 3), (16, 0, 65, 63, 4), (17, 17, 64, 64, 3),
+    (1, 0, 1, 1, 1), (1, 1, 1, 1, 2), (8, 0, 63, 7, 3), (9, 2, 31, 33, 3), (25, 3, 33, 32, 6), (9, 1, 64, 64, 3), (16, 0, 65, 63, 4), (17, 17, 64, 64, 3),
     (16, 16, 130, 65, 5), (20, 4, 200, 64, 3), (29, 5, 129, 128, 1), (32, 8, 127, 129, 2), (40, 15, 500, 66, 8),
     (33, 16, 257, 65, 9), (33, 17, 257, 65, 9), (24, 0, 640, 31, 16), (57, 9, 1000, 200, 11), (130, 12, 4099, 70, 3),
+    (20, 2, 2561, 1000, 3),       # 640 tiles of 64 x 64 and more: the other side of the rule
 ])
-def test_ring_edges(fk, fko, nb, nv, C, G, nw):
-    _check(fk, fko, fko.gpp_random(nb, nv, C, G, nw=nw, seed=nb + C, wtilde_re=(0.5, 5.5)))
+def test_ring_edges(fk, fko, config, nb, nv, C, G, nw):
+    _check(fk, fko, fko.gpp_random(nb, nv, C, G, nw=nw, seed=nb + C, wtilde_re=(0.5, 5.5)), config=config)
 
 
-@pytest.mark.parametrize("nw", [2, 3, 7])
-def test_general_elements(fk, fko, nw):
+@pytest.mark.parametrize("config", [0, 2])
+@pytest.mark.parametrize("nw", [2, 3, 7, 12])
+def test_general_elements(fk, fko, config, nw):
     """|wtilde| from 1e-6 to 1e5 and wx = wtilde among ordinary elements."""
     p = fko.gpp_random(37, 6, 321, 90, nw=nw, seed=3, wtilde_re=(0.5, 5.5))
     rng = np.random.default_rng(5)
@@ -53,7 +56,7 @@ def test_general_elements(fk, fko, nw):
     w[k[200:400]] = 10.0 ** rng.uniform(2, 5, 200) * np.exp(1j * rng.uniform(0, 6, 200))
     w[k[400:500]] = p.wx[rng.integers(0, nw, 100)] + 1e-9 * rng.normal(size=100)
     w[k[500:]] = -p.wx[rng.integers(0, nw, 100)] + 1e-3j
-    _check(fk, fko, p)
+    _check(fk, fko, p, config=config)
 
 
 def test_band_edges_with_batch(fk, fko):
@@ -108,3 +111,16 @@ def test_inputs_aligned_to_8_bytes(fk, fko):
     torch.cuda.synchronize()
     ref_ach, ref_asx, _ = fko.gpp(p, nthreads=0)
     assert _rel(out[0].cpu().numpy(), ref_ach) <= RTOL and _rel(out[1].cpu().numpy(), ref_asx) <= RTOL
+
+
+@pytest.mark.parametrize("nb,nv,C,G,nw", [(25, 0, 300, 40, 3), (37, 5, 700, 130, 2), (150, 9, 5000, 300, 4)])
+def test_workspace_serves_gppsum(fk, fko, nb, nv, C, G, nw):
+    """The canonical workspace and a stop per column hold the gppsum = 1 form."""
+    import torch
+    p = fko.gpp_random(nb, nv, C, G, nw=nw, seed=nb)
+    d = {k: torch.from_numpy(np.ascontiguousarray(getattr(p, k))).to("cuda:0")
+         for k in ("aqsm", "aqsn", "I_eps", "wtilde", "vcoul")}
+    ws = torch.empty(fk.gpp_workspace_size(nb, nv, C, G, nw) + 4 * G + 256, dtype=torch.uint8, device="cuda:0")
+    fk.gpp_kernel(nb, nv, C, G, p.wx, d["aqsm"], d["aqsn"], d["I_eps"], d["wtilde"], d["vcoul"], p.inv_igp_index,
+                  p.indinv, semantics=fk.FK_GPP_GPPSUM, workspace=ws)
+    torch.cuda.synchronize()
