@@ -34,6 +34,7 @@
 #include "fk_complex.h"
 #include "fk_gpp_common.h"
 #include "fk_internal.h"
+#include "fk_mfma_ring.h"
 
 #include <climits>
 
@@ -42,20 +43,9 @@ namespace {
 
 using namespace gpp;
 
-typedef double d4 __attribute__((ext_vector_type(4)));
-
-constexpr int kSymTile = 64;     // workgroup tile: 2 x 2 waves of 32 x 32
-constexpr int kSymNwc = 4;       // frequencies per epilogue pass
-
-__device__ __forceinline__ d4 mfma(double a, double b, d4 c)
-{
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-// -a * b + c (the neg modifier on A)
-__device__ __forceinline__ d4 mfma_nega(double a, double b, d4 c)
-{
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 1);
-}
+constexpr int kSymTile = 64;     // workgroup tile: two 64 x 32 halves, one after the other
+constexpr int kSymNwc = 3;       // frequencies per epilogue pass
+constexpr int kSymStages = 3, kSymWgs = 3;   // ring stages, workgroups per CU
 
 // std::complex<double> product and quotient as the reference rounds them.
 __device__ __forceinline__ double2 zmul(double2 a, double2 b)
@@ -131,223 +121,327 @@ struct SymArgs {
     double2 *partials;       // [tiles][nw][2]
     int nb, nv, C, G, nw, ldc, nvpad, nks, tiles_m, tiles_n;
     double limittwo, limitone, to1, gamma;
+    double lo, hi;           // sym_terms takes an element with lo < |wtilde|^2 < hi
+    int aligned;             // aqsn and aqsm are 16-byte aligned
     double wx[kMaxFreq];
 };
 
-__device__ __forceinline__ void sym_tile_coords(int b, int tiles_m, int total, int &tm, int &tn)
+// One element's unocc_kind, its occupied flag and whether its mirror counts.
+struct SymElem { int kind; bool occ, mirror; };
+
+__device__ __forceinline__ SymElem sym_elem(const SymArgs &a, int row, int col)
 {
-    // tiles of one XCD (every kXcds-th workgroup) are consecutive in tm,
-    // so they share an aqsn / aqsm column block in that XCD's L2
-    const int q = total / kXcds, r = total % kXcds, x = b % kXcds, i = b / kXcds;
-    const int t = (x < r) ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
-    tm = t % tiles_m;
-    tn = t / tiles_m;
+    SymElem e;
+    const int g = (row < a.G && col < a.C) ? a.igp[row] : -1;
+    e.kind = g >= 0 ? unocc_kind(col, g) : 0;
+    e.occ = g >= 0 && a.nv > 0 && col < a.stop[row];
+    e.mirror = col != g - 1;
+    return e;
 }
 
-__global__ __launch_bounds__(256, 1) void gpp_sym_kernel(SymArgs a)
+// The terms of one element at the NWC frequencies from w0, in the reference's
+// operations and order (any wtilde, any limits).
+template <int NWC>
+__device__ __forceinline__ void sym_element(const SymArgs &a, int w0, SymElem e, double2 wt, double2 ie, double2 Bu,
+                                            double2 Bp, double2 Bo, double2 Bpo, double2 (&sach)[NWC],
+                                            double2 (&sasx)[NWC])
 {
-    constexpr int MB = 2, NB = 2, WM = 32, WN = 32, NWAVES = 4;
-    __shared__ double red[NWAVES][4 * kSymNwc];
-    __shared__ int s_maxg;
+    const double2 wt2 = zmul(wt, wt);
+    const double2 Om = zmul(wt2, ie);
+    const double2 half = e.occ ? zdiv(make_double2(0.5, 0.0), wt) : make_double2(0.0, 0.0);
+#pragma unroll
+    for (int q = 0; q < NWC; ++q) {
+        if (w0 + q >= a.nw) break;
+        const double wxt = a.wx[w0 + q];
+        const double2 wdiff = make_double2(wxt - wt.x, -wt.y);
+        if (e.kind) {
+            const double2 delw = zdiv(wt, wdiff);
+            const double delw2 = znorm2(delw), wdiffr = znorm2(wdiff);
+            if (fabs(wdiffr) < a.limittwo || delw2 > a.limitone) {
+                const double2 sch = zmul(delw, ie);
+                double2 t = cmul(Bu, sch);
+                if (e.kind == 1) t = cadd(t, cconj(cmul(Bp, sch)));
+                sach[q] = cadd(sach[q], t);
+            }
+        }
+        if (e.occ) {
+            const double2 delw = zmul(wdiff, half);
+            const double ad = hypot(delw.x, delw.y);
+            double2 sch = make_double2(0.0, 0.0), ssx = make_double2(0.0, 0.0);
+            if (hypot(wdiff.x, wdiff.y) < a.gamma || ad * ad < a.to1) {
+                if (hypot(wt.x, wt.y) > a.to1) {
+                    const double2 den =
+                        zmul(make_double2(4.0 * wt2.x, 4.0 * wt2.y), make_double2(1.0 + delw.x, delw.y));
+                    ssx = zdiv(make_double2(-Om.x, -Om.y), den);
+                }
+            } else {
+                sch = zdiv(zmul(wt, ie), wdiff);
+                ssx = zdiv(Om, make_double2(wxt * wxt - wt2.x, -wt2.y));
+            }
+            double2 th = cmul(Bo, sch), ts = cmul(Bo, ssx);
+            if (e.mirror) {
+                th = cadd(th, cconj(cmul(Bpo, sch)));
+                ts = cadd(ts, cconj(cmul(Bpo, ssx)));
+            }
+            sach[q] = cadd(sach[q], th);
+            sasx[q] = cadd(sasx[q], ts);
+        }
+    }
+}
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// B x + conj(B' x) as four fused operations: (B + B').re etc. formed once.
+struct SymPair {
+    double xr, xi, yr, yi;     // Re B + Re B', Im B + Im B', Re B - Re B', Im B - Im B'
+    __device__ __forceinline__ SymPair(double2 b, double2 p)
+        : xr(b.x + p.x), xi(b.y + p.y), yr(b.x - p.x), yi(b.y - p.y) {}
+    __device__ __forceinline__ void add(double2 &sum, double2 x) const
+    {
+        sum.x = __builtin_fma(xr, x.x, __builtin_fma(-xi, x.y, sum.x));
+        sum.y = __builtin_fma(yr, x.y, __builtin_fma(yi, x.x, sum.y));
+    }
+};
+
+// The same terms in a fifth of the operations, for lo < |wtilde|^2 < hi (else
+// false, and nothing is added).  With u = wx - wtilde, s = wx + wtilde, T =
+// wtilde I_eps:
+//   near the pole (|u|^2 < limittwo):  unoccupied sch = T / u,
+//                                      occupied   ssx = -T / (2 s)
+//     (1 + delw = s / (2 wtilde), so Omega2 / (4 wtilde^2 (1 + delw)) = T / (2 s));
+//   elsewhere, occupied only:          sch = T / u,  ssx = Omega2 / (wx^2 - wtilde^2).
+// |wtilde|^2 < 0.99 limitone limittwo makes |delw|^2 > limitone imply |u|^2 <
+// limittwo, and |wtilde|^2 < limittwo / (4.04 to1) makes |u / (2 wtilde)|^2 < to1
+// imply it; |wtilde|^2 > 1.01 to1^2 decides |wtilde| > to1.  |u|^2 is rounded as
+// the reference rounds it, but its occupied loop compares hypot(u) with gamma =
+// sqrt(limittwo): an occupied element within 1e-12 of that line returns false too.
+template <int NWC>
+__device__ __forceinline__ bool sym_terms(const SymArgs &a, int w0, SymElem e, double2 wt, double2 ie, double2 Bu,
+                                          double2 Bp, double2 Bo, double2 Bpo, double2 (&sach)[NWC],
+                                          double2 (&sasx)[NWC])
+{
+#pragma clang fp contract(off)
+    const double wy2 = wt.y * wt.y;
+    const double wt2 = __builtin_fma(wt.x, wt.x, wy2);
+    bool fast = wt2 > a.lo && wt2 < a.hi;
+#pragma unroll
+    for (int q = 0; q < NWC; ++q) {
+        const double wdr = a.wx[min(w0 + q, a.nw - 1)] - wt.x, d = wdr * wdr + wy2;
+        fast = fast && !(e.occ && fabs(d - a.limittwo) <= 1e-12 * a.limittwo);
+    }
+    if (!fast) return false;
+    const double2 zero = make_double2(0.0, 0.0);
+    const double2 T = cmul_fused(ie, wt), Om = cmul_fused(T, wt);
+    const double w2r = __builtin_fma(wt.x, wt.x, -wy2), w2i = 2.0 * wt.x * wt.y;
+    const SymPair U(Bu, e.kind == 1 ? Bp : zero), O(Bo, e.mirror ? Bpo : zero);
+#pragma unroll
+    for (int q = 0; q < NWC; ++q) {
+        if (w0 + q >= a.nw) break;
+        const double wx = a.wx[w0 + q];
+        const double wdr = wx - wt.x, d = wdr * wdr + wy2;
+        const bool near = d < a.limittwo;
+        if (near ? e.kind != 0 : e.occ) {
+            const double r = rcp_cubic(d);
+            const double2 sch = make_double2(__builtin_fma(T.x, wdr, -(T.y * wt.y)) * r,
+                                             __builtin_fma(T.y, wdr, T.x * wt.y) * r);
+            if (near) U.add(sach[q], sch);
+            else O.add(sach[q], sch);
+        }
+        if (e.occ) {
+            // N conj(D) / |D|^2
+            const double2 N = near ? make_double2(-0.5 * T.x, -0.5 * T.y) : Om;
+            const double2 D = near ? make_double2(wx + wt.x, wt.y) : make_double2(wx * wx - w2r, -w2i);
+            const double r = rcp_cubic(__builtin_fma(D.x, D.x, D.y * D.y));
+            O.add(sasx[q], make_double2(__builtin_fma(N.x, D.x, N.y * D.y) * r, __builtin_fma(N.y, D.x, -(N.x * D.y)) * r));
+        }
+    }
+    return true;
+}
+
+struct SymLds {
+    union {
+        double2 ring[kSymStages][2][8][64];      // [slot][coefficients; aqsn, aqsm][k][column]
+        double2 b[4][3][4][64];                  // [wave][block - 1][register][lane]
+    };
+    double red[4][4 * kSymNwc];
+    double tot[kMaxFreq * 4];
+    int maxg;
+};
+
+// A 64 x 64 tile of (my_igp, ig) as two halves of 32 ig, each with both right
+// operands side by side: 32 columns of aqsn and the same 32 of aqsm are the 64
+// columns of an LDS ring stage (fk_mfma_ring.h), and of a wave's two column blocks
+// one is Bu and one Bu' of the same 16 ig.  Its three workgroups per CU and the
+// three real products per complex one are the FP64 tiles' of fk_gpp.hip, where
+// the reasons stand, as is the epilogue: three of a wave's four blocks wait in
+// the ring's memory, and the occupied bands are contracted per block.
+//
+// Tiles run in plain order.  (Giving each XCD a contiguous range of columns, for
+// its L2, put the half plane ig <= igp mostly on the first XCDs: twice the time.)
+// Measured at 256/4/16384/819, 3 frequencies: 720 us, before 1476 (two
+// workgroups per CU, four real products, every quotient and hypot evaluated).
+__global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
+{
+    constexpr int MB = 2, NB = 2, NWAVES = 4, LPW = 4;
+    __shared__ SymLds sh;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave & 1, wn = wave >> 1;
-    int tm, tn;
-    sym_tile_coords(blockIdx.x, a.tiles_m, a.tiles_m * a.tiles_n, tm, tn);
-    const int m0 = tm * kSymTile, n0 = tn * kSymTile;
-    const int rowbase = m0 + wm * WM, colbase = n0 + wn * WN;
+    const int tm = blockIdx.x % a.tiles_m, tn = blockIdx.x / a.tiles_m;
+    const int rowbase = tm * kSymTile + wm * 32, nmax = a.C - 1;
     const int kl = lane >> 4, cl = lane & 15;
     const size_t tile = (size_t)tm + (size_t)tn * a.tiles_m;
 
-    if (tid == 0) s_maxg = -1;
+    if (tid == 0) sh.maxg = -1;
+    if (tid < kMaxFreq * 4) sh.tot[tid] = 0.0;
     __syncthreads();
-    if (tid < kSymTile && m0 + tid < a.G) atomicMax(&s_maxg, a.igp[m0 + tid]);
+    if (tid < kSymTile && tm * kSymTile + tid < a.G) atomicMax(&sh.maxg, a.igp[tm * kSymTile + tid]);
     __syncthreads();
-    if (n0 > s_maxg) {   // no ig <= igp in this tile: its partials are zero
-        for (int k = tid; k < 4 * a.nw; k += 256)
-            reinterpret_cast<double *>(a.partials + tile * a.nw * 2)[k] = 0.0;
-        return;
-    }
+    const int maxg = sh.maxg;
 
-    // ---- GEMM over the unoccupied bands: Bu (right operand aqsn), Bu' (aqsm)
-    d4 acc_re[MB][NB], acc_im[MB][NB], acc2_re[MB][NB], acc2_im[MB][NB];
-#pragma unroll
-    for (int i = 0; i < MB; ++i)
-#pragma unroll
-        for (int j = 0; j < NB; ++j) {
-            acc_re[i][j] = d4{0, 0, 0, 0};
-            acc_im[i][j] = d4{0, 0, 0, 0};
-            acc2_re[i][j] = d4{0, 0, 0, 0};
-            acc2_im[i][j] = d4{0, 0, 0, 0};
-        }
-    const int nmax = a.C - 1;
-    int colj[NB];
-#pragma unroll
-    for (int j = 0; j < NB; ++j) colj[j] = min(colbase + j * 16 + cl, nmax);
-    const double2 *pa = a.c + (size_t)kl * a.ldc + rowbase + cl;
-    struct Fr { double2 a[MB], b[NB], b2[NB]; };
-    auto load = [&](Fr &f, int s) {
-        s = min(s, a.nks - 1);
-        const double2 *qa = pa + (size_t)(4 * s) * a.ldc;
-#pragma unroll
-        for (int i = 0; i < MB; ++i) f.a[i] = qa[i * 16];
-        // coefficient row 4s + kl holds band kr - nvpad + nv (a zero row
-        // past the last band makes the clamped band irrelevant)
-        const int kr = 4 * s + kl;
-        const int band = min(max(kr - a.nvpad + a.nv, 0), a.nb - 1);
-        const double2 *qn = a.aqsn + (size_t)band * a.C, *qm = a.aqsm + (size_t)band * a.C;
-#pragma unroll
-        for (int j = 0; j < NB; ++j) {
-            f.b[j] = qn[colj[j]];
-            f.b2[j] = qm[colj[j]];
-        }
-    };
-    auto mma = [&](const Fr &f) {
-#pragma unroll
-        for (int i = 0; i < MB; ++i)
-#pragma unroll
-            for (int j = 0; j < NB; ++j) {
-                acc_re[i][j] = mfma(f.a[i].x, f.b[j].x, acc_re[i][j]);
-                acc_im[i][j] = mfma(f.a[i].x, f.b[j].y, acc_im[i][j]);
-                acc2_re[i][j] = mfma(f.a[i].x, f.b2[j].x, acc2_re[i][j]);
-                acc2_im[i][j] = mfma(f.a[i].x, f.b2[j].y, acc2_im[i][j]);
-            }
-#pragma unroll
-        for (int i = 0; i < MB; ++i)
-#pragma unroll
-            for (int j = 0; j < NB; ++j) {
-                acc_re[i][j] = mfma_nega(f.a[i].y, f.b[j].y, acc_re[i][j]);
-                acc_im[i][j] = mfma(f.a[i].y, f.b[j].x, acc_im[i][j]);
-                acc2_re[i][j] = mfma_nega(f.a[i].y, f.b2[j].y, acc2_re[i][j]);
-                acc2_im[i][j] = mfma(f.a[i].y, f.b2[j].x, acc2_im[i][j]);
-            }
-    };
-    const int s_begin = a.nvpad / 4;
-    if (s_begin < a.nks) {
-        Fr f0, f1;
-        load(f0, s_begin);
-        load(f1, s_begin + 1);
-        int s = s_begin;
-        for (; s + 1 < a.nks; s += 2) {
-            mma(f0);
-            load(f0, s + 2);
-            mma(f1);
-            load(f1, s + 3);
-        }
-        if (s < a.nks) mma(f0);
-    }
+    const bool side_a = wave < 2;
+    const int k0 = 4 * (wave & 1);
+    const int nun = a.nb - a.nv, nst = (nun + 7) / 8;
+    const size_t ld = side_a ? (size_t)a.ldc : (size_t)a.C;
+    const int row0 = (side_a ? a.nvpad : a.nv) + k0;
+    const int last = side_a ? a.nks * 4 - 1 : a.nb - 1;
+    const bool direct = side_a || a.aligned;
+    const int nko = (a.nv + 3) / 4;
 
-    // ---- epilogue ----------------------------------------------------------
-    for (int w0 = 0; w0 < a.nw; w0 += kSymNwc) {
-        double2 sach[kSymNwc], sasx[kSymNwc];
+    for (int n0 = tn * kSymTile; n0 < (tn + 1) * kSymTile && n0 <= min(maxg, nmax); n0 += 32) {
+        // ---- GEMM over the unoccupied bands: Bu (right operand aqsn), Bu' (aqsm)
+        const int lcol = min(n0 + (lane & 31), nmax);
+        const double2 *src = side_a ? a.c + tm * kSymTile + lane : (lane < 32 ? a.aqsn : a.aqsm) + lcol;
+        auto issue = [&](int s, int slot) {
+            const int r = row0 + 8 * s;
+            double2 *dst = &sh.ring[slot][side_a ? 0 : 1][k0][0];
+            if (direct) {
 #pragma unroll
-        for (int q = 0; q < kSymNwc; ++q) { sach[q] = make_double2(0.0, 0.0); sasx[q] = make_double2(0.0, 0.0); }
-        // The 16 elements of a lane in a runtime loop (the body is too large
-        // to repeat 16 times); a wave-uniform switch picks the element's
-        // accumulator registers with constant indices.
-#pragma unroll 1
-        for (int el = 0; el < MB * NB * 4; ++el) {
-                    const int i = el >> 3, j = (el >> 2) & 1, r = el & 3;
-                    double2 Bu = make_double2(0.0, 0.0), Bp = make_double2(0.0, 0.0);
-                    switch (el) {
-#define FK_SYM_PICK(I, J, R)                                                        \
-    case (I) * 8 + (J) * 4 + (R):                                                   \
-        Bu = make_double2(acc_re[I][J][R], acc_im[I][J][R]);                        \
-        Bp = make_double2(acc2_re[I][J][R], acc2_im[I][J][R]);                      \
-        break;
-                        FK_SYM_PICK(0, 0, 0) FK_SYM_PICK(0, 0, 1) FK_SYM_PICK(0, 0, 2) FK_SYM_PICK(0, 0, 3)
-                        FK_SYM_PICK(0, 1, 0) FK_SYM_PICK(0, 1, 1) FK_SYM_PICK(0, 1, 2) FK_SYM_PICK(0, 1, 3)
-                        FK_SYM_PICK(1, 0, 0) FK_SYM_PICK(1, 0, 1) FK_SYM_PICK(1, 0, 2) FK_SYM_PICK(1, 0, 3)
-                        FK_SYM_PICK(1, 1, 0) FK_SYM_PICK(1, 1, 1) FK_SYM_PICK(1, 1, 2) FK_SYM_PICK(1, 1, 3)
-#undef FK_SYM_PICK
-                    default: break;
-                    }
-                    const int row = rowbase + i * 16 + 4 * r + (lane >> 4);
-                    const int col = colbase + j * 16 + cl;
-                    const int g = (row < a.G && col <= nmax) ? a.igp[row] : -1;
-                    const int kind = g >= 0 ? unocc_kind(col, g) : 0;
-                    const bool occ = g >= 0 && a.nv > 0 && col < a.stop[row];
-                    if (kind || occ) {
-                    const size_t e = (size_t)row * a.C + col;
-                    const double2 wt = a.wtilde[e], ie = a.I_eps[e];
-                    double2 Bo = make_double2(0.0, 0.0), Bpo = make_double2(0.0, 0.0);
-                    if (occ) {
-                        for (int n1 = 0; n1 < a.nv; ++n1) {
-                            const double2 cn = a.c[(size_t)n1 * a.ldc + row];
-                            Bo = cadd(Bo, cmul(cn, a.aqsn[(size_t)n1 * a.C + col]));
-                            Bpo = cadd(Bpo, cmul(cn, a.aqsm[(size_t)n1 * a.C + col]));
-                        }
-                    }
-                    const double2 wt2 = zmul(wt, wt);
-                    const double2 Om = zmul(wt2, ie);
-                    const double2 half = occ ? zdiv(make_double2(0.5, 0.0), wt) : make_double2(0.0, 0.0);
-                    const bool mirror = col != g - 1;
+                for (int j = 0; j < LPW; ++j) ring::lds_load16(src + (size_t)min(r + j, last) * ld, dst + 64 * j);
+            } else {
 #pragma unroll
-                    for (int q = 0; q < kSymNwc; ++q) {
-                        const int iw = min(w0 + q, a.nw - 1);
-                        const bool live = w0 + q < a.nw;
-                        const double wxt = a.wx[iw];
-                        const double2 wdiff = make_double2(wxt - wt.x, -wt.y);
-                        if (live && kind) {
-                            const double2 delw = zdiv(wt, wdiff);
-                            const double delw2 = znorm2(delw), wdiffr = znorm2(wdiff);
-                            if (fabs(wdiffr) < a.limittwo || delw2 > a.limitone) {
-                                const double2 sch = zmul(delw, ie);
-                                double2 t = cmul(Bu, sch);
-                                if (kind == 1) t = cadd(t, cconj(cmul(Bp, sch)));
-                                sach[q] = cadd(sach[q], t);
-                            }
-                        }
-                        if (live && occ) {
-                            const double2 delw = zmul(wdiff, half);
-                            const double ad = hypot(delw.x, delw.y);
-                            double2 sch = make_double2(0.0, 0.0), ssx = make_double2(0.0, 0.0);
-                            if (hypot(wdiff.x, wdiff.y) < a.gamma || ad * ad < a.to1) {
-                                if (hypot(wt.x, wt.y) > a.to1) {
-                                    const double2 den = zmul(make_double2(4.0 * wt2.x, 4.0 * wt2.y),
-                                                             make_double2(1.0 + delw.x, delw.y));
-                                    ssx = zdiv(make_double2(-Om.x, -Om.y), den);
-                                }
-                            } else {
-                                sch = zdiv(zmul(wt, ie), wdiff);
-                                ssx = zdiv(Om, make_double2(wxt * wxt - wt2.x, -wt2.y));
-                            }
-                            double2 th = cmul(Bo, sch), ts = cmul(Bo, ssx);
-                            if (mirror) {
-                                th = cadd(th, cconj(cmul(Bpo, sch)));
-                                ts = cadd(ts, cconj(cmul(Bpo, ssx)));
-                            }
-                            sach[q] = cadd(sach[q], th);
-                            sasx[q] = cadd(sasx[q], ts);
-                        }
-                    }
+                for (int j = 0; j < LPW; ++j) dst[64 * j + lane] = ring::load16(src + (size_t)min(r + j, last) * ld);
+            }
+        };
+        auto read = [&](ring::Frags<MB, NB> &f, int s, int slot, int q) {
+            const double2 *st = &sh.ring[slot][0][4 * q + kl][cl];
+#pragma unroll
+            for (int i = 0; i < MB; ++i) f.a[i] = st[wm * 32 + 16 * i];
+#pragma unroll
+            for (int j = 0; j < NB; ++j) f.b[j] = st[8 * 64 + 32 * j + wn * 16];
+            if (8 * s + 8 > nun) {   // rows past the last band
+                const bool kok = 8 * s + 4 * q + kl < nun;
+#pragma unroll
+                for (int i = 0; i < MB; ++i) f.a[i] = kok ? f.a[i] : make_double2(0.0, 0.0);
+            }
+        };
+        ring::Acc3<MB, NB> acc;
+        acc.zero();
+        ring::main_loop<MB, NB, kSymStages, LPW>(nst, acc, issue, read);
+        ring::wait_barrier<0>();
+
+        // ---- epilogue
+        double2 Bu0[4];
+#pragma unroll
+        for (int k = 0; k < MB * NB; ++k)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const double2 v = acc.value(k / NB, k % NB, r);
+                if (k == 0) Bu0[r] = v;
+                else sh.b[wave][k - 1][r][lane] = v;
+            }
+        for (int w0 = 0; w0 < a.nw; w0 += kSymNwc) {
+            double2 sach[kSymNwc], sasx[kSymNwc];
+#pragma unroll
+            for (int q = 0; q < kSymNwc; ++q) { sach[q] = make_double2(0.0, 0.0); sasx[q] = make_double2(0.0, 0.0); }
+            unsigned general = 0;
+            int kp = kl, cp = cl;      // opaque in each pass (gpp_ring_tile)
+            asm volatile("" : "+v"(kp), "+v"(cp));
+            const int col = n0 + wn * 16 + cp;
+#pragma unroll
+            for (int i = 0; i < MB; ++i) {
+                __builtin_amdgcn_sched_barrier(0);
+                double2 cwt[4], cie[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int row = rowbase + i * 16 + 4 * r + kp;
+                    const size_t e = (size_t)min(row, a.G - 1) * a.C + min(col, nmax);
+                    cwt[r] = a.wtilde[e];
+                    cie[r] = a.I_eps[e];
+                }
+                ring::Acc3<1, 2> o;
+                o.zero();
+                for (int ks = 0; ks < nko; ++ks) {
+                    ring::Frags<1, 2> f;
+                    const size_t rb = (size_t)min(4 * ks + kp, a.nb - 1) * a.C + min(col, nmax);
+                    f.a[0] = a.c[(size_t)(4 * ks + kp) * a.ldc + rowbase + 16 * i + cp];
+                    f.b[0] = a.aqsn[rb];
+                    f.b[1] = a.aqsm[rb];
+                    o.mma(f);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    const SymElem e = sym_elem(a, rowbase + i * 16 + 4 * r + kp, col);
+                    if (e.kind || e.occ) {
+                        const double2 Bu = i == 0 ? Bu0[r] : sh.b[wave][1][r][lane];
+                        const double2 Bp = sh.b[wave][2 * i][r][lane];
+                        if (!sym_terms<kSymNwc>(a, w0, e, cwt[r], cie[r], Bu, Bp, o.value(0, 0, r), o.value(0, 1, r), sach,
+                                                sasx))
+                            general |= 1u << (4 * i + r);
                     }
                 }
-        // wave reduction, then a fixed-order sum over the waves
-#pragma unroll
-        for (int q = 0; q < kSymNwc; ++q) {
-            const double v0 = wave_sum(sach[q].x), v1 = wave_sum(sach[q].y);
-            const double v2 = wave_sum(sasx[q].x), v3 = wave_sum(sasx[q].y);
-            if (lane == 0) {
-                red[wave][4 * q + 0] = v0;
-                red[wave][4 * q + 1] = v1;
-                red[wave][4 * q + 2] = v2;
-                red[wave][4 * q + 3] = v3;
             }
-        }
-        __syncthreads();
-        if (tid < 4 * kSymNwc) {
-            const int q = tid >> 2, comp = tid & 3;
-            const int iw = w0 + q;
-            if (iw < a.nw) {
-                double sum = red[0][tid];
-#pragma unroll
-                for (int w = 1; w < NWAVES; ++w) sum += red[w][tid];
-                reinterpret_cast<double *>(a.partials + (tile * a.nw + iw) * 2)[comp] = sum;
+            // the elements sym_terms left out, one at a time
+            if (__ballot(general != 0)) {
+#pragma unroll 1
+                for (int el = 0; el < MB * 4; ++el) {
+                    if ((general >> el) & 1u) {
+                        const int i = el >> 2, r = el & 3, row = rowbase + 16 * i + 4 * r + kp;
+                        double2 Bu;
+                        switch (el) {             // constant register indices
+                        case 0: Bu = Bu0[0]; break;
+                        case 1: Bu = Bu0[1]; break;
+                        case 2: Bu = Bu0[2]; break;
+                        case 3: Bu = Bu0[3]; break;
+                        default: Bu = sh.b[wave][1][r][lane];
+                        }
+                        const double2 Bp = sh.b[wave][2 * i][r][lane];
+                        double2 Bo = make_double2(0.0, 0.0), Bpo = Bo;
+                        for (int n1 = 0; n1 < a.nv; ++n1) {
+                            const double2 cn = a.c[(size_t)n1 * a.ldc + row];
+                            Bo = cfma(Bo, cn, a.aqsn[(size_t)n1 * a.C + col]);
+                            Bpo = cfma(Bpo, cn, a.aqsm[(size_t)n1 * a.C + col]);
+                        }
+                        const size_t x = (size_t)row * a.C + col;
+                        sym_element<kSymNwc>(a, w0, sym_elem(a, row, col), a.wtilde[x], a.I_eps[x], Bu, Bp, Bo, Bpo, sach,
+                                             sasx);
+                    }
+                }
             }
+            // wave reduction, then a fixed-order sum over the waves and halves
+            double v[4 * kSymNwc];
+#pragma unroll
+            for (int q = 0; q < kSymNwc; ++q) {
+                v[4 * q + 0] = sach[q].x;
+                v[4 * q + 1] = sach[q].y;
+                v[4 * q + 2] = sasx[q].x;
+                v[4 * q + 3] = sasx[q].y;
+            }
+#pragma unroll
+            for (int q = 0; q < 4 * kSymNwc; ++q) {
+                const double x = wave_sum(v[q]);
+                if (lane == 0) sh.red[wave][q] = x;
+            }
+            __syncthreads();
+            if (tid < 4 * kSymNwc && w0 + (tid >> 2) < a.nw) {
+                double sum = sh.red[0][tid];
+#pragma unroll
+                for (int w = 1; w < NWAVES; ++w) sum += sh.red[w][tid];
+                sh.tot[4 * w0 + tid] += sum;
+            }
+            __syncthreads();
         }
-        __syncthreads();
     }
+    __syncthreads();
+    for (int k = tid; k < 4 * a.nw; k += 256) reinterpret_cast<double *>(a.partials + tile * a.nw * 2)[k] = sh.tot[k];
 }
 
 }  // namespace
@@ -367,6 +461,13 @@ int gpp_sym_launch(const fk_gpp_problem *p, const double2 *c, int ldc, int Kpad,
     a.nb = p->number_bands; a.nv = p->nvband; a.C = p->ncouls; a.G = p->ngpown; a.nw = p->nfreq;
     a.ldc = ldc; a.nvpad = nvpad; a.nks = Kpad / 4; a.tiles_m = tiles_m; a.tiles_n = tiles_n;
     a.limittwo = p->limittwo; a.limitone = p->limitone; a.to1 = p->to1; a.gamma = std::sqrt(p->limittwo);
+    a.lo = a.hi = 0.0;
+    if (p->limittwo > 0.0 && p->limitone > 0.0 && p->to1 >= 0.0) {
+        a.lo = 1.01 * p->to1 * p->to1;
+        a.hi = 0.99 * p->limitone * p->limittwo;
+        if (p->to1 > 0.0) a.hi = std::min(a.hi, p->limittwo / (4.04 * p->to1));
+    }
+    a.aligned = ((reinterpret_cast<uintptr_t>(aqsn) | reinterpret_cast<uintptr_t>(aqsm)) & 15) == 0;
     for (int iw = 0; iw < kMaxFreq; ++iw) a.wx[iw] = iw < p->nfreq ? p->wx[iw] : 0.0;
     KernelTimer timer(kernel_ms, s);
     FK_TRY(timer.start());
