@@ -1094,9 +1094,12 @@ int launch_gpp_sym(const fk_gpp_problem *p, const fk_options *o, const Layout &L
     int *igp = static_cast<int *>(ws.at(L.off_igp));
     double2 *part = static_cast<double2 *>(ws.at(L.off_part));
     FK_TRY(launch_coef<double2>(p, L, cols, aqsm, vcoul, c, igp, s));
-    FK_TRY(gpp_sym_launch(p, c, L.ldc, L.Kpad, L.nvpad, igp, static_cast<int *>(ws.at(L.off_stop)), aqsm, aqsn,
-                          ieps, wt, part, L.tiles_m, L.tiles_n, o->kernel_ms, s));
-    return gpp_reduce_launch(part, L.tiles_m * L.tiles_n, p->nfreq, 2.0 * p->occ, d_ach, d_asx, s);
+    // the partials may run on into the (here unused) static-CH ones behind them
+    const size_t room = (L.off_stop - L.off_part) / (sizeof(double2) * 2 * (size_t)p->nfreq);
+    int count = 0;
+    FK_TRY(gpp_sym_launch(p, cols, c, L.ldc, L.Kpad, L.nvpad, igp, static_cast<int *>(ws.at(L.off_stop)), aqsm, aqsn,
+                          ieps, wt, part, room, &count, o->kernel_ms, s));
+    return gpp_reduce_launch(part, count, p->nfreq, 2.0 * p->occ, d_ach, d_asx, s);
 }
 
 template <class E>

@@ -22,11 +22,11 @@
 // coefficient matrix of the canonical path):
 //   Bu  = sum_{n1 >= nv} c aqsn[n1][ig],   Bu' = sum_{n1 >= nv} c aqsm[n1][ig],
 // and m2-sums are conj(Bu'), so a term is Bu x + conj(Bu' x).  The kernel
-// runs both on FP64 MFMA over the unoccupied bands of a 64 x 64 tile of
+// runs both on FP64 MFMA over the unoccupied bands of a 64 x 32 tile of
 // (my_igp, ig) (a tile with no ig <= igp of its rows is skipped), forms the
-// occupied-band sums Bo, Bo' directly in the epilogue (nvband is small) and
-// evaluates the factors per element and frequency in FP64.  Complex
-// division is Smith's algorithm (R. L. Smith, "Algorithm 116: Complex
+// occupied-band sums Bo, Bo' by MFMA in the epilogue and evaluates the factors
+// per element and frequency in FP64.  Near a branch threshold complex division
+// is Smith's algorithm (R. L. Smith, "Algorithm 116: Complex
 // division", CACM 5(8), 1962), the order of libgcc's __divdc3 that the
 // reference's std::complex<double> calls, with IEEE quotients and no
 // contraction; |z| is hypot.  Per-tile partials go to the reduction of the
@@ -36,14 +36,17 @@
 #include "fk_internal.h"
 #include "fk_mfma_ring.h"
 
+#include <algorithm>
 #include <climits>
+#include <cmath>
 
 namespace fk {
 namespace {
 
 using namespace gpp;
 
-constexpr int kSymTile = 64;     // workgroup tile: two 64 x 32 halves, one after the other
+constexpr int kSymTile = 64, kSymCols = 32;   // rows and columns of a tile
+constexpr int kSymBlocks = 512;  // row blocks whose tiles the kernel arguments can list
 constexpr int kSymNwc = 3;       // frequencies per epilogue pass
 constexpr int kSymStages = 3, kSymWgs = 3;   // ring stages, workgroups per CU
 
@@ -118,8 +121,11 @@ struct SymArgs {
     const double2 *wtilde;   // [G][C]
     const int *igp;          // [G], -1 = skipped column
     const int *stop;         // [G] (read when nv > 0)
-    double2 *partials;       // [tiles][nw][2]
-    int nb, nv, C, G, nw, ldc, nvpad, nks, tiles_m, tiles_n;
+    double2 *partials;       // [workgroups][nw][2]
+    int nb, nv, C, G, nw, ldc, nvpad, nks;
+    int nblk, per;           // row blocks; tiles per workgroup
+    int every;               // > 0: workgroups of every row block (more than kSymBlocks blocks)
+    int first[kSymBlocks + 1];   // first workgroup of each row block
     double limittwo, limitone, to1, gamma;
     double lo, hi;           // sym_terms takes an element with lo < |wtilde|^2 < hi
     int aligned;             // aqsn and aqsm are 16-byte aligned
@@ -263,38 +269,46 @@ struct SymLds {
     };
     double red[4][4 * kSymNwc];
     double tot[kMaxFreq * 4];
-    int maxg;
 };
 
-// A 64 x 64 tile of (my_igp, ig) as two halves of 32 ig, each with both right
-// operands side by side: 32 columns of aqsn and the same 32 of aqsm are the 64
+// A 64 x 32 tile of (my_igp, ig) with both right operands side by side: 32
+// columns of aqsn and the same 32 of aqsm are the 64
 // columns of an LDS ring stage (fk_mfma_ring.h), and of a wave's two column blocks
 // one is Bu and one Bu' of the same 16 ig.  Its three workgroups per CU and the
 // three real products per complex one are the FP64 tiles' of fk_gpp.hip, where
 // the reasons stand, as is the epilogue: three of a wave's four blocks wait in
 // the ring's memory, and the occupied bands are contracted per block.
 //
-// Tiles run in plain order.  (Giving each XCD a contiguous range of columns, for
-// its L2, put the half plane ig <= igp mostly on the first XCDs: twice the time.)
-// Measured at 256/4/16384/819, 3 frequencies: 720 us, before 1476 (two
-// workgroups per CU, four real products, every quotient and hypot evaluated).
+// Only the tiles with some ig <= igp have a workgroup: the host lists them by
+// row block (`per` of them in one workgroup where there are more than partials).
+// Measured at 256/4/16384/819, 3 frequencies: 561 us; with a workgroup for
+// every 64 x 64 tile, half of them empty, 720; with those in contiguous ranges of
+// columns per XCD, two workgroups per CU, four real products and every quotient
+// and hypot evaluated 1476.
 __global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
 {
     constexpr int MB = 2, NB = 2, NWAVES = 4, LPW = 4;
     __shared__ SymLds sh;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave & 1, wn = wave >> 1;
-    const int tm = blockIdx.x % a.tiles_m, tn = blockIdx.x / a.tiles_m;
+    int tm, h0;
+    if (a.every > 0) {
+        tm = blockIdx.x / a.every;
+        h0 = (blockIdx.x - tm * a.every) * a.per;
+    } else {
+        int lo = 0, hi = a.nblk - 1;               // last row block with first <= this workgroup
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (a.first[mid] <= (int)blockIdx.x) lo = mid;
+            else hi = mid - 1;
+        }
+        tm = lo;
+        h0 = ((int)blockIdx.x - a.first[lo]) * a.per;
+    }
     const int rowbase = tm * kSymTile + wm * 32, nmax = a.C - 1;
     const int kl = lane >> 4, cl = lane & 15;
-    const size_t tile = (size_t)tm + (size_t)tn * a.tiles_m;
-
-    if (tid == 0) sh.maxg = -1;
     if (tid < kMaxFreq * 4) sh.tot[tid] = 0.0;
     __syncthreads();
-    if (tid < kSymTile && tm * kSymTile + tid < a.G) atomicMax(&sh.maxg, a.igp[tm * kSymTile + tid]);
-    __syncthreads();
-    const int maxg = sh.maxg;
 
     const bool side_a = wave < 2;
     const int k0 = 4 * (wave & 1);
@@ -305,7 +319,7 @@ __global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
     const bool direct = side_a || a.aligned;
     const int nko = (a.nv + 3) / 4;
 
-    for (int n0 = tn * kSymTile; n0 < (tn + 1) * kSymTile && n0 <= min(maxg, nmax); n0 += 32) {
+    for (int n0 = h0 * kSymCols; n0 < (h0 + a.per) * kSymCols && n0 <= nmax; n0 += kSymCols) {
         // ---- GEMM over the unoccupied bands: Bu (right operand aqsn), Bu' (aqsm)
         const int lcol = min(n0 + (lane & 31), nmax);
         const double2 *src = side_a ? a.c + tm * kSymTile + lane : (lane < 32 ? a.aqsn : a.aqsm) + lcol;
@@ -359,13 +373,14 @@ __global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
             for (int i = 0; i < MB; ++i) {
                 __builtin_amdgcn_sched_barrier(0);
                 double2 cwt[4], cie[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
+                auto load = [&](int r) {
                     const int row = rowbase + i * 16 + 4 * r + kp;
                     const size_t e = (size_t)min(row, a.G - 1) * a.C + min(col, nmax);
                     cwt[r] = a.wtilde[e];
                     cie[r] = a.I_eps[e];
-                }
+                };
+                load(0);
+                load(1);
                 ring::Acc3<1, 2> o;
                 o.zero();
                 for (int ks = 0; ks < nko; ++ks) {
@@ -379,6 +394,10 @@ __global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     __builtin_amdgcn_sched_barrier(0);
+                    if (r == 1) {
+                        load(2);
+                        load(3);
+                    }
                     const SymElem e = sym_elem(a, rowbase + i * 16 + 4 * r + kp, col);
                     if (e.kind || e.occ) {
                         const double2 Bu = i == 0 ? Bu0[r] : sh.b[wave][1][r][lane];
@@ -416,7 +435,7 @@ __global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
                     }
                 }
             }
-            // wave reduction, then a fixed-order sum over the waves and halves
+            // wave reduction, then a fixed-order sum over the waves and tiles
             double v[4 * kSymNwc];
 #pragma unroll
             for (int q = 0; q < kSymNwc; ++q) {
@@ -441,14 +460,14 @@ __global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
         }
     }
     __syncthreads();
-    for (int k = tid; k < 4 * a.nw; k += 256) reinterpret_cast<double *>(a.partials + tile * a.nw * 2)[k] = sh.tot[k];
+    for (int k = tid; k < 4 * a.nw; k += 256) reinterpret_cast<double *>(a.partials + (size_t)blockIdx.x * a.nw * 2)[k] = sh.tot[k];
 }
 
 }  // namespace
 
-int gpp_sym_launch(const fk_gpp_problem *p, const double2 *c, int ldc, int Kpad, int nvpad, const int *d_igp,
-                   int *d_stop, const double2 *aqsm, const double2 *aqsn, const double2 *ieps, const double2 *wt,
-                   double2 *partials, int tiles_m, int tiles_n, float *kernel_ms, hipStream_t s)
+int gpp_sym_launch(const fk_gpp_problem *p, const std::vector<int32_t> &cols, const double2 *c, int ldc, int Kpad,
+                   int nvpad, const int *d_igp, int *d_stop, const double2 *aqsm, const double2 *aqsn, const double2 *ieps,
+                   const double2 *wt, double2 *partials, size_t max_partials, int *count, float *kernel_ms, hipStream_t s)
 {
     if (p->nvband > 0) {
         hipLaunchKernelGGL(gpp_sym_stop_kernel, dim3(p->ngpown), dim3(256), 0, s, wt, ieps, d_igp, p->ncouls, p->to1,
@@ -459,7 +478,28 @@ int gpp_sym_launch(const fk_gpp_problem *p, const double2 *c, int ldc, int Kpad,
     a.c = c; a.aqsn = aqsn; a.aqsm = aqsm; a.I_eps = ieps; a.wtilde = wt; a.igp = d_igp; a.stop = d_stop;
     a.partials = partials;
     a.nb = p->number_bands; a.nv = p->nvband; a.C = p->ncouls; a.G = p->ngpown; a.nw = p->nfreq;
-    a.ldc = ldc; a.nvpad = nvpad; a.nks = Kpad / 4; a.tiles_m = tiles_m; a.tiles_n = tiles_n;
+    a.ldc = ldc; a.nvpad = nvpad; a.nks = Kpad / 4;
+    // the tiles of each row block: columns 0 .. its largest igp
+    a.nblk = div_up(p->ngpown, kSymTile);
+    std::vector<int> tiles(a.nblk, div_up(p->ncouls, kSymCols));
+    const bool listed = a.nblk <= kSymBlocks;
+    int64_t total = 0;
+    for (int b = 0; b < a.nblk; ++b) {
+        if (listed) {
+            int g = -1;
+            for (int m = b * kSymTile; m < std::min((b + 1) * kSymTile, p->ngpown); ++m) g = std::max(g, (int)cols[m]);
+            tiles[b] = (std::min(g, p->ncouls - 1) + kSymCols) / kSymCols;   // 0 for g = -1
+        }
+        total += tiles[b];
+    }
+    a.per = total <= (int64_t)max_partials ? 1 : 2;   // two per workgroup are a 64 x 64 tile's worth of partials
+    a.every = listed ? 0 : div_up(tiles[0], a.per);
+    int blocks = 0;
+    for (int b = 0; b < a.nblk; ++b) {
+        if (listed) a.first[b] = blocks;
+        blocks += div_up(tiles[b], a.per);
+    }
+    *count = blocks;
     a.limittwo = p->limittwo; a.limitone = p->limitone; a.to1 = p->to1; a.gamma = std::sqrt(p->limittwo);
     a.lo = a.hi = 0.0;
     if (p->limittwo > 0.0 && p->limitone > 0.0 && p->to1 >= 0.0) {
@@ -471,7 +511,7 @@ int gpp_sym_launch(const fk_gpp_problem *p, const double2 *c, int ldc, int Kpad,
     for (int iw = 0; iw < kMaxFreq; ++iw) a.wx[iw] = iw < p->nfreq ? p->wx[iw] : 0.0;
     KernelTimer timer(kernel_ms, s);
     FK_TRY(timer.start());
-    hipLaunchKernelGGL(gpp_sym_kernel, dim3(tiles_m * tiles_n), dim3(256), 0, s, a);
+    if (blocks > 0) hipLaunchKernelGGL(gpp_sym_kernel, dim3(blocks), dim3(256), 0, s, a);
     FK_HIP(hipGetLastError());
     FK_TRY(timer.stop());
     return timer.finish();
