@@ -79,13 +79,6 @@ __device__ __forceinline__ void split4(double x, double scale, int8_t (&s)[kSlic
 }
 
 
-__device__ __forceinline__ double2 coef(const float2 *aqsm, const double *vcoul, int C, int n1, int g)
-{
-    const float2 am = aqsm[(size_t)n1 * C + g];
-    const double s = 0.5 * vcoul[g];
-    return make_double2((double)am.x * s, -(double)am.y * s);
-}
-
 // ---------------------------------------------------------------------------
 // Slices of both operands in one launch.  A workgroup takes 4 coefficient
 // rows (the first ldm/4 workgroups) or 16 aqsn columns (the rest).  Each
@@ -106,90 +99,106 @@ struct PrepArgs {
     int nb, nv, C, G, ldm, ldn, nkb, blocks_a;
 };
 
-// R rows (coefficients, IS_A) or columns (aqsn) per workgroup, 256 / R band
-// groups: the coefficients are gathered at scattered igp columns, so their
-// slabs are kept thin to spread the gathers over more workgroups.
+// R rows (coefficients, IS_A) or columns (aqsn) per workgroup, kPrepThreads / R
+// band groups: the coefficients are gathered at scattered igp columns, so their
+// slabs are kept thin to spread the gathers over more workgroups.  A thread's
+// first 16 bands stay in registers between the two passes (all of them up to 512
+// bands of aqsn), loaded 16 at once.  Measured at 512/2/32768/1638: 114 us, with
+// 256 threads that read every band twice 184.
+constexpr int kPrepThreads = 512;
+
 template <int R, bool IS_A>
 __device__ __forceinline__ void prep_slab(const PrepArgs &a, int slab)
 {
-    constexpr int NG = 256 / R;
-    __shared__ double sm[kProds][NG][R];
+    constexpr int NG = kPrepThreads / R, NW = kPrepThreads / 64;
+    __shared__ double sm[kProds][NW][R];
     const int tid = threadIdx.x, c = tid % R, grp = tid / R;
     const int idx = slab * R + c;
-    const int g = IS_A ? (idx < a.G ? a.igp[idx] : -1) : 0;
+    const int g = IS_A ? (idx < a.G ? a.igp[idx] : -1) : idx;
     const bool in = IS_A ? g >= 0 : idx < a.C;
-    // element n1 of this row (the coefficient c) or column (aqsn)
-    auto value = [&](int n1) -> double2 {
-        if (!in || n1 >= a.nb) return make_double2(0.0, 0.0);
-        if constexpr (IS_A) {
-            return coef(a.aqsm, a.vcoul, a.C, n1, g);
-        } else {
-            const float2 v = a.aqsn[(size_t)n1 * a.C + idx];
-            return make_double2((double)v.x, (double)v.y);
-        }
+    const float2 *src = (IS_A ? a.aqsm : a.aqsn) + (in ? g : 0);
+    const double vs = IS_A && in ? 0.5 * a.vcoul[g] : 0.0;
+    // bands 16 j .. 16 j + 15 of this row or column, as stored
+    float2 raw[16];
+    auto load = [&](int j) {
+#pragma unroll
+        for (int b = 0; b < 16; ++b)
+            raw[b] = in && 16 * j + b < a.nb ? src[(size_t)(16 * j + b) * a.C] : make_float2(0.f, 0.f);
+    };
+    // the coefficient c or the value of aqsn
+    auto value = [&](float2 v) -> double2 {
+        if constexpr (IS_A) return make_double2((double)v.x * vs, -(double)v.y * vs);
+        else return make_double2((double)v.x, (double)v.y);
     };
     const int nblk = (a.nb + 15) / 16;
     double mx[kProds] = {0.0, 0.0, 0.0};
-    for (int j = grp; j < nblk; j += NG)
-#pragma unroll 8
+    auto maxima = [&]() {
+#pragma unroll
         for (int b = 0; b < 16; ++b) {
-            const double2 v = value(16 * j + b);
+            const double2 v = value(raw[b]);
             mx[0] = fmax(mx[0], fabs(v.x));
             mx[1] = fmax(mx[1], fabs(v.y));
             mx[2] = fmax(mx[2], fabs(v.x + v.y));
         }
+    };
+    for (int j = grp + NG; j < nblk; j += NG) {
+        load(j);
+        maxima();
+    }
+    load(grp);
+    maxima();
 #pragma unroll
-    for (int pr = 0; pr < kProds; ++pr) sm[pr][grp][c] = mx[pr];
+    for (int pr = 0; pr < kProds; ++pr) {
+#pragma unroll
+        for (int off = R; off < 64; off <<= 1) mx[pr] = fmax(mx[pr], __shfl_xor(mx[pr], off, 64));
+        if ((tid & 63) < R) sm[pr][tid >> 6][c] = mx[pr];
+    }
     __syncthreads();
     const int ld = IS_A ? a.ldm : a.ldn;
     double scale[kProds];
 #pragma unroll
     for (int pr = 0; pr < kProds; ++pr) {
         double m = 0.0;
-        for (int k = 0; k < NG; ++k) m = fmax(m, sm[pr][k][c]);
+#pragma unroll
+        for (int k = 0; k < NW; ++k) m = fmax(m, sm[pr][k][c]);
         scale[pr] = m > 0.0 ? 127.0 / m : 0.0;
         if (grp == 0) (IS_A ? a.ra : a.rb)[(size_t)pr * ld + idx] = m / 127.0;
     }
 
     int8_t *base = IS_A ? a.as : a.bs;
     const size_t blk = idx >> 5, nblks = (size_t)ld / 32;
-    // 16-band blocks of the padded K, split in two halves of 8 bands (a
-    // scheduling barrier keeps each half's loads and splits together, so
-    // only 8 values are live at once; 4 waves per SIMD), then one 16-byte
-    // store per plane
+    // 16-band blocks of the padded K, one 16-byte store per plane
     for (int j = grp; j < a.nkb * 2; j += NG) {
+        if (j != grp) load(j);
         const int lane = (idx & 31) + 32 * (j & 1), kb = j >> 1;
-        uint32_t q[kProds][kSlices][4] = {};   // the 16 bytes of each plane, packed
+        // One product's planes at a time: 16 registers of packed bytes.  The
+        // stored values are opaque in each, or their 32 FP64 forms would be kept
+        // from one to the next (spilled).
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int pr = 0; pr < kProds; ++pr) {
+            uint32_t q[kSlices][4] = {};
 #pragma unroll
-            for (int b = 0; b < 8; ++b) {
-                const int n1 = 16 * j + 8 * h + b, byte = 8 * h + b;
-                const double2 v = value(n1);
-                if (IS_A && n1 < a.nv) a.c_occ[(size_t)n1 * a.ldm + idx] = v;
-                const double x[kProds] = {v.x, v.y, v.x + v.y};
+            for (int b = 0; b < 16; ++b) asm volatile("" : "+v"(raw[b].x), "+v"(raw[b].y));
 #pragma unroll
-                for (int pr = 0; pr < kProds; ++pr) {
-                    int8_t sl[kSlices];
-                    split4(x[pr], scale[pr], sl);
+            for (int b = 0; b < 16; ++b) {
+                const double2 v = value(raw[b]);
+                if (IS_A && pr == 0 && 16 * j + b < a.nv) a.c_occ[(size_t)(16 * j + b) * a.ldm + idx] = v;
+                int8_t sl[kSlices];
+                split4(pr == 0 ? v.x : pr == 1 ? v.y : v.x + v.y, scale[pr], sl);
 #pragma unroll
-                    for (int k = 0; k < kSlices; ++k)
-                        q[pr][k][byte >> 2] |= (uint32_t)(uint8_t)sl[k] << (8 * (byte & 3));
-                }
+                for (int k = 0; k < kSlices; ++k) q[k][b >> 2] |= (uint32_t)(uint8_t)sl[k] << (8 * (b & 3));
             }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int pr = 0; pr < kProds; ++pr)
 #pragma unroll
             for (int k = 0; k < kSlices; ++k) {
                 int8_t *dst = base + (((size_t)(pr * kSlices + k) * nblks + blk) * a.nkb + kb) * kFrag + 16 * lane;
-                *reinterpret_cast<uint4 *>(dst) = make_uint4(q[pr][k][0], q[pr][k][1], q[pr][k][2], q[pr][k][3]);
+                *reinterpret_cast<uint4 *>(dst) = make_uint4(q[k][0], q[k][1], q[k][2], q[k][3]);
             }
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
 }
 
-constexpr int kPrepRowsA = 4, kPrepColsB = 16;
+constexpr int kPrepRowsA = 8, kPrepColsB = 16;
 
 __device__ __forceinline__ void oz_prep_block(const PrepArgs &a, int b)
 {
@@ -197,7 +206,7 @@ __device__ __forceinline__ void oz_prep_block(const PrepArgs &a, int b)
     else prep_slab<kPrepColsB, false>(a, b - a.blocks_a);
 }
 
-__global__ __launch_bounds__(256) void oz_prep_kernel(PrepArgs a)
+__global__ __launch_bounds__(kPrepThreads, 4) void oz_prep_kernel(PrepArgs a)
 {
     oz_prep_block(a, blockIdx.x);
 }
@@ -738,7 +747,7 @@ __device__ __forceinline__ int batch_problem(const int *first, int n, int b)
     return __builtin_amdgcn_readfirstlane(lo);
 }
 
-__global__ __launch_bounds__(256) void oz_prep_batch_kernel(const OzRecord *rec, const int *first, int n)
+__global__ __launch_bounds__(kPrepThreads, 4) void oz_prep_batch_kernel(const OzRecord *rec, const int *first, int n)
 {
     const int b = (int)blockIdx.x, p = batch_problem(first, n, b);
     const PrepArgs pr = rec[p].pr;   // in registers: not reloaded after each barrier
@@ -828,7 +837,7 @@ int gpp_oz_batch_launch(const void *records, const int *first_prep, const int *f
 {
     const OzRecord *rec = static_cast<const OzRecord *>(records);
     if (total_prep > 0)
-        hipLaunchKernelGGL(oz_prep_batch_kernel, dim3(total_prep), dim3(256), 0, s, rec, first_prep, n);
+        hipLaunchKernelGGL(oz_prep_batch_kernel, dim3(total_prep), dim3(kPrepThreads), 0, s, rec, first_prep, n);
     if (total_gemm > 0) {
         int dev = 0, ncu = 0;
         FK_HIP(hipGetDevice(&dev));
@@ -894,7 +903,7 @@ int gpp_oz_launch(const fk_gpp_problem *p, const fk_options *o, const OzLayout &
     pr.c_occ = static_cast<double2 *>(ws.at(L.off_cocc));
     pr.nb = p->number_bands; pr.nv = p->nvband; pr.C = p->ncouls; pr.G = p->ngpown;
     pr.ldm = L.ldm; pr.ldn = L.ldn; pr.nkb = nkb; pr.blocks_a = L.ldm / kPrepRowsA;
-    hipLaunchKernelGGL(oz_prep_kernel, dim3(L.ldm / kPrepRowsA + L.ldn / kPrepColsB), dim3(256), 0, s, pr);
+    hipLaunchKernelGGL(oz_prep_kernel, dim3(L.ldm / kPrepRowsA + L.ldn / kPrepColsB), dim3(kPrepThreads), 0, s, pr);
     FK_HIP(hipGetLastError());
 
     GemmArgs ga;
