@@ -641,7 +641,7 @@ def main():
         "data": "synthetic",
         "config": {"workload": "GPP band sum 512/2/32768/20 (ngpown 1638, 3 frequencies), FP64",
                    "number_bands": NB, "nvband": NV, "ncouls": C, "ngpown": G, "nfreq": NW},
-        "roofline": {"bound": "mfma", "kernel": "gpp_fused_kernel", "achieved": achieved, "peak": PEAK_FP64,
+        "roofline": {"bound": "mfma", "kernel": "gpp_ring_kernel", "achieved": achieved, "peak": PEAK_FP64,
                      "unit": "TFLOP/s", "frac": achieved / PEAK_FP64,
                      "traffic": load_traffic("gpp_fused_fp64_traffic.json"),
                      "alg_flops_per_launch": f_alg, "kernel_ms": r["kernel_ms"],

@@ -154,7 +154,10 @@ struct FfBatch {
                 if (rc == FK_OK &&
                     (hipEventSynchronize(e1) != hipSuccess || hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
                     rc = FK_ERR_HIP;
-                if (rc == FK_OK && ms < best_ms) { best_ms = ms; best = c; }
+                // split BF16: a larger chunk of FP32 sums (a later configuration)
+                // has to be faster by more than one timing's noise
+                const float margin = mixed && c > 1 ? 0.98f : 1.0f;
+                if (rc == FK_OK && ms < margin * best_ms) { best_ms = ms; best = c; }
             }
             (void)hipEventDestroy(e0);
             (void)hipEventDestroy(e1);
