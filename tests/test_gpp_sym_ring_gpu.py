@@ -73,3 +73,15 @@ def test_threshold_and_general_elements(fk, fko, nw):
     s = rng.choice([-1.0, 1.0], 200)
     w[k[400:]] = p.wx[rng.integers(0, nw, 200)] + s * np.sqrt(p.limittwo) * (1 + 2.0 ** -52 * rng.integers(-3, 4, 200))
     _check(fk, fko, p)
+
+
+def test_stop_positions(fk, fko):
+    """The occupied loop's break at the edges of the scan's steps (256 threads of
+    4 ig), at to1 to the last bits, and two breaks in one column."""
+    p = fko.gpp_random(6, 3, 2300, 12, seed=8, wtilde_re=(0.5, 5.5))
+    p.inv_igp_index[:] = p.ncouls - 1 - np.arange(p.ngpown)
+    for m, at in enumerate([0, 1, 255, 256, 511, 767, 768, 1023, 1024, 2047, 2048]):
+        p.I_eps[m, at] = p.to1 * (1 - 1e-12) / p.wtilde[m, at] ** 2
+    p.I_eps[2, 100] = p.to1 * (1 + 1e-12) / p.wtilde[2, 100] ** 2
+    p.I_eps[5, 2000] = 0.0
+    _check(fk, fko, p)
