@@ -228,6 +228,11 @@ def _ptr(x):
     return x.ctypes.data
 
 
+def _addr(a):
+    """Address of a C-contiguous numpy array (a.ctypes.data builds an object for it)."""
+    return a.__array_interface__["data"][0]
+
+
 _PRECISIONS = {"fp64": FK_PREC_FP64, "mixed": FK_PREC_MIXED}
 _NP = {"c128": np.complex128, "c64": np.complex64, "f64": np.float64}
 
@@ -256,14 +261,15 @@ def _bulk(where, arrays):
     if on_dev:
         import torch
         tdt = {"c128": torch.complex128, "c64": torch.complex64, "f64": torch.float64}
-        dev = torch.cuda.current_device() if torch.cuda.is_available() else None
     for name, x, kind, numel in arrays:
         if x is None:
             raise ValueError(f"{where}: {name} is missing")
         if on_dev:
             if not x.is_cuda:
                 raise TypeError(f"{where}: {name} is a CPU tensor; pass numpy arrays for host memory")
-            if x.device.index != dev:
+            if dev is None:
+                dev = torch.cuda.current_device()
+            if x.get_device() != dev:
                 raise ValueError(f"{where}: {name} is on {x.device}, the library runs on cuda:{dev}")
             if x.dtype != tdt[kind]:
                 raise TypeError(f"{where}: {name} must be {tdt[kind]}, not {x.dtype}")
@@ -341,8 +347,9 @@ def gpp_kernel(nb, nv, ncouls, ngpown, wx, aqsm, aqsn, I_eps, wtilde, vcoul, inv
                                   ("wtilde", wtilde, ck, GC), ("vcoul", vcoul, "f64", int(ncouls))])
     _host_len("gpp_kernel", "inv_igp_index", inv, int(ngpown))
     _host_len("gpp_kernel", "indinv", ind, int(ncouls) + 1)
-    prob = GppProblem(int(nb), int(nv), int(ncouls), int(ngpown), nw, wx.ctypes.data, _ptr(aqsm), _ptr(aqsn),
-                      _ptr(I_eps), _ptr(wtilde), _ptr(vcoul), inv.ctypes.data, ind.ctypes.data,
+    # (contiguity was checked above)
+    ptrs = [x.data_ptr() if on_dev else _ptr(x) for x in (aqsm, aqsn, I_eps, wtilde, vcoul)]
+    prob = GppProblem(int(nb), int(nv), int(ncouls), int(ngpown), nw, _addr(wx), *ptrs, _addr(inv), _addr(ind),
                       float(to1), float(limittwo), float(limitone), float(occ), int(semantics))
     opt = default_options()
     opt.memory = FK_MEM_DEVICE if on_dev else FK_MEM_HOST
