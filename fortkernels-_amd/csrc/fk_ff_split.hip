@@ -34,7 +34,8 @@
 // is split once by ff_split_a_kernel into the three A matrices in MFMA
 // fragment order, and each wave loads its own fragments from L2 one stage
 // ahead.  The MFMAs of a stage run in six groups of 24 (k-step, product);
-// the splitting of X and the loads ride between them.
+// the splitting of X, the loads and the LDS reads of the next group's B
+// fragments ride between them.
 #include "fk_complex.h"
 #include "fk_internal.h"
 
@@ -235,49 +236,70 @@ __global__ __launch_bounds__(256, 1) void ff_split_gemm_kernel(SplitArgs a)
     for (int j = 0; j < 4; ++j) xv[j] = load_x(min(1, nst - 1), j);
     __syncthreads();
 
+    // B fragments of group (q, pr) of the stage in `buf`: [column block][slice]
+    struct BFrags { uint4 v[2][kSlices]; };
+    auto read_b = [&](BFrags &b, int buf, int q, int pr) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int sl = 0; sl < kSlices; ++sl)
+                b.v[j][sl] = *reinterpret_cast<const uint4 *>(lds + buf * kBufDw + (pr * kSlices + sl) * kSliceDw +
+                                                              (32 * j + (L & 31)) * kRowDw + 8 * q + 4 * (L >> 5));
+    };
+    BFrags bf[2];
+    read_b(bf[0], 0, 0, 0);
     for (int s = 0; s < nst; ++s) {
-        const uint32_t *buf = lds + (s & 1) * kBufDw;
         const int sn = min(s + 1, nst - 1), sx = min(s + 2, nst - 1);
 #pragma unroll
-        for (int q = 0; q < kSteps; ++q) {
+        for (int g = 0; g < kSteps * kProds; ++g) {
+            const int q = g / kProds, pr = g % kProds;
+            // the other LDS buffer is complete (groups 1..4) and this one was
+            // read to its end by group 4 (which read group 5's fragments)
+            if (g == 5) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            // the next group's fragments arrive behind this group's MFMAs
+            if (g < 5) read_b(bf[(g + 1) & 1], s & 1, (g + 1) / kProds, (g + 1) % kProds);
+            else read_b(bf[0], (s + 1) & 1, 0, 0);
+            const BFrags &b = bf[g & 1];
+            // slice pairs (A, B): (0,0) (0,1) (0,2) (1,0) (1,1) (2,0)
 #pragma unroll
-            for (int pr = 0; pr < kProds; ++pr) {
-                uint4 b[2][kSlices];   // [column block][slice] of B matrix pr
+            for (int sa = 0; sa < kSlices; ++sa)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+                for (int sb = 0; sb < kSlices - sa; ++sb)
 #pragma unroll
-                    for (int sl = 0; sl < kSlices; ++sl)
-                        b[j][sl] = *reinterpret_cast<const uint4 *>(buf + (pr * kSlices + sl) * kSliceDw +
-                                                                    (32 * j + (L & 31)) * kRowDw + 8 * q +
-                                                                    4 * (L >> 5));
-                // slice pairs (A, B): (0,0) (0,1) (0,2) (1,0) (1,1) (2,0)
+                    for (int i = 0; i < 2; ++i)
 #pragma unroll
-                for (int sa = 0; sa < kSlices; ++sa)
-#pragma unroll
-                    for (int sb = 0; sb < kSlices - sa; ++sb)
-#pragma unroll
-                        for (int i = 0; i < 2; ++i)
-#pragma unroll
-                            for (int j = 0; j < 2; ++j)
-                                acc[i][j][pr] = mfma(av[q][pr][i][sa], b[j][sb], acc[i][j][pr]);
-                // work between the groups: X of stage s+1 split into the
-                // other LDS buffer (last read before the previous barrier),
-                // each pair reloaded with stage s+2 at once (groups 1..4),
-                // and this group's A fragments reloaded with stage s+1
-                const int g = q * kProds + pr;
-                if (g >= 1 && g <= 4) {
-                    store_x((s + 1) & 1, g - 1, xv[g - 1]);
-                    xv[g - 1] = load_x(sx, g - 1);
-                }
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int sl = 0; sl < kSlices; ++sl) av[q][pr][i][sl] = load_a(sn, q, pr, i, sl);
-                __builtin_amdgcn_sched_barrier(0);
+                        for (int j = 0; j < 2; ++j)
+                            acc[i][j][pr] = mfma(av[q][pr][i][sa], b.v[j][sb], acc[i][j][pr]);
+            // work between the MFMAs: X of stage s+1 split into the other LDS
+            // buffer (last read before the previous barrier), each pair
+            // reloaded with stage s+2 at once (groups 1..4), and this group's
+            // A fragments reloaded with stage s+1
+            if (g >= 1 && g <= 4) {
+                store_x((s + 1) & 1, g - 1, xv[g - 1]);
+                xv[g - 1] = load_x(sx, g - 1);
             }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int sl = 0; sl < kSlices; ++sl) av[q][pr][i][sl] = load_a(sn, q, pr, i, sl);
+            // One wave per SIMD: the matrix pipe waits whenever the wave issues
+            // something else in a row, so the rest is dealt out between the
+            // MFMAs, fragments first (256/8/4096/4096/32/10: 5.00 ms per
+            // evaluation as the compiler orders it, 4.83 so; two or four vector
+            // operations per MFMA 4.93-4.98, LDS reads after the sixth MFMA the
+            // same, global loads from the first or the sixteenth 4.86, 4.91)
+#pragma unroll
+            for (int k = 0; k < 24; ++k) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                        // MFMA
+                if (k < 6) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);             // LDS read
+                __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);                        // vector ALU
+                if (k >= 8 && k % 2) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);   // LDS write
+                if (k >= 8) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);            // global load
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        __syncthreads();
     }
+    __syncthreads();
 
     // epilogue: T (FP32) -> LDS, one band per thread, FP64 contraction over
     // the tile's columns in ascending order
