@@ -209,15 +209,19 @@ __device__ __forceinline__ void sym_element(const SymArgs &a, int w0, SymElem e,
     }
 }
 
-// B x + conj(B' x) as four fused operations: (B + B').re etc. formed once.
+// B x + conj(B' x) with (B + B').re etc. formed once.  A term is formed before it
+// meets the sum, which is larger and rounds at its own size: with its two products
+// added one by one the error against long double (rms of 150 problems of
+// 30/4/400/64, 3M) is 3.5e-16 of the largest achtemp and 3.6e-16 of the largest
+// asxtemp, so 3.4e-16 and 3.45e-16.
 struct SymPair {
     double xr, xi, yr, yi;     // Re B + Re B', Im B + Im B', Re B - Re B', Im B - Im B'
     __device__ __forceinline__ SymPair(double2 b, double2 p)
         : xr(b.x + p.x), xi(b.y + p.y), yr(b.x - p.x), yi(b.y - p.y) {}
     __device__ __forceinline__ void add(double2 &sum, double2 x) const
     {
-        sum.x = __builtin_fma(xr, x.x, __builtin_fma(-xi, x.y, sum.x));
-        sum.y = __builtin_fma(yr, x.y, __builtin_fma(yi, x.x, sum.y));
+        sum.x += __builtin_fma(xr, x.x, -(xi * x.y));
+        sum.y += __builtin_fma(yr, x.y, yi * x.x);
     }
 };
 
@@ -288,17 +292,21 @@ struct SymLds {
 // A 64 x 32 tile of (my_igp, ig) with both right operands side by side: 32
 // columns of aqsn and the same 32 of aqsm are the 64
 // columns of an LDS ring stage (fk_mfma_ring.h), and of a wave's two column blocks
-// one is Bu and one Bu' of the same 16 ig.  Its three workgroups per CU and the
-// three real products per complex one are the FP64 tiles' of fk_gpp.hip, where
-// the reasons stand, as is the epilogue: three of a wave's four blocks wait in
-// the ring's memory, and the occupied bands are contracted per block.
+// one is Bu and one Bu' of the same 16 ig.  Its three workgroups per CU are the
+// FP64 tiles' of fk_gpp.hip, where the reasons stand, as is the epilogue: three of
+// a wave's four blocks wait in the ring's memory, and the occupied bands are
+// contracted per block.  The complex products are four real ones (ring::Acc4):
+// with three (3M) the call below takes 550 us, but the imaginary parts of nearly
+// real sums are lost (wavefunctions and matrices with inversion symmetry), and the
+// error of the case itself is larger: 3.4e-16 against 3.0e-16 of the largest
+// achtemp, 3.45e-16 against 3.2e-16 of the largest asxtemp (150 problems of
+// 30/4/400/64 against long double).
 //
 // Only the tiles with some ig <= igp have a workgroup: the host lists them by
 // row block (`per` of them in one workgroup where there are more than partials).
-// Measured at 256/4/16384/819, 3 frequencies: 561 us; with a workgroup for
-// every 64 x 64 tile, half of them empty, 720; with those in contiguous ranges of
-// columns per XCD, two workgroups per CU, four real products and every quotient
-// and hypot evaluated 1476.
+// Measured at 256/4/16384/819, 3 frequencies: the call 640 us, with contiguous ranges
+// of 64 x 64 tiles per XCD, half of them empty, two workgroups per CU and every
+// quotient and hypot evaluated 1486.
 __global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
 {
     constexpr int MB = 2, NB = 2, NWAVES = 4, LPW = 4;
@@ -360,7 +368,7 @@ __global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
                 for (int i = 0; i < MB; ++i) f.a[i] = kok ? f.a[i] : make_double2(0.0, 0.0);
             }
         };
-        ring::Acc3<MB, NB> acc;
+        ring::Acc4<MB, NB> acc;
         acc.zero();
         ring::main_loop<MB, NB, kSymStages, LPW>(nst, acc, issue, read);
         ring::wait_barrier<0>();
@@ -395,7 +403,7 @@ __global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
                 };
                 load(0);
                 load(1);
-                ring::Acc3<1, 2> o;
+                ring::Acc4<1, 2> o;
                 o.zero();
                 for (int ks = 0; ks < nko; ++ks) {
                     ring::Frags<1, 2> f;

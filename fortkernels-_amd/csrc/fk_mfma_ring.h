@@ -1,6 +1,6 @@
 // fk_mfma_ring.h -- the FP64 MFMA main loop shared by the GPP and FF GEMMs:
 // operands staged through an LDS ring by direct global->LDS loads, the
-// complex product as three real MFMA products.
+// complex product as three or four real MFMA products.
 //
 // Why LDS and not fragments loaded straight into registers (the form before):
 // a CU's eight waves then issue four 1 KB fragment loads per 12 MFMAs, each
@@ -111,6 +111,42 @@ struct Acc3 {
     }
 };
 
+// The complex product as four real ones: a third more MFMAs, but the error of
+// each part stays relative to that part's own products, while the 3M form adds
+// errors of the size of |re| to im.  With operands whose imaginary parts are
+// 1e-8 of the real ones, sums of 32 and 256 products: im good to 3e-16 and
+// 8e-16 of itself, 3M 2e-8 and 5e-8.
+template <int MB, int NB>
+struct Acc4 {
+    d4 re[MB][NB], im[MB][NB];
+
+    __device__ __forceinline__ void zero()
+    {
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) re[i][j] = im[i][j] = d4{0, 0, 0, 0};
+    }
+    __device__ __forceinline__ void mma(const Frags<MB, NB> &f)
+    {
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) {
+                re[i][j] = mfma(f.a[i].x, f.b[j].x, re[i][j]);
+                im[i][j] = mfma(f.a[i].x, f.b[j].y, im[i][j]);
+            }
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) {
+                re[i][j] = mfma_nega(f.a[i].y, f.b[j].y, re[i][j]);
+                im[i][j] = mfma(f.a[i].y, f.b[j].x, im[i][j]);
+            }
+    }
+    __device__ __forceinline__ double2 value(int i, int j, int r) const { return make_double2(re[i][j][r], im[i][j][r]); }
+};
+
 // The main loop: nst stages of 8 k (two k-steps) through a ring of NS LDS
 // slots.  issue(stage, slot) starts this wave's LPW direct loads of a stage;
 // read(frags, stage, slot, q) reads its fragments of k-step q.  Stage s+NS-1
@@ -121,8 +157,8 @@ struct Acc3 {
 // end, where fewer are in flight, everything is waited for.  On return no
 // load is in flight and every wave may still be reading the last slot: meet a
 // barrier before the ring is used for something else.
-template <int MB, int NB, int NS, int LPW, class Issue, class Read>
-__device__ __forceinline__ void main_loop(int nst, Acc3<MB, NB> &acc, Issue issue, Read read)
+template <int MB, int NB, int NS, int LPW, class Acc, class Issue, class Read>
+__device__ __forceinline__ void main_loop(int nst, Acc &acc, Issue issue, Read read)
 {
     auto arrived = [&](int s) {
         if (s + NS - 2 < nst) wait_barrier<LPW *(NS - 2)>();
