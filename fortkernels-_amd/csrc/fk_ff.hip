@@ -519,7 +519,7 @@ static int ff_fp64_gemm(const FfLayout &L, const double2 *aqsn, const double2 *X
     a.tiles_m = L.tiles_m; a.mtiles = L.mtiles; a.tiles_n = nf * L.mtiles;
     a.ksplit = L.ksplit;
     a.kper = L.kper;
-    a.aligned = ((reinterpret_cast<uintptr_t>(aqsn) | reinterpret_cast<uintptr_t>(X)) & 15) == 0;
+    a.aligned = ring::aligned16(aqsn) & ring::aligned16(X);
     const int tiles = a.tiles_m * a.tiles_n;
     FK_TRY(timer.start());
     launch_ff_fused(L.cfg, tiles, s, a);

@@ -56,7 +56,7 @@ struct GppArgs {
     int nb, nv, C, G, nw, ldc, Kpad;
     int nvpad;             // occupied bands rounded up to a k-step (4)
     int nks;               // k-steps (Kpad / 4)
-    int aligned;           // gpp_ring_tile: aqsn is 16-byte aligned
+    int aligned;           // gpp_ring_tile: 16-byte aligned: c (bit 0), aqsn (bit 1)
     int tiles_m, tiles_n, group_m;
     int stagger_lo, stagger_hi;   // workgroups that start late ...
     int stagger_ticks;            // ... by this many wall-clock ticks (100 MHz)
@@ -528,7 +528,7 @@ __device__ __forceinline__ void gpp_ring_tile(const GppArgs<double2> &a, int tm,
     const size_t ld = side_a ? (size_t)a.ldc : (size_t)a.C;
     const int row0 = (side_a ? a.nvpad : a.nv) + k0;
     const int last = side_a ? a.nks * 4 - 1 : a.nb - 1;
-    const bool direct = side_a || a.aligned;
+    const bool direct = a.aligned & (side_a ? 1 : 2);
     auto issue = [&](int s, int slot) {
         const int r = row0 + 8 * s + lane / T;
         double2 *dst = &sh.ring[slot][side_a ? 0 : 1][k0][0];
@@ -1123,7 +1123,7 @@ int launch_gpp(const fk_gpp_problem *p, const fk_options *o, const Layout &L, Sc
     a.achs_part = d_achs ? static_cast<double2 *>(ws.at(L.off_achs)) : nullptr;
     a.nb = p->number_bands; a.nv = p->nvband; a.C = C; a.G = G; a.nw = p->nfreq; a.ldc = L.ldc; a.Kpad = L.Kpad;
     a.nvpad = L.nvpad; a.nks = L.Kpad / 4;
-    a.aligned = (reinterpret_cast<uintptr_t>(aqsn) & 15) == 0;
+    a.aligned = ring::aligned16(c) | ring::aligned16(aqsn) << 1;
     a.tiles_m = L.tiles_m; a.tiles_n = L.tiles_n;
     a.group_m = std::min(L.tiles_m, kGroupM);
     const int tiles = L.tiles_m * L.tiles_n;
@@ -1483,7 +1483,7 @@ struct GppBatch {
             a.Kpad = ring(c) ? b.nvpad + div_up(b.nb - b.nv, 8) * 8
                              : div_up(std::max(b.nvpad + b.nb - b.nv, 1), kstep) * kstep;
             a.nks = a.Kpad / 4;
-            a.aligned = (reinterpret_cast<uintptr_t>(a.aqsn) & 15) == 0;
+            a.aligned = ring::aligned16(a.c) | ring::aligned16(a.aqsn) << 1;
             a.tiles_m = div_up(b.G, t.bm);
             a.tiles_n = div_up(b.C, t.bn);
             a.group_m = a.tiles_m;   // unused: the batch walks its own tile table
@@ -1924,7 +1924,7 @@ int gpp_kernel_ex(const fk_gpp_problem *p, const fk_options *o, const fk_gpp_out
         gpp_oz_plan(p, ws, Z);
         const size_t off_igp = ws.plan(sizeof(int) * (size_t)p->ngpown);
         void *n1_base = workspace_tail(o, ws.total(), n1 ? n1_bytes(p, false) : 0);
-        rc = ws.acquire(o->workspace, o->workspace_bytes, s);
+        rc = ws.acquire(o->workspace, o->workspace_bytes, s, 16);   // operand slices move by direct 16-byte loads
         int *d_igp = static_cast<int *>(ws.at(off_igp));
         if (rc == FK_OK) {
             hipError_t e = hipMemcpyAsync(d_igp, igp.data(), sizeof(int) * igp.size(), hipMemcpyHostToDevice, s);

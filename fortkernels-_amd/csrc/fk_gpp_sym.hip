@@ -142,7 +142,7 @@ struct SymArgs {
     int first[kSymBlocks + 1];   // first workgroup of each row block
     double limittwo, limitone, to1, gamma;
     double lo, hi;           // sym_terms takes an element with lo < |wtilde|^2 < hi
-    int aligned;             // aqsn and aqsm are 16-byte aligned
+    int aligned;             // 16-byte aligned: c (bit 0), aqsn and aqsm (bit 1)
     double wx[kMaxFreq];
 };
 
@@ -338,7 +338,7 @@ __global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
     const size_t ld = side_a ? (size_t)a.ldc : (size_t)a.C;
     const int row0 = (side_a ? a.nvpad : a.nv) + k0;
     const int last = side_a ? a.nks * 4 - 1 : a.nb - 1;
-    const bool direct = side_a || a.aligned;
+    const bool direct = a.aligned & (side_a ? 1 : 2);
     const int nko = (a.nv + 3) / 4;
 
     for (int n0 = h0 * kSymCols; n0 < (h0 + a.per) * kSymCols && n0 <= nmax; n0 += kSymCols) {
@@ -529,7 +529,7 @@ int gpp_sym_launch(const fk_gpp_problem *p, const std::vector<int32_t> &cols, co
         a.hi = 0.99 * p->limitone * p->limittwo;
         if (p->to1 > 0.0) a.hi = std::min(a.hi, p->limittwo / (4.04 * p->to1));
     }
-    a.aligned = ((reinterpret_cast<uintptr_t>(aqsn) | reinterpret_cast<uintptr_t>(aqsm)) & 15) == 0;
+    a.aligned = ring::aligned16(c) | (ring::aligned16(aqsn) & ring::aligned16(aqsm)) << 1;
     for (int iw = 0; iw < kMaxFreq; ++iw) a.wx[iw] = iw < p->nfreq ? p->wx[iw] : 0.0;
     KernelTimer timer(kernel_ms, s);
     FK_TRY(timer.start());

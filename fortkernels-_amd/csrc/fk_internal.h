@@ -56,7 +56,9 @@ public:
     // acquire(), then ptr() in the same order.
     size_t plan(size_t bytes) { size_t off = total_; total_ = align_up(total_ + bytes, 256); return off; }
     size_t total() const { return total_; }
-    int acquire(void *user, size_t user_bytes, hipStream_t stream);
+    // A caller's workspace that is not `align`-byte aligned is left alone and the
+    // call takes an allocation of its own, as without a workspace.
+    int acquire(void *user, size_t user_bytes, hipStream_t stream, size_t align = 1);
     void *at(size_t offset) const { return static_cast<char *>(base_) + offset; }
 
 private:

@@ -44,9 +44,13 @@ __device__ __forceinline__ void lds_load16(const void *g, const void *lds)
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(la) : "memory", "m0");
 }
 
+// Whether p may be the source of direct loads (16-byte aligned).
+inline int aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
 // The element at g where g need not be 16-byte aligned (an array of complex
-// numbers is aligned to its 8-byte parts only): such sources are staged by
-// way of registers, stored to LDS when the direct load would be issued.
+// numbers is aligned to its 8-byte parts only, and a workspace may start
+// anywhere): such sources are staged by way of registers, stored to LDS when the
+// direct load would be issued.
 __device__ __forceinline__ double2 load16(const double2 *g)
 {
     const __attribute__((address_space(1))) double *p = (const __attribute__((address_space(1))) double *)g;

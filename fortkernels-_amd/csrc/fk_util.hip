@@ -49,7 +49,7 @@ Scratch::~Scratch()
     if (owned_ && base_) (void)hipFreeAsync(base_, stream_);
 }
 
-int Scratch::acquire(void *user, size_t user_bytes, hipStream_t stream)
+int Scratch::acquire(void *user, size_t user_bytes, hipStream_t stream, size_t align)
 {
     stream_ = stream;
     if (total_ == 0) return FK_OK;
@@ -58,9 +58,11 @@ int Scratch::acquire(void *user, size_t user_bytes, hipStream_t stream)
             set_error("workspace of %zu bytes is smaller than the %zu bytes needed", user_bytes, total_);
             return FK_ERR_WORKSPACE;
         }
-        base_ = user;
-        owned_ = false;
-        return FK_OK;
+        if (reinterpret_cast<uintptr_t>(user) % align == 0) {
+            base_ = user;
+            owned_ = false;
+            return FK_OK;
+        }
     }
     hipError_t e = hipMallocAsync(&base_, total_, stream);
     if (e != hipSuccess) {

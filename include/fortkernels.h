@@ -87,7 +87,11 @@ typedef struct {
     int32_t device;          /* HIP device ordinal for FK_MEM_HOST (-1 = current) */
     void *stream;            /* hipStream_t; NULL = the null stream */
     void *workspace;         /* device scratch; NULL = allocated per call
-                                (stream-ordered) */
+                                (stream-ordered).  Any 8-byte aligned address
+                                serves; from a 16-byte aligned one the FP64
+                                kernels move it straight into LDS.  The
+                                int8-split GPP path needs 16 and allocates per
+                                call otherwise. */
     size_t workspace_bytes;
     int32_t config;          /* kernel tile configuration; 0 = choose by shape */
     float *kernel_ms;        /* if non-NULL: the call times its dominant kernel
