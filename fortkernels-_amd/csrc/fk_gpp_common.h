@@ -79,34 +79,29 @@ __device__ __forceinline__ double pole_wdiffr(double wdr, double wdi)
     return wdr * wdr + wdi * wdi;
 }
 
+// The sum over the wave in every lane: lanes l and l ^ 1 first, then l ^ 2, ...
 __device__ __forceinline__ double wave_sum(double v)
 {
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
+    for (int off = 1; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
     return v;
 }
 
-// Sums of N <= 16 values over the wave through `buf`, 65 P doubles of LDS of
-// its own (P = N rounded up to 8 or 16): lane q < N returns the total of value
-// q.  Lane q + P h adds value q of lanes P h .. P h + P - 1, then the parts
-// meet: for 16 values 16 writes, 16 reads and 18 additions where 16 butterflies
-// take 192 shuffles and 96 additions (13312 tiles of 12 values: 0.05 ms less).
-// A fixed order.
-template <int N>
-__device__ __forceinline__ double wave_sums_lds(const double (&v)[N], int lane, double *buf)
+// Sums of 8 values over the wave through `buf`, 8 * 65 doubles of LDS of its own:
+// lane q < 8 returns wave_sum(v[q]), the same bits.  Lane q + 8 h adds value q of
+// lanes 8 h .. 8 h + 7, pairs first, then the parts meet: 8 writes, 8 reads and 10
+// additions where 8 butterflies take 96 shuffles and 48 additions (13312 tiles
+// of 12 values: 0.05 ms less).
+__device__ __forceinline__ double wave_sums_lds(const double (&v)[8], int lane, double *buf)
 {
-    constexpr int P = N <= 8 ? 8 : 16;
-    static_assert(N <= 16, "one value per lane of a part");
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-    for (int q = 0; q < N; ++q) buf[q * 65 + lane] = v[q];
+    for (int q = 0; q < 8; ++q) buf[q * 65 + lane] = v[q];
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    const double *p = buf + (lane & (P - 1)) * 65 + (lane & ~(P - 1));
-    double x = 0.0;
+    const double *p = buf + (lane & 7) * 65 + (lane & ~7);
+    double x = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
 #pragma unroll
-    for (int k = 0; k < P; ++k) x += p[k];
-#pragma unroll
-    for (int off = P; off < 64; off <<= 1) x += __shfl_xor(x, off, 64);
+    for (int off = 8; off < 64; off <<= 1) x += __shfl_xor(x, off, 64);
     return x;
 }
 
