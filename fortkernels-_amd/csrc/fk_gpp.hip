@@ -604,7 +604,9 @@ __device__ __forceinline__ void gpp_ring_tile(const GppArgs<double2> &a, int tm,
             for (int ks = 0; ks < nko; ++ks) {
                 ring::Frags<1, 1> f;
                 f.a[0] = gld<TABLE>(a.c, (size_t)(4 * ks + kp) * a.ldc + rowbase + 16 * i + cp);
-                f.b[0] = gld<TABLE>(a.aqsn, (size_t)min(4 * ks + kp, a.nb - 1) * a.C + min(col, nmax));
+                // (a zero row of c past the last occupied band meets an occupied
+                // band: asxtemp depends on no other, infinities included)
+                f.b[0] = gld<TABLE>(a.aqsn, (size_t)min(4 * ks + kp, a.nv - 1) * a.C + min(col, nmax));
                 o.mma(f);
             }
 #pragma unroll

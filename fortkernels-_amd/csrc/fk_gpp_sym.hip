@@ -407,7 +407,7 @@ __global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
                 o.zero();
                 for (int ks = 0; ks < nko; ++ks) {
                     ring::Frags<1, 2> f;
-                    const size_t rb = (size_t)min(4 * ks + kp, a.nb - 1) * a.C + min(col, nmax);
+                    const size_t rb = (size_t)min(4 * ks + kp, a.nv - 1) * a.C + min(col, nmax);   // occupied bands only (gpp_ring_tile)
                     f.a[0] = a.c[(size_t)(4 * ks + kp) * a.ldc + rowbase + 16 * i + cp];
                     f.b[0] = a.aqsn[rb];
                     f.b[1] = a.aqsm[rb];
