@@ -185,7 +185,8 @@ __device__ __forceinline__ double2 cmul_fused(double2 a, double2 b)
 // near-pole test |delw|^2 > to1 from |u|^2 <= limittwo when |wtilde|^2 >
 // 1.01 to1 limittwo (u = 0, where |delw|^2 is a NaN, adds nothing).  Other
 // elements (|wtilde| outside 5e-4 .. 249 with the default limits, NaNs), and
-// all with the mask off, return false and are left to pole_element.
+// all with the mask off, return false and are left to pole_element.  So are those
+// whose Bo is not finite: 0 Bo, added where the mask is off, is a NaN then.
 //
 // The branches are taken under the execution mask: with selected factors instead
 // (five more operations, no branch) every kernel that uses this is slower, by 7%
@@ -202,11 +203,11 @@ __device__ __forceinline__ bool pole_terms(const PoleParams &pp, Table wx, Table
 #pragma clang fp contract(off)
     const double wy2 = wt.y * wt.y;
     const double wt2 = __builtin_fma(wt.x, wt.x, wy2);
-    if (!(wt2 > pp.lo && wt2 < pp.hi)) return false;
     const double2 T = cmul_fused(ie, wt), P = cmul_fused(B, T);
     const double2 PQ = make_double2(P.y * wt.y, P.x * wt.y);
     const double2 BoOm = cmul_fused(Bo, cmul_fused(T, wt));
     const double2 R = cmul_fused(Bo, make_double2(-0.5 * T.x, -0.5 * T.y));
+    if (!(wt2 > pp.lo && wt2 < pp.hi && fabs(R.x + R.y) < __builtin_inf())) return false;
     const double2 RQ = make_double2(R.y * wt.y, R.x * wt.y);
 #pragma unroll
     for (int q = 0; q < NWC; ++q) {

@@ -245,7 +245,8 @@ __device__ __forceinline__ bool sym_terms(const SymArgs &a, int w0, SymElem e, d
 #pragma clang fp contract(off)
     const double wy2 = wt.y * wt.y;
     const double wt2 = __builtin_fma(wt.x, wt.x, wy2);
-    bool fast = wt2 > a.lo && wt2 < a.hi;
+    // 0 Bo near the pole is a NaN where Bo is not finite
+    bool fast = wt2 > a.lo && wt2 < a.hi && fabs((Bo.x + Bo.y) + (Bpo.x + Bpo.y)) < __builtin_inf();
 #pragma unroll
     for (int q = 0; q < NWC; ++q) {
         const double wdr = a.wx[min(w0 + q, a.nw - 1)] - wt.x, d = wdr * wdr + wy2;

@@ -45,3 +45,23 @@ def test_an_unoccupied_band_leaves_asxtemp_alone(fk, fko, form, nv, bad):
     ach, asx = _run(fk, p, form)
     assert not np.all(np.isfinite(ach.real))
     assert np.max(np.abs(asx - clean)) <= 1e-12 * np.max(np.abs(clean))
+
+
+@pytest.mark.parametrize("form,occupied", [("small", True), ("large", True), ("batch", True), ("gppsum", True),
+                                           ("small", False), ("large", False), ("batch", False)])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_a_band_element_near_the_pole(fk, fko, form, occupied, bad):
+    """One element of aqsn is not finite and every factor that it meets is near the
+    pole at frequency 0, where sch = 0: an occupied band adds 0 times it (a NaN), an
+    unoccupied one is left out.  (The sequential program adds 0 times it in the
+    gppsum = 1 form, which the library has always left out: not compared.)"""
+    p = fko.gpp_random(20, 3, 300, 70, seed=3, wtilde_re=(0.5, 2.0))
+    ig = 33
+    p.aqsn[1 if occupied else 9, ig] = bad
+    p.wtilde[:, ig] = p.wx[0] + 0.1
+    ref, got = _oracle(fko, p, form), _run(fk, p, form)
+    for g, r in zip(got, ref):
+        assert np.array_equal(np.isfinite(g), np.isfinite(r)), (g, r)
+        ok = np.isfinite(r)
+        assert np.all(np.abs(g[ok] - r[ok]) <= 1e-12 * np.max(np.abs(r[ok]), initial=0.0))
+    assert not np.all(np.isfinite(ref[0]))
