@@ -35,9 +35,20 @@ inline PoleParams make_pole_params(const double *wx, int nfreq, double limittwo,
     pp.mask_on = mask_on ? 1 : 0;
     pp.nw = nfreq;
     pp.lo = pp.hi = 0.0;
-    if (mask_on && limittwo > 0.0 && limitone > 0.0 && to1 == to1) {
+    if (limittwo > 0.0 && limitone > 0.0 && to1 == to1) {
         pp.lo = 1.01 * (to1 > 0.0 ? to1 : 0.0) * limittwo;
         pp.hi = 0.99 * limitone * limittwo;
+        // |wtilde| so far from every frequency that the mask is on at each
+        double near = INFINITY, far = 0.0;      // the smallest and largest |wx|
+        for (int iw = 0; iw < nfreq; ++iw) {
+            near = !(std::fabs(wx[iw]) >= near) ? std::fabs(wx[iw]) : near;
+            far = !(std::fabs(wx[iw]) <= far) ? std::fabs(wx[iw]) : far;
+        }
+        const double pole = std::sqrt(1.01 * limittwo), below = near - pole;
+        const double above = std::max(far + pole, far / (1.0 - std::sqrt(1.01 / limitone)));
+        const double lo = pp.lo, hi = pp.hi;
+        if (lo < hi && below > 0.0 && below * below > 1.01 * lo) pp.lo = -1.0;
+        if (limitone > 1.02 && above * above < 0.99 * hi) pp.hi = 1e300;
     }
     for (int iw = 0; iw < kMaxFreq; ++iw) {
         const double w = iw < nfreq ? wx[iw] : 0.0;
@@ -183,10 +194,13 @@ __device__ __forceinline__ double2 cmul_fused(double2 a, double2 b)
 // reference rounds it): the mask's second test |delw|^2 < limitone follows
 // from |u|^2 > limittwo when |wtilde|^2 < 0.99 limitone limittwo, and the
 // near-pole test |delw|^2 > to1 from |u|^2 <= limittwo when |wtilde|^2 >
-// 1.01 to1 limittwo (u = 0, where |delw|^2 is a NaN, adds nothing).  Other
-// elements (|wtilde| outside 5e-4 .. 249 with the default limits, NaNs), and
-// all with the mask off, return false and are left to pole_element.  So are those
-// whose Bo is not finite: 0 Bo, added where the mask is off, is a NaN then.
+// 1.01 to1 limittwo (u = 0, where |delw|^2 is a NaN, adds nothing).  That is 5e-4 ..
+// 249 with the default limits.  A larger |wtilde| keeps the mask on where |u| >=
+// |wtilde| - |wx| alone is beyond both lines at every frequency, a smaller one
+// where |wx| - |wtilde| is, so with every |wx| between 0.51 and 248 the range has
+// no end; a wtilde of 0 (padding) adds nothing but zeros anywhere.  Other elements,
+// NaNs and those whose Bo is not finite (0 Bo, added where the mask is off, is a
+// NaN then) return false and are left to pole_element.
 //
 // The branches are taken under the execution mask: with selected factors instead
 // (five more operations, no branch) every kernel that uses this is slower, by 7%
@@ -207,7 +221,7 @@ __device__ __forceinline__ bool pole_terms(const PoleParams &pp, Table wx, Table
     const double2 PQ = make_double2(P.y * wt.y, P.x * wt.y);
     const double2 BoOm = cmul_fused(Bo, cmul_fused(T, wt));
     const double2 R = cmul_fused(Bo, make_double2(-0.5 * T.x, -0.5 * T.y));
-    if (!(wt2 > pp.lo && wt2 < pp.hi && fabs(R.x + R.y) < __builtin_inf())) return false;
+    if (!((wt2 > pp.lo || wt2 == 0.0) && wt2 < pp.hi && fabs(R.x + R.y) < __builtin_inf())) return false;
     const double2 RQ = make_double2(R.y * wt.y, R.x * wt.y);
 #pragma unroll
     for (int q = 0; q < NWC; ++q) {
@@ -225,6 +239,22 @@ __device__ __forceinline__ bool pole_terms(const PoleParams &pp, Table wx, Table
             const double rs = du > 0.0 ? r : 0.0;
             sasx[q].x = __builtin_fma(__builtin_fma(R.x, ys, RQ.x), rs, sasx[q].x);
             sasx[q].y = __builtin_fma(__builtin_fma(R.y, ys, -RQ.y), rs, sasx[q].y);
+        }
+    }
+    if (!pp.mask_on) {
+        // B D where the mask would be off.  Opaque: otherwise the |u|^2 of the loop
+        // above are kept for this one.
+        double x = wt.x, y2 = wy2;
+        asm volatile("" : "+v"(x), "+v"(y2));
+#pragma unroll
+        for (int q = 0; q < NWC; ++q) {
+            if (!ALL && q > 0 && w0 + q >= pp.nw) break;
+            const double yu = wx[w0 + q] - x, du = yu * yu + y2;
+            if (!(du > pp.limittwo)) {
+                const double r = rcp_cubic(du);
+                sach[q].x = __builtin_fma(__builtin_fma(P.x, yu, -PQ.x), r, sach[q].x);
+                sach[q].y = __builtin_fma(__builtin_fma(P.y, yu, PQ.y), r, sach[q].y);
+            }
         }
     }
     return true;
