@@ -288,6 +288,7 @@ struct SymLds {
     };
     double red[4][4 * kSymNwc];
     double tot[kMaxFreq * 4];
+    int last;                                    // the largest igp of the row block
 };
 
 // A 64 x 32 tile of (my_igp, ig) with both right operands side by side: 32
@@ -305,6 +306,10 @@ struct SymLds {
 //
 // Only the tiles with some ig <= igp have a workgroup: the host lists them by
 // row block (`per` of them in one workgroup where there are more than partials).
+// Past kSymBlocks row blocks all tiles have one and those with none end at once,
+// row blocks fastest (the kernel at 64/2/2000/40000: 1.39 ms with igp spread over
+// all G-vectors, 0.11 with every igp below 64; with every tile evaluated, tile
+// columns fastest, 2.33 and 2.28).
 // Measured at 256/4/16384/819, 3 frequencies: the call 640 us, with contiguous ranges
 // of 64 x 64 tiles per XCD, half of them empty, two workgroups per CU and every
 // quotient and hypot evaluated 1486.
@@ -315,9 +320,9 @@ __global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave & 1, wn = wave >> 1;
     int tm, h0;
-    if (a.every > 0) {
-        tm = blockIdx.x / a.every;
-        h0 = (blockIdx.x - tm * a.every) * a.per;
+    if (a.every > 0) {                             // row blocks fastest: few tile columns spread over all XCDs
+        tm = blockIdx.x % a.nblk;
+        h0 = (int)blockIdx.x / a.nblk * a.per;
     } else {
         int lo = 0, hi = a.nblk - 1;               // last row block with first <= this workgroup
         while (lo < hi) {
@@ -331,7 +336,14 @@ __global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
     const int rowbase = tm * kSymTile + wm * 32, nmax = a.C - 1;
     const int kl = lane >> 4, cl = lane & 15;
     if (tid < kMaxFreq * 4) sh.tot[tid] = 0.0;
+    if (a.every > 0 && wave == 0) {              // not listed: some of the tiles have no ig <= igp
+        int g = tm * kSymTile + lane < a.G ? a.igp[tm * kSymTile + lane] : -1;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) g = max(g, __shfl_xor(g, off, 64));
+        if (lane == 0) sh.last = min(g, nmax);
+    }
     __syncthreads();
+    const int n_last = a.every > 0 ? __builtin_amdgcn_readfirstlane(sh.last) : nmax;
 
     const bool side_a = wave < 2;
     const int k0 = 4 * (wave & 1);
@@ -342,7 +354,7 @@ __global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
     const bool direct = a.aligned & (side_a ? 1 : 2);
     const int nko = (a.nv + 3) / 4;
 
-    for (int n0 = h0 * kSymCols; n0 < (h0 + a.per) * kSymCols && n0 <= nmax; n0 += kSymCols) {
+    for (int n0 = h0 * kSymCols; n0 < (h0 + a.per) * kSymCols && n0 <= n_last; n0 += kSymCols) {
         // ---- GEMM over the unoccupied bands: Bu (right operand aqsn), Bu' (aqsm)
         const int lcol = min(n0 + (lane & 31), nmax);
         const double2 *src = side_a ? a.c + tm * kSymTile + lane : (lane < 32 ? a.aqsn : a.aqsm) + lcol;
