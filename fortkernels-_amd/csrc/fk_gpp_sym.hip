@@ -47,8 +47,8 @@ using namespace gpp;
 
 constexpr int kSymTile = 64, kSymCols = 32;   // rows and columns of a tile
 constexpr int kSymBlocks = 512;  // row blocks whose tiles the kernel arguments can list
-constexpr int kSymNwc = 3;       // frequencies per epilogue pass
 constexpr int kSymStages = 3, kSymWgs = 3;   // ring stages, workgroups per CU
+constexpr int kSymWide = 256;    // workgroups of two tiles side by side, at most
 
 // std::complex<double> product and quotient as the reference rounds them.
 __device__ __forceinline__ double2 zmul(double2 a, double2 b)
@@ -281,12 +281,13 @@ __device__ __forceinline__ bool sym_terms(const SymArgs &a, int w0, SymElem e, d
     return true;
 }
 
+template <int NWC, int NG>
 struct SymLds {
     union {
         double2 ring[kSymStages][2][8][64];      // [slot][coefficients; aqsn, aqsm][k][column]
         double2 b[4][3][4][64];                  // [wave][block - 1][register][lane]
-    };
-    double red[4][4 * kSymNwc];
+    } tile[NG];
+    double red[4 * NG][4 * NWC];
     double tot[kMaxFreq * 4];
     int last;                                    // the largest igp of the row block
 };
@@ -313,11 +314,24 @@ struct SymLds {
 // Measured at 256/4/16384/819, 3 frequencies: the call 640 us, with contiguous ranges
 // of 64 x 64 tiles per XCD, half of them empty, two workgroups per CU and every
 // quotient and hypot evaluated 1486.
-__global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
+//
+// NWC frequencies per epilogue pass: 4 where that takes fewer passes than 3
+// (84/0/405/16 with 4 frequencies 41 us, in two passes 60; 422/13/14154/2971 with 16
+// 4.2 ms, in six passes 4.5), else 3, which spills nothing (39/5/306/43 with 5
+// frequencies 71 us, with 4 per pass 77).
+//
+// NG = 2: two tiles of a workgroup side by side on eight waves, for calls with two
+// tiles per workgroup that do not fill the GPU (a few row blocks): 800/0/4000/50,
+// the kernel 222 us, one after the other 256 (two workgroups would take 130, but the
+// workspace holds a partial for each 64 x 64 tile only).
+template <int NWC, int NG>
+__global__ __launch_bounds__(256 * NG, NG == 1 ? kSymWgs : 1) void gpp_sym_kernel(SymArgs a)
 {
-    constexpr int MB = 2, NB = 2, NWAVES = 4, LPW = 4;
-    __shared__ SymLds sh;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int MB = 2, NB = 2, NWAVES = 4 * NG, LPW = 4;
+    __shared__ SymLds<NWC, NG> lds;
+    const int tid = threadIdx.x, lane = tid & 63, wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = wave_id & 3, group = wave_id >> 2;
+    auto &sh = lds.tile[group];
     const int wm = wave & 1, wn = wave >> 1;
     int tm, h0;
     if (a.every > 0) {                             // row blocks fastest: few tile columns spread over all XCDs
@@ -335,15 +349,15 @@ __global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
     }
     const int rowbase = tm * kSymTile + wm * 32, nmax = a.C - 1;
     const int kl = lane >> 4, cl = lane & 15;
-    if (tid < kMaxFreq * 4) sh.tot[tid] = 0.0;
-    if (a.every > 0 && wave == 0) {              // not listed: some of the tiles have no ig <= igp
+    if (tid < kMaxFreq * 4) lds.tot[tid] = 0.0;
+    if (a.every > 0 && wave_id == 0) {              // not listed: some of the tiles have no ig <= igp
         int g = tm * kSymTile + lane < a.G ? a.igp[tm * kSymTile + lane] : -1;
 #pragma unroll
         for (int off = 1; off < 64; off <<= 1) g = max(g, __shfl_xor(g, off, 64));
-        if (lane == 0) sh.last = min(g, nmax);
+        if (lane == 0) lds.last = min(g, nmax);
     }
     __syncthreads();
-    const int n_last = a.every > 0 ? __builtin_amdgcn_readfirstlane(sh.last) : nmax;
+    const int n_last = a.every > 0 ? __builtin_amdgcn_readfirstlane(lds.last) : nmax;
 
     const bool side_a = wave < 2;
     const int k0 = 4 * (wave & 1);
@@ -354,7 +368,9 @@ __global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
     const bool direct = a.aligned & (side_a ? 1 : 2);
     const int nko = (a.nv + 3) / 4;
 
-    for (int n0 = h0 * kSymCols; n0 < (h0 + a.per) * kSymCols && n0 <= n_last; n0 += kSymCols) {
+    // (a second group past the last column has clamped ones and adds nothing)
+    for (int h = h0; h < h0 + a.per && h * kSymCols <= n_last; h += NG) {
+        const int n0 = (h + group) * kSymCols;
         // ---- GEMM over the unoccupied bands: Bu (right operand aqsn), Bu' (aqsm)
         const int lcol = min(n0 + (lane & 31), nmax);
         const double2 *src = side_a ? a.c + tm * kSymTile + lane : (lane < 32 ? a.aqsn : a.aqsm) + lcol;
@@ -396,10 +412,10 @@ __global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
                 if (k == 0) Bu0[r] = v;
                 else sh.b[wave][k - 1][r][lane] = v;
             }
-        for (int w0 = 0; w0 < a.nw; w0 += kSymNwc) {
-            double2 sach[kSymNwc], sasx[kSymNwc];
+        for (int w0 = 0; w0 < a.nw; w0 += NWC) {
+            double2 sach[NWC], sasx[NWC];
 #pragma unroll
-            for (int q = 0; q < kSymNwc; ++q) { sach[q] = make_double2(0.0, 0.0); sasx[q] = make_double2(0.0, 0.0); }
+            for (int q = 0; q < NWC; ++q) { sach[q] = make_double2(0.0, 0.0); sasx[q] = make_double2(0.0, 0.0); }
             unsigned general = 0;
             int kp = kl, cp = cl;      // opaque in each pass (gpp_ring_tile)
             asm volatile("" : "+v"(kp), "+v"(cp));
@@ -437,7 +453,7 @@ __global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
                     if (e.kind || e.occ) {
                         const double2 Bu = i == 0 ? Bu0[r] : sh.b[wave][1][r][lane];
                         const double2 Bp = sh.b[wave][2 * i][r][lane];
-                        if (!sym_terms<kSymNwc>(a, w0, e, cwt[r], cie[r], Bu, Bp, o.value(0, 0, r), o.value(0, 1, r), sach,
+                        if (!sym_terms<NWC>(a, w0, e, cwt[r], cie[r], Bu, Bp, o.value(0, 0, r), o.value(0, 1, r), sach,
                                                 sasx))
                             general |= 1u << (4 * i + r);
                     }
@@ -465,37 +481,37 @@ __global__ __launch_bounds__(256, kSymWgs) void gpp_sym_kernel(SymArgs a)
                             Bpo = cfma(Bpo, cn, a.aqsm[(size_t)n1 * a.C + col]);
                         }
                         const size_t x = (size_t)row * a.C + col;
-                        sym_element<kSymNwc>(a, w0, sym_elem(a, row, col), a.wtilde[x], a.I_eps[x], Bu, Bp, Bo, Bpo, sach,
+                        sym_element<NWC>(a, w0, sym_elem(a, row, col), a.wtilde[x], a.I_eps[x], Bu, Bp, Bo, Bpo, sach,
                                              sasx);
                     }
                 }
             }
             // wave reduction, then a fixed-order sum over the waves and tiles
-            double v[4 * kSymNwc];
+            double v[4 * NWC];
 #pragma unroll
-            for (int q = 0; q < kSymNwc; ++q) {
+            for (int q = 0; q < NWC; ++q) {
                 v[4 * q + 0] = sach[q].x;
                 v[4 * q + 1] = sach[q].y;
                 v[4 * q + 2] = sasx[q].x;
                 v[4 * q + 3] = sasx[q].y;
             }
 #pragma unroll
-            for (int q = 0; q < 4 * kSymNwc; ++q) {
+            for (int q = 0; q < 4 * NWC; ++q) {
                 const double x = wave_sum(v[q]);
-                if (lane == 0) sh.red[wave][q] = x;
+                if (lane == 0) lds.red[wave_id][q] = x;
             }
             __syncthreads();
-            if (tid < 4 * kSymNwc && w0 + (tid >> 2) < a.nw) {
-                double sum = sh.red[0][tid];
+            if (tid < 4 * NWC && w0 + (tid >> 2) < a.nw) {
+                double sum = lds.red[0][tid];
 #pragma unroll
-                for (int w = 1; w < NWAVES; ++w) sum += sh.red[w][tid];
-                sh.tot[4 * w0 + tid] += sum;
+                for (int w = 1; w < NWAVES; ++w) sum += lds.red[w][tid];
+                lds.tot[4 * w0 + tid] += sum;
             }
             __syncthreads();
         }
     }
     __syncthreads();
-    for (int k = tid; k < 4 * a.nw; k += 256) reinterpret_cast<double *>(a.partials + (size_t)blockIdx.x * a.nw * 2)[k] = sh.tot[k];
+    if (tid < 4 * a.nw) reinterpret_cast<double *>(a.partials + (size_t)blockIdx.x * a.nw * 2)[tid] = lds.tot[tid];
 }
 
 }  // namespace
@@ -546,7 +562,16 @@ int gpp_sym_launch(const fk_gpp_problem *p, const std::vector<int32_t> &cols, co
     for (int iw = 0; iw < kMaxFreq; ++iw) a.wx[iw] = iw < p->nfreq ? p->wx[iw] : 0.0;
     KernelTimer timer(kernel_ms, s);
     FK_TRY(timer.start());
-    if (blocks > 0) hipLaunchKernelGGL(gpp_sym_kernel, dim3(blocks), dim3(256), 0, s, a);
+    if (blocks > 0) {
+        const bool four = div_up(p->nfreq, 4) < div_up(p->nfreq, 3);
+        if (a.per == 2 && blocks <= kSymWide) {
+            if (four) hipLaunchKernelGGL((gpp_sym_kernel<4, 2>), dim3(blocks), dim3(512), 0, s, a);
+            else hipLaunchKernelGGL((gpp_sym_kernel<3, 2>), dim3(blocks), dim3(512), 0, s, a);
+        } else {
+            if (four) hipLaunchKernelGGL((gpp_sym_kernel<4, 1>), dim3(blocks), dim3(256), 0, s, a);
+            else hipLaunchKernelGGL((gpp_sym_kernel<3, 1>), dim3(blocks), dim3(256), 0, s, a);
+        }
+    }
     FK_HIP(hipGetLastError());
     FK_TRY(timer.stop());
     return timer.finish();
