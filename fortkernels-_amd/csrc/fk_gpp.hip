@@ -945,13 +945,30 @@ void launch_fused(int cfg, int tiles, hipStream_t s, const GppArgs<E> &a)
 // cost nothing that could be measured against 4).
 bool ring_form(int cfg, size_t elem, int nv) { return cfg == 1 && elem == sizeof(double2) && nv <= kRingOcc; }
 
+// ring_idle: long band loops on a GPU that the 64 x 64 tiles do not fill.  With one
+// workgroup on a CU, one wave on a SIMD, nothing runs while the ring's barriers are
+// met, and gpp_tile, which has none, is faster by more than its longer epilogue
+// costs.  Time of the ring over gpp_tile's by tiles, bands and frequencies: 256
+// tiles 200 bands 1.09 (1 frequency), 0.94 (3); 400 bands 1.08, 0.98; 900 bands 1.08,
+// 1.02; 2000 bands 1.08, 1.05.  264 to 512 tiles (two workgroups on a CU): 200 bands
+// 1.01, 0.89; 900 bands 1.02, 0.97; 2000 bands 1.03, 1.00.  528 and more: below 1.
+//
 // 32 x 32 tiles, for calls of few 64 x 64 tiles: four times the workgroups, a
 // quarter of the epilogue in each, at about 0.8 of the larger tiles' rate once the
 // GPU is full.  Time of the 64 x 64 tiles over that of these, by tiles (64 x 64)
 // and bands: 128 tiles 1.8 at 32 bands to 1.53 at 1000; 256 tiles 1.37, 1.16 (130
 // bands), 0.99 (400), 0.93; 384 tiles 1.23, 1.13, 1.08, 0.99; 512 tiles 1.13, 0.97,
 // 0.86; 640 tiles 1.06, 0.98, 0.93; 768 tiles 0.98, 0.87.
-bool ring_small(int tiles64, int nb) { return tiles64 <= (nb <= 48 ? 640 : nb <= 160 ? 384 : 255); }
+// Past 192 tiles four 32 x 32 tiles meet on some CUs: ring_idle's calls are left to it.
+bool ring_idle(int tiles64, int nb, int nw)
+{
+    return tiles64 <= 256 ? nb > 275 * nw - 215 : tiles64 <= 512 && nb > 700 * nw - 600;
+}
+bool ring_small(int tiles64, int nb, int nw)
+{
+    if (nb <= 160) return tiles64 <= (nb <= 48 ? 640 : 384);
+    return tiles64 <= 192 || (tiles64 <= 255 && !ring_idle(tiles64, nb, nw));
+}
 
 template <int MB, bool ACHS>
 void launch_ring_mb(int tiles, hipStream_t s, const GppArgs<double2> &a)
@@ -1003,7 +1020,9 @@ Layout plan_layout(const fk_gpp_problem *p, const fk_options *o, Scratch &ws, si
     L.ring = 0;
     if (!sym && ring_form(L.cfg, elem, p->nvband)) {
         const int64_t tiles64 = (int64_t)div_up(p->ngpown, 64) * div_up(p->ncouls, 64);
-        L.ring = o->config == 0 && tiles64 <= 1024 && ring_small((int)tiles64, p->number_bands) ? 32 : 64;
+        const int tiles = (int)std::min<int64_t>(tiles64, 1 << 20);
+        if (o->config == 0 && ring_small(tiles, p->number_bands, p->nfreq)) L.ring = 32;
+        else L.ring = ring_idle(tiles, p->number_bands, p->nfreq) ? 0 : 64;
     }
     const int bm = L.ring ? L.ring : t.bm, bn = L.ring ? L.ring : t.bn;
     const int kstep = L.ring ? 8 : 4 * t.p;
