@@ -505,8 +505,8 @@ struct RingLds {
 };
 
 // MB x MB blocks per wave: 64 x 64 tiles (MB = 2) or 32 x 32.  ALL: nw == NWC,
-// one epilogue pass.
-template <int MB, int NWC, bool ALL, bool ACHS, bool TABLE>
+// one epilogue pass.  MASK: pp.mask_on.
+template <int MB, int NWC, bool ALL, bool ACHS, bool MASK, bool TABLE>
 __device__ __forceinline__ void gpp_ring_tile(const GppArgs<double2> &a, int tm, int tn, RingLds<MB, NWC> &sh)
 {
     constexpr int NB = MB, T = 32 * MB, NWAVES = 4;
@@ -615,7 +615,7 @@ __device__ __forceinline__ void gpp_ring_tile(const GppArgs<double2> &a, int tm,
                 if (((rowok >> (i * 4 + r)) & 1u) && col <= nmax) {
                     const double2 Bo = o.value(0, 0, r);
                     const double2 B = cadd(k == 0 ? Bu0[r] : sh.bu[wave][k > 0 ? k - 1 : 0][r][lane], Bo);
-                    if (!pole_terms<NWC, ALL>(a.pp, a.pp.pc.wx, a.pp.pc.iwx2, w0, cwt[r], cie[r], B, Bo, sach, sasx))
+                    if (!pole_terms<NWC, ALL, MASK>(a.pp, a.pp.pc.wx, a.pp.pc.iwx2, w0, cwt[r], cie[r], B, Bo, sach, sasx))
                         general |= 1u << (k * 4 + r);
                     if constexpr (ACHS) {
                         if (w0 == 0) sachs = csub(sachs, cmul(B, cie[r]));
@@ -704,7 +704,7 @@ __device__ __forceinline__ void gpp_ring_tile(const GppArgs<double2> &a, int tm,
     }
 }
 
-template <int MB, int NWC, bool ALL, bool ACHS>
+template <int MB, int NWC, bool ALL, bool ACHS, bool MASK>
 __global__ __launch_bounds__(256, MB == 2 ? kRingWgs : kRingSmallWgs) void gpp_ring_kernel(GppArgs<double2> a)
 {
     __shared__ RingLds<MB, NWC> sh;
@@ -716,7 +716,7 @@ __global__ __launch_bounds__(256, MB == 2 ? kRingWgs : kRingSmallWgs) void gpp_r
     }
     int tm, tn;
     tile_coords(blockIdx.x, a.tiles_m, a.tiles_n, a.group_m, tm, tn);
-    gpp_ring_tile<MB, NWC, ALL, ACHS, false>(a, tm, tn, sh);
+    gpp_ring_tile<MB, NWC, ALL, ACHS, MASK, false>(a, tm, tn, sh);
 }
 
 // One problem, one tile per workgroup.
@@ -769,6 +769,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINW) void gpp_batch_kernel(const G
 }
 
 // The same for gpp_ring_tile (problems with at most kRingOcc occupied bands).
+template <bool MASK>
 __global__ __launch_bounds__(256, kRingWgs) void gpp_ring_batch_kernel(const GppArgs<double2> *__restrict__ probs,
                                                                        const BatchTile *__restrict__ tiles, int ntiles,
                                                                        int *counter)
@@ -784,7 +785,7 @@ __global__ __launch_bounds__(256, kRingWgs) void gpp_ring_batch_kernel(const Gpp
         const BatchTile bt = tiles[t];
         const int prob = __builtin_amdgcn_readfirstlane(bt.prob);
         const int tm = __builtin_amdgcn_readfirstlane(bt.tm), tn = __builtin_amdgcn_readfirstlane(bt.tn);
-        gpp_ring_tile<2, ring_nwc(2, false), false, false, true>(probs[prob], tm, tn, sh);
+        gpp_ring_tile<2, ring_nwc(2, false), false, false, MASK, true>(probs[prob], tm, tn, sh);
     }
 }
 
@@ -973,14 +974,17 @@ bool ring_small(int tiles64, int nb, int nw)
 template <int MB, bool ACHS>
 void launch_ring_mb(int tiles, hipStream_t s, const GppArgs<double2> &a)
 {
+    constexpr int kNwc = ring_nwc(MB, ACHS);
+    const dim3 grid(tiles), block(256);
+    if (!a.pp.mask_on) {
+        hipLaunchKernelGGL((gpp_ring_kernel<MB, kNwc, false, ACHS, false>), grid, block, 0, s, a);
+        return;
+    }
     switch (a.nw) {
-    case 1: hipLaunchKernelGGL((gpp_ring_kernel<MB, 1, true, ACHS>), dim3(tiles), dim3(256), 0, s, a); break;
-    case 2: hipLaunchKernelGGL((gpp_ring_kernel<MB, 2, true, ACHS>), dim3(tiles), dim3(256), 0, s, a); break;
-    case 3: hipLaunchKernelGGL((gpp_ring_kernel<MB, 3, true, ACHS>), dim3(tiles), dim3(256), 0, s, a); break;
-    default:
-        hipLaunchKernelGGL((gpp_ring_kernel<MB, ring_nwc(MB, ACHS), false, ACHS>), dim3(tiles), dim3(256),
-                           0, s, a);
-        break;
+    case 1: hipLaunchKernelGGL((gpp_ring_kernel<MB, 1, true, ACHS, true>), grid, block, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((gpp_ring_kernel<MB, 2, true, ACHS, true>), grid, block, 0, s, a); break;
+    case 3: hipLaunchKernelGGL((gpp_ring_kernel<MB, 3, true, ACHS, true>), grid, block, 0, s, a); break;
+    default: hipLaunchKernelGGL((gpp_ring_kernel<MB, kNwc, false, ACHS, true>), grid, block, 0, s, a); break;
     }
 }
 
@@ -1549,8 +1553,9 @@ struct GppBatch {
         bool done = false;
         if constexpr (sizeof(E) == sizeof(double2)) {
             if (ring(cfg)) {
-                hipLaunchKernelGGL(gpp_ring_batch_kernel, dim3(ncu * kRingWgs), dim3(256), 0, s, args, tiles, ntiles,
-                                   counter);
+                const dim3 grid(ncu * kRingWgs), block(256);
+                if (opt.mask) hipLaunchKernelGGL(gpp_ring_batch_kernel<true>, grid, block, 0, s, args, tiles, ntiles, counter);
+                else hipLaunchKernelGGL(gpp_ring_batch_kernel<false>, grid, block, 0, s, args, tiles, ntiles, counter);
                 done = true;
             }
         }
@@ -1729,7 +1734,7 @@ struct OzBatch {
     {
         const int *first = reinterpret_cast<const int *>(at(off_first));
         FK_TRY(gpp_oz_batch_launch(at(off_rec), first, first + (n + 1), first + 2 * (n + 1), n, total_prep, total_gemm,
-                                   total_pole, s));
+                                   total_pole, opt.mask != 0, s));
         hipLaunchKernelGGL(gpp_reduce_batch_kernel, dim3(2 * kMaxFreq, n), dim3(256), 0, s,
                            reinterpret_cast<const ReduceBatch *>(at(off_red)), reinterpret_cast<double2 *>(at(off_out)));
         FK_HIP(hipGetLastError());

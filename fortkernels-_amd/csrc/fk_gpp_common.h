@@ -208,8 +208,9 @@ __device__ __forceinline__ double2 cmul_fused(double2 a, double2 b)
 //
 // Without occupied bands (Bo = 0) the sums of sasx are to be dropped: a 0 / wx^2
 // at wx = 0 leaves a NaN there.
-// wx, iwx2: the frequencies' tables (PoleConst).
-template <int NWC, bool ALL, class Table>
+// MASK: pp.mask_on, a kernel of its own (tested here per element, it costs a tile's
+// epilogue 10%).  wx, iwx2: the frequencies' tables (PoleConst).
+template <int NWC, bool ALL, bool MASK, class Table>
 __device__ __forceinline__ bool pole_terms(const PoleParams &pp, Table wx, Table iwx2, int w0, double2 wt, double2 ie, double2 B,
                                            double2 Bo, double2 (&sach)[NWC], double2 (&sasx)[NWC])
 {
@@ -241,15 +242,12 @@ __device__ __forceinline__ bool pole_terms(const PoleParams &pp, Table wx, Table
             sasx[q].y = __builtin_fma(__builtin_fma(R.y, ys, -RQ.y), rs, sasx[q].y);
         }
     }
-    if (!pp.mask_on) {
-        // B D where the mask would be off.  Opaque: otherwise the |u|^2 of the loop
-        // above are kept for this one.
-        double x = wt.x, y2 = wy2;
-        asm volatile("" : "+v"(x), "+v"(y2));
+    if constexpr (!MASK) {
+        // B D where the mask would be off
 #pragma unroll
         for (int q = 0; q < NWC; ++q) {
             if (!ALL && q > 0 && w0 + q >= pp.nw) break;
-            const double yu = wx[w0 + q] - x, du = yu * yu + y2;
+            const double yu = wx[w0 + q] - wt.x, du = yu * yu + wy2;
             if (!(du > pp.limittwo)) {
                 const double r = rcp_cubic(du);
                 sach[q].x = __builtin_fma(__builtin_fma(P.x, yu, -PQ.x), r, sach[q].x);

@@ -596,7 +596,7 @@ struct PoleLds {
 typedef const __attribute__((address_space(4))) double cdbl;
 static_assert(offsetof(PoleConst, iwx2) == sizeof(double) * kMaxFreq, "tab + kMaxFreq is iwx2");
 
-template <int W, bool ALL, bool ACHS>
+template <int W, bool ALL, bool ACHS, bool MASK>
 __device__ __forceinline__ void oz_pole_block(const PoleArgs &a, cdbl *tab, int b, PoleLds<W> &L)
 {
     constexpr int R = pole_rows(W);
@@ -647,7 +647,7 @@ __device__ __forceinline__ void oz_pole_block(const PoleArgs &a, cdbl *tab, int 
             // kept in scalar registers all along they push others out of them
             // (nw 7: 119 to 150 us at 12000 x 600)
             if constexpr (W > 4) asm volatile("" : "+s"(tab));
-            if (!pole_terms<W, ALL>(a.pp, tab, tab + kMaxFreq, 0, widen(wt[r]), widen(ie[r]), B[r], Bo[r], sach, sasx))
+            if (!pole_terms<W, ALL, MASK>(a.pp, tab, tab + kMaxFreq, 0, widen(wt[r]), widen(ie[r]), B[r], Bo[r], sach, sasx))
                 general |= 1u << r;
             // static-CH remainder -sum B I_eps (gppkernel.deslippe.09.30.2014.f90:192-230)
             if constexpr (ACHS) sachs = csub(sachs, cmul(B[r], widen(ie[r])));
@@ -694,27 +694,38 @@ __device__ __forceinline__ void oz_pole_block(const PoleArgs &a, cdbl *tab, int 
     }
 }
 
-template <int W, bool ALL, bool ACHS>
+template <int W, bool ALL, bool ACHS, bool MASK>
 __global__ __launch_bounds__(256, pole_waves(W)) void gpp_oz_pole_kernel(PoleArgs a)
 {
     __shared__ PoleLds<W> L;
     cdbl *args = (cdbl *)__builtin_amdgcn_kernarg_segment_ptr();   // a is the first argument
-    oz_pole_block<W, ALL, ACHS>(a, args + (offsetof(PoleArgs, pp) + offsetof(PoleParams, pc)) / sizeof(double), blockIdx.x, L);
+    oz_pole_block<W, ALL, ACHS, MASK>(a, args + (offsetof(PoleArgs, pp) + offsetof(PoleParams, pc)) / sizeof(double), blockIdx.x, L);
 }
 
 template <bool ACHS>
 void launch_pole(int blocks, hipStream_t s, const PoleArgs &a)
 {
+    const dim3 grid(blocks), block(256);
+    const int c = oz_class(a.pp.nw);
+    if (!a.pp.mask_on) {
+        switch (c) {
+        case 0: hipLaunchKernelGGL((gpp_oz_pole_kernel<4, false, ACHS, false>), grid, block, 0, s, a); break;
+        case 1: hipLaunchKernelGGL((gpp_oz_pole_kernel<8, false, ACHS, false>), grid, block, 0, s, a); break;
+        case 2: hipLaunchKernelGGL((gpp_oz_pole_kernel<12, false, ACHS, false>), grid, block, 0, s, a); break;
+        default: hipLaunchKernelGGL((gpp_oz_pole_kernel<16, false, ACHS, false>), grid, block, 0, s, a); break;
+        }
+        return;
+    }
     switch (a.pp.nw) {
-    case 1: hipLaunchKernelGGL((gpp_oz_pole_kernel<1, true, ACHS>), dim3(blocks), dim3(256), 0, s, a); break;
-    case 2: hipLaunchKernelGGL((gpp_oz_pole_kernel<2, true, ACHS>), dim3(blocks), dim3(256), 0, s, a); break;
-    case 3: hipLaunchKernelGGL((gpp_oz_pole_kernel<3, true, ACHS>), dim3(blocks), dim3(256), 0, s, a); break;
-    case 4: hipLaunchKernelGGL((gpp_oz_pole_kernel<4, true, ACHS>), dim3(blocks), dim3(256), 0, s, a); break;
+    case 1: hipLaunchKernelGGL((gpp_oz_pole_kernel<1, true, ACHS, true>), grid, block, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((gpp_oz_pole_kernel<2, true, ACHS, true>), grid, block, 0, s, a); break;
+    case 3: hipLaunchKernelGGL((gpp_oz_pole_kernel<3, true, ACHS, true>), grid, block, 0, s, a); break;
+    case 4: hipLaunchKernelGGL((gpp_oz_pole_kernel<4, true, ACHS, true>), grid, block, 0, s, a); break;
     default:
-        switch (oz_class(a.pp.nw)) {
-        case 1: hipLaunchKernelGGL((gpp_oz_pole_kernel<8, false, ACHS>), dim3(blocks), dim3(256), 0, s, a); break;
-        case 2: hipLaunchKernelGGL((gpp_oz_pole_kernel<12, false, ACHS>), dim3(blocks), dim3(256), 0, s, a); break;
-        default: hipLaunchKernelGGL((gpp_oz_pole_kernel<16, false, ACHS>), dim3(blocks), dim3(256), 0, s, a); break;
+        switch (c) {
+        case 1: hipLaunchKernelGGL((gpp_oz_pole_kernel<8, false, ACHS, true>), grid, block, 0, s, a); break;
+        case 2: hipLaunchKernelGGL((gpp_oz_pole_kernel<12, false, ACHS, true>), grid, block, 0, s, a); break;
+        default: hipLaunchKernelGGL((gpp_oz_pole_kernel<16, false, ACHS, true>), grid, block, 0, s, a); break;
         }
     }
 }
@@ -780,13 +791,25 @@ __global__ __launch_bounds__(768, 1) void gpp_oz_gemm_batch_kernel(const OzRecor
 // The problems of one frequency class (first: no blocks for the others).  The
 // arguments by reference: a register copy of them (with the pole parameters of
 // up to 16 frequencies) made this kernel 1.7x slower.
-template <int W>
+template <int W, bool MASK>
 __global__ __launch_bounds__(256, pole_waves(W)) void gpp_oz_pole_batch_kernel(const OzRecord *__restrict__ rec,
                                                                                const int *first, int n)
 {
     __shared__ PoleLds<W> L;
     const int b = (int)blockIdx.x, p = batch_problem(first, n, b);
-    oz_pole_block<W, false, false>(rec[p].pa, (cdbl *)&rec[p].pa.pp.pc, b - first[p], L);
+    oz_pole_block<W, false, false, MASK>(rec[p].pa, (cdbl *)&rec[p].pa.pp.pc, b - first[p], L);
+}
+
+template <bool MASK>
+void launch_pole_batch(int c, int blocks, hipStream_t s, const OzRecord *rec, const int *first, int n)
+{
+    const dim3 grid(blocks), block(256);
+    switch (c) {
+    case 0: hipLaunchKernelGGL((gpp_oz_pole_batch_kernel<4, MASK>), grid, block, 0, s, rec, first, n); break;
+    case 1: hipLaunchKernelGGL((gpp_oz_pole_batch_kernel<8, MASK>), grid, block, 0, s, rec, first, n); break;
+    case 2: hipLaunchKernelGGL((gpp_oz_pole_batch_kernel<12, MASK>), grid, block, 0, s, rec, first, n); break;
+    default: hipLaunchKernelGGL((gpp_oz_pole_batch_kernel<16, MASK>), grid, block, 0, s, rec, first, n); break;
+    }
 }
 
 }  // namespace
@@ -833,7 +856,7 @@ OzBlocks gpp_oz_batch_record(const fk_gpp_problem *p, const fk_options *o, const
 }
 
 int gpp_oz_batch_launch(const void *records, const int *first_prep, const int *first_gemm, const int *first_pole,
-                        int n, int total_prep, int total_gemm, const int *total_pole, hipStream_t s)
+                        int n, int total_prep, int total_gemm, const int *total_pole, bool mask, hipStream_t s)
 {
     const OzRecord *rec = static_cast<const OzRecord *>(records);
     if (total_prep > 0)
@@ -847,14 +870,9 @@ int gpp_oz_batch_launch(const void *records, const int *first_prep, const int *f
     }
     for (int c = 0; c < kOzPoleClasses; ++c) {
         if (total_pole[c] <= 0) continue;
-        const dim3 grid(total_pole[c]), block(256);
         const int *first = first_pole + c * (n + 1);
-        switch (c) {
-        case 0: hipLaunchKernelGGL(gpp_oz_pole_batch_kernel<4>, grid, block, 0, s, rec, first, n); break;
-        case 1: hipLaunchKernelGGL(gpp_oz_pole_batch_kernel<8>, grid, block, 0, s, rec, first, n); break;
-        case 2: hipLaunchKernelGGL(gpp_oz_pole_batch_kernel<12>, grid, block, 0, s, rec, first, n); break;
-        default: hipLaunchKernelGGL(gpp_oz_pole_batch_kernel<16>, grid, block, 0, s, rec, first, n); break;
-        }
+        if (mask) launch_pole_batch<true>(c, total_pole[c], s, rec, first, n);
+        else launch_pole_batch<false>(c, total_pole[c], s, rec, first, n);
     }
     FK_HIP(hipGetLastError());
     return FK_OK;

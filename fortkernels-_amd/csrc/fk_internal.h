@@ -137,7 +137,7 @@ size_t gpp_oz_batch_record_bytes();
 OzBlocks gpp_oz_batch_record(const fk_gpp_problem *p, const fk_options *o, const OzLayout &L, const Scratch &ws,
                              const int *d_igp, void *record);
 int gpp_oz_batch_launch(const void *records, const int *first_prep, const int *first_gemm, const int *first_pole,
-                        int n, int total_prep, int total_gemm, const int *total_pole, hipStream_t s);
+                        int n, int total_prep, int total_gemm, const int *total_pole, bool mask, hipStream_t s);
 
 // FF contraction in split BF16 on MFMA (FK_PREC_MIXED): workspace layout and
 // the launch of the slice pre-pass and the GEMM.  The GEMM writes FP64
