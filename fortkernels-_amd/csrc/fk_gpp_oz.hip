@@ -800,6 +800,30 @@ __global__ __launch_bounds__(256, pole_waves(W)) void gpp_oz_pole_batch_kernel(c
     oz_pole_block<W, false, false, MASK>(rec[p].pa, (cdbl *)&rec[p].pa.pp.pc, b - first[p], L);
 }
 
+// All classes in one launch, in the registers of the largest: for batches of few
+// blocks, where the launches count.  A batch's run with one launch and with one per
+// class, by blocks: 71 58 us and 73; 105 46 and 62; 464 58 and 78; 1196 87 and 92;
+// 1946 115 and 119; 2933 166 and 159; 7417 320 and 285.
+constexpr int kPoleSmallBatch = 2048;
+
+template <bool MASK>
+__global__ __launch_bounds__(256, pole_waves(16)) void gpp_oz_pole_small_batch_kernel(const OzRecord *__restrict__ rec,
+                                                                                     const int *first, int n)
+{
+    __shared__ PoleLds<16> L;
+    int b = (int)blockIdx.x, c = 0;
+    while (b >= first[c * (n + 1) + n]) b -= first[c++ * (n + 1) + n];     // first[n]: the class's blocks
+    c = __builtin_amdgcn_readfirstlane(c);
+    first += c * (n + 1);
+    const int p = batch_problem(first, n, b);
+    cdbl *tab = (cdbl *)&rec[p].pa.pp.pc;
+    const int k = b - first[p];
+    if (c == 0) oz_pole_block<4, false, false, MASK>(rec[p].pa, tab, k, reinterpret_cast<PoleLds<4> &>(L));
+    else if (c == 1) oz_pole_block<8, false, false, MASK>(rec[p].pa, tab, k, reinterpret_cast<PoleLds<8> &>(L));
+    else if (c == 2) oz_pole_block<12, false, false, MASK>(rec[p].pa, tab, k, reinterpret_cast<PoleLds<12> &>(L));
+    else oz_pole_block<16, false, false, MASK>(rec[p].pa, tab, k, L);
+}
+
 template <bool MASK>
 void launch_pole_batch(int c, int blocks, hipStream_t s, const OzRecord *rec, const int *first, int n)
 {
@@ -867,6 +891,18 @@ int gpp_oz_batch_launch(const void *records, const int *first_prep, const int *f
         FK_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
         const int grid = std::max(1, std::min(total_gemm, ncu));
         hipLaunchKernelGGL(gpp_oz_gemm_batch_kernel, dim3(grid), dim3(kWaves12 * 64), 0, s, rec, first_gemm, n);
+    }
+    int pole = 0, classes = 0;
+    for (int c = 0; c < kOzPoleClasses; ++c) {
+        pole += total_pole[c];
+        classes += total_pole[c] > 0;
+    }
+    if (classes > 1 && pole <= kPoleSmallBatch) {
+        const dim3 grid(pole), block(256);
+        if (mask) hipLaunchKernelGGL(gpp_oz_pole_small_batch_kernel<true>, grid, block, 0, s, rec, first_pole, n);
+        else hipLaunchKernelGGL(gpp_oz_pole_small_batch_kernel<false>, grid, block, 0, s, rec, first_pole, n);
+        FK_HIP(hipGetLastError());
+        return FK_OK;
     }
     for (int c = 0; c < kOzPoleClasses; ++c) {
         if (total_pole[c] <= 0) continue;
