@@ -1459,14 +1459,14 @@ struct GppBatch {
     size_t bytes = 0, off_args = 0, off_tiles = 0, off_counter = 0, off_out = 0, off_coef = 0, off_red = 0,
            off_nw = 0, off_ptrs = 0;
     int64_t coef_total = 0;
-    bool few_occ = false;      // every problem has at most kRingOcc occupied bands
+    bool ring_tiles = false;   // configuration 2 runs gpp_ring_tile
     hipStream_t cs = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     fk_options opt;
 
     char *at(size_t off) const { return static_cast<char *>(mem) + off; }
-    bool ring(int c) const { return few_occ && ring_form(c, elem(), 0); }
+    bool ring(int c) const { return ring_tiles && ring_form(c, elem(), 0); }
     size_t elem() const { return mixed ? sizeof(float2) : sizeof(double2); }
 
     ~GppBatch()
@@ -1556,7 +1556,9 @@ struct GppBatch {
         bool done = false;
         if constexpr (sizeof(E) == sizeof(double2)) {
             if (ring(cfg)) {
-                const dim3 grid(ncu * kRingWgs), block(256);
+                // no more workgroups than tiles: with idle ones the dispatch leaves some
+                // CUs three tiles and others one (512 tiles, 400 bands: 170 us, 128 so)
+                const dim3 grid(std::max(1, std::min(ncu * kRingWgs, ntiles))), block(256);
                 if (opt.mask) hipLaunchKernelGGL(gpp_ring_batch_kernel<true>, grid, block, 0, s, args, tiles, ntiles, counter);
                 else hipLaunchKernelGGL(gpp_ring_batch_kernel<false>, grid, block, 0, s, args, tiles, ntiles, counter);
                 done = true;
@@ -1584,8 +1586,18 @@ struct GppBatch {
         off_counter = plan.plan(sizeof(int));
         max_tiles_total = 0;
         coef_total = 0;
-        few_occ = true;
-        for (const fk_gpp_problem &p : src) few_occ = few_occ && p.nvband <= kRingOcc;
+        // gpp_ring_tile if no problem has more than kRingOcc occupied bands and some
+        // problem, with the tiles of all on the GPU, is not ring_idle's
+        int64_t tiles64 = 0;
+        for (const fk_gpp_problem &p : src)
+            if (p.number_bands > 0) tiles64 += (int64_t)div_up(p.ngpown, 64) * div_up(p.ncouls, 64);
+        const int all = (int)std::min<int64_t>(tiles64, 1 << 20);
+        bool few_occ = true, idle = true;
+        for (const fk_gpp_problem &p : src) {
+            few_occ = few_occ && p.nvband <= kRingOcc;
+            idle = idle && ring_idle(all, p.number_bands, p.nfreq);
+        }
+        ring_tiles = few_occ && !idle;
         for (int i = 0; i < n; ++i) {
             BatchProb &b = prob[i];
             const fk_gpp_problem &p = src[i];

@@ -21,3 +21,26 @@ def test_both_sides(fk, fko, nb, C, G, nw, config):
     assert np.max(np.abs(asx - ref_asx)) <= 1e-12 * np.max(np.abs(ref_asx))
     out = fk.gpp_problem(p, config=config, achstemp=True)
     assert out[0].tobytes() == ach.tobytes() and out[1].tobytes() == asx.tobytes()
+
+
+@pytest.mark.parametrize("shapes", [
+    [(336, 1000, 64, 2), (400, 1500, 130, 1)],                # every problem idle on the ring: no ring
+    [(335, 1000, 64, 2), (400, 1500, 130, 1)],                # one is not
+    [(20, 900, 100, 3), (9, 64, 64, 7), (30, 5000, 500, 1)],  # more tiles than workgroups
+    [(5, 64, 64, 1)],                                         # one tile
+])
+def test_batch_both_sides(fk, fko, shapes):
+    import torch
+    ps = [fko.gpp_random(nb, 3, C, G, nw=nw, seed=nb, wtilde_re=(0.5, 5.5)) for nb, C, G, nw in shapes]
+    dev = [dict(nb=p.nb, nv=p.nv, ncouls=p.ncouls, ngpown=p.ngpown, wx=p.wx, inv_igp_index=p.inv_igp_index,
+                indinv=p.indinv, **{k: torch.from_numpy(np.ascontiguousarray(getattr(p, k))).to("cuda:0")
+                                    for k in ("aqsm", "aqsn", "I_eps", "wtilde", "vcoul")}) for p in ps]
+    torch.cuda.synchronize()
+    batch = fk.GppBatch(dev, precision="fp64", config=2)
+    for _ in range(2):
+        ach, asx, _ = batch.run()
+        torch.cuda.synchronize()
+        for p, a, x in zip(ps, ach, asx):
+            ref_ach, ref_asx, _ = fko.gpp(p, nthreads=0)
+            assert np.max(np.abs(a.cpu().numpy() - ref_ach)) <= 1e-12 * np.max(np.abs(ref_ach))
+            assert np.max(np.abs(x.cpu().numpy() - ref_asx)) <= 1e-12 * np.max(np.abs(ref_asx))
