@@ -630,6 +630,9 @@ __device__ __forceinline__ void oz_pole_block(const PoleArgs &a, cdbl *tab, int 
             ie[r] = a.I_eps[row[r] * a.C + ig];
             Bo[r] = make_double2(0.0, 0.0);
         }
+        // unrolled for the latency of the coefficients' scalar loads (512/64/32768/1638
+        // 2.68 ms, so 2.37; 1000/1000/200/200, 1 frequency, 331 us, so 162)
+#pragma unroll 4
         for (int n1 = 0; n1 < a.nv; ++n1) {
             const double2 x = widen(a.aqsn[(size_t)n1 * a.C + ig]);
             cdbl *co = occ + (size_t)n1 * a.ldm * 2;
