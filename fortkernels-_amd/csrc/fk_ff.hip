@@ -422,7 +422,9 @@ void launch_ff_fused(int cfg, int tiles, hipStream_t s, const FfArgs &a)
 // tiles to fill the GPU: the time of the busiest CU, counting a part's
 // set-up and epilogue as kPartCost stages and one or two workgroups on a CU
 // as slower than three (they leave the MFMA pipes idle at their barriers).
+// (A workspace is sized without a device, so the CU count is the MI355X's.)
 constexpr int kPartCost = 24;
+constexpr int kPlanCus = 256;
 int ig_parts(int tiles, int stages, int most, int least_stages)
 {
     const double rate[4] = {0.0, 0.75, 0.92, 1.0};
@@ -431,7 +433,7 @@ int ig_parts(int tiles, int stages, int most, int least_stages)
     for (int k = 1; k <= most && (k == 1 || stages >= k * least_stages); ++k) {
         const int per = div_up(stages, k);
         if (div_up(stages, per) != k) continue;   // no part empty
-        const int on_cu = (int)(((int64_t)tiles * k + 255) / 256);
+        const int on_cu = (int)(((int64_t)tiles * k + kPlanCus - 1) / kPlanCus);
         const double cost = (double)on_cu * (per + kPartCost) / rate[std::min(on_cu, 3)];
         if (cost < best_cost) { best_cost = cost; best = k; }
     }
@@ -466,6 +468,11 @@ FfLayout ff_plan(const fk_ff_problem *p, const fk_options *o, Scratch &ws)
             while (tiles * L.ksplit < 1024 && L.ksplit < 8 && chunks / (2 * L.ksplit) >= 2) L.ksplit *= 2;
         } else {
             L.nks = div_up(p->ncouls, 8);
+            // A named configuration keeps the workspace that it has always asked for, at
+            // most 8 parts (of at least 24 stages), and pays for it where tiles are few:
+            // 32/512/256/8 47 us, the default 31; 64/1000/100/2 40, 30.  A batch runs
+            // named configurations and gives their calls' results bit for bit (6 problems
+            // of 32/512/256/8 279 us, 171 if they were split as the default).
             L.ksplit = o->config > 0 ? ig_parts(tiles, L.nks, 8, 24) : ig_parts(tiles, L.nks, 32, 8);
             L.kper = div_up(L.nks, L.ksplit);
         }

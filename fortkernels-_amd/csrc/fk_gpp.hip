@@ -16,7 +16,7 @@
 // Kernels (one call = three launches on the caller's stream):
 //   gpp_coef_kernel   c[Kpad][ldc] from aqsm / vcoul / the column map, with
 //                     the occupied bands first, zero-padded to a k-step
-//   gpp_ring_kernel   FP64, up to 16 occupied bands: MFMA GEMM tile with its
+//   gpp_ring_kernel   FP64, up to 24 occupied bands: MFMA GEMM tile with its
 //                     operands through an LDS ring, the pole/SX epilogue and
 //                     a wave/workgroup reduction -> per-tile partials
 //   gpp_fused_kernel  otherwise: MFMA GEMM tile with operand fragments loaded straight
@@ -487,7 +487,7 @@ __device__ __forceinline__ void gpp_tile(const GppArgs<E> &a, int tm, int tn, Ti
 constexpr int kRingStages = 3;
 constexpr int kRingWgs = 3;      // workgroups per CU
 constexpr int kRingSmallWgs = 3; // of the 32 x 32 tiles, at least
-constexpr int kRingOcc = 16;
+constexpr int kRingOcc = 24;
 // Frequencies per epilogue pass of calls with more than three: what the registers
 // hold (a batch of 12 problems of 3 to 11 frequencies takes 6.58 ms with 3, 6.42
 // with 4, 6.24 with 5, 6.17 with 6; with the static-CH remainder, 7 frequencies of
@@ -945,8 +945,12 @@ void launch_fused(int cfg, int tiles, hipStream_t s, const GppArgs<E> &a)
 
 // gpp_ring_tile runs FP64 calls with the 64 x 64 tiles and at most kRingOcc
 // occupied bands: it contracts those block by block, half the work per loaded
-// fragment, which is lost in the whole while they are few (16 of 512 bands
-// cost nothing that could be measured against 4).
+// fragment, and once per pass over the frequencies.  Up to 24 it is the faster one
+// everywhere, past that it depends on the rest (occupied bands, ring and gpp_tile,
+// us): 512/./32768/1638 32 2820 and 3111, 128 2989 and 3112; 128/./8192/409 32 91 and
+// 107, 64 103 and 106, 128 126 and 106; 333/./10007/1001 with 7 frequencies 17 530 and
+// 592, 32 556 and 592, 64 632 and 592; 200/./3000/300 in 64 x 64 tiles 20 47 and 48,
+// 32 50 and 48.
 bool ring_form(int cfg, size_t elem, int nv) { return cfg == 1 && elem == sizeof(double2) && nv <= kRingOcc; }
 
 // ring_idle: long band loops on a GPU that the 64 x 64 tiles do not fill.  With one
@@ -1006,7 +1010,7 @@ int choose_cfg(const fk_gpp_problem *p, const fk_options *o)
 {
     (void)p;
     if (o->config > 0) return o->config - 1;
-    // 32x32 wave tiles, two staggered workgroups per CU: the fastest measured
+    // 32x32 wave tiles (the ring ones where ring_form allows): the fastest measured
     // at 512/2/32768/20 and 128/2/8192/20
     return 1;
 }

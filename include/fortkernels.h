@@ -298,7 +298,8 @@ typedef struct {
  * and achsDtemp_Kernel (FFKer_cori/ffKernel.cpp:107).  schDt: [nb][nfreq];
  * schDv: [nb][nfreq] or NULL; achsDtemp: one value or NULL.
  * options->config: FK_PREC_FP64: 0 = default, 1 = 64x64 tiles, 2 = 64x128
- * tiles, 3 = 16x64 tiles staged through LDS, the ig range split over
+ * tiles (the default has 64x64 ones too; with few of them it splits the ig
+ * range into up to 32 parts, 1 and 2 into up to 8), 3 = 16x64 tiles staged through LDS, the ig range split over
  * workgroups (for 16 bands or fewer); FK_PREC_MIXED (split
  * BF16): ig chunk of 0 = 1024 (default), 1 = 256, 2 = 512, 3 = 1024 (a
  * smaller chunk: less FP32 rounding, more workgroups and partials). */

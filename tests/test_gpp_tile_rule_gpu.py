@@ -23,6 +23,18 @@ def test_both_sides(fk, fko, nb, C, G, nw, config):
     assert out[0].tobytes() == ach.tobytes() and out[1].tobytes() == asx.tobytes()
 
 
+@pytest.mark.parametrize("config", [0, 2])
+@pytest.mark.parametrize("nb,nv,C,G,nw", [(40, 17, 300, 70, 3), (40, 24, 300, 70, 3), (40, 25, 300, 70, 3), (24, 24, 129, 65, 8),
+                                          (60, 23, 2561, 1000, 2)])
+def test_occupied_bands(fk, fko, config, nb, nv, C, G, nw):
+    """Up to 24 occupied bands on the ring, more without it."""
+    p = fko.gpp_random(nb, nv, C, G, nw=nw, seed=nb + nv, wtilde_re=(0.5, 5.5))
+    ref_ach, ref_asx, _ = fko.gpp(p, nthreads=0)
+    ach, asx, _ = fk.gpp_problem(p, config=config)
+    assert np.max(np.abs(ach - ref_ach)) <= 1e-12 * np.max(np.abs(ref_ach))
+    assert np.max(np.abs(asx - ref_asx)) <= 1e-12 * np.max(np.abs(ref_asx))
+
+
 @pytest.mark.parametrize("shapes", [
     [(336, 1000, 64, 2), (400, 1500, 130, 1)],                # every problem idle on the ring: no ring
     [(335, 1000, 64, 2), (400, 1500, 130, 1)],                # one is not
