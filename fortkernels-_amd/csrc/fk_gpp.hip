@@ -972,6 +972,10 @@ bool ring_idle(int tiles64, int nb, int nw)
 {
     return tiles64 <= 256 ? nb > 275 * nw - 215 : tiles64 <= 512 && nb > 700 * nw - 600;
 }
+int tiles64(const fk_gpp_problem *p)
+{
+    return (int)std::min<int64_t>((int64_t)div_up(p->ngpown, 64) * div_up(p->ncouls, 64), 1 << 20);
+}
 bool ring_small(int tiles64, int nb, int nw)
 {
     if (nb <= 160) return tiles64 <= (nb <= 48 ? 640 : 384);
@@ -1030,10 +1034,8 @@ Layout plan_layout(const fk_gpp_problem *p, const fk_options *o, Scratch &ws, si
     const TileCfg &t = kCfgs[L.cfg];
     L.ring = 0;
     if (!sym && ring_form(L.cfg, elem, p->nvband)) {
-        const int64_t tiles64 = (int64_t)div_up(p->ngpown, 64) * div_up(p->ncouls, 64);
-        const int tiles = (int)std::min<int64_t>(tiles64, 1 << 20);
-        if (o->config == 0 && ring_small(tiles, p->number_bands, p->nfreq)) L.ring = 32;
-        else L.ring = ring_idle(tiles, p->number_bands, p->nfreq) ? 0 : 64;
+        if (o->config == 0 && ring_small(tiles64(p), p->number_bands, p->nfreq)) L.ring = 32;
+        else L.ring = ring_idle(tiles64(p), p->number_bands, p->nfreq) ? 0 : 64;
     }
     const int bm = L.ring ? L.ring : t.bm, bn = L.ring ? L.ring : t.bn;
     const int kstep = L.ring ? 8 : 4 * t.p;
@@ -1404,9 +1406,9 @@ __global__ __launch_bounds__(256) void gpp_reduce_batch_kernel(const ReduceBatch
     }
 }
 
-__global__ void set_int_kernel(int *p, int v)
+__global__ void clear_counters_kernel(int *p)
 {
-    if (threadIdx.x == 0) *p = v;
+    if (threadIdx.x < 2) p[threadIdx.x] = 0;
 }
 
 // ach[p][iw] = out[p][0][iw], asx[p][iw] = out[p][1][iw] for iw < nw[p]
@@ -1463,14 +1465,19 @@ struct GppBatch {
     size_t bytes = 0, off_args = 0, off_tiles = 0, off_counter = 0, off_out = 0, off_coef = 0, off_red = 0,
            off_nw = 0, off_ptrs = 0;
     int64_t coef_total = 0;
-    bool ring_tiles = false;   // configuration 2 runs gpp_ring_tile
+    int nring = 0;             // tiles of gpp_ring_tile, the first of the table
     hipStream_t cs = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     fk_options opt;
 
     char *at(size_t off) const { return static_cast<char *>(mem) + off; }
-    bool ring(int c) const { return ring_tiles && ring_form(c, elem(), 0); }
+    // whether problem i runs on gpp_ring_tile: as its single call of that configuration
+    bool ring(int i, int c) const
+    {
+        const fk_gpp_problem &p = src[i];
+        return ring_form(c, elem(), p.nvband) && !ring_idle(tiles64(&p), p.number_bands, p.nfreq);
+    }
     size_t elem() const { return mixed ? sizeof(float2) : sizeof(double2); }
 
     ~GppBatch()
@@ -1512,7 +1519,7 @@ struct GppBatch {
             // larger padding.  (With the common padding the batch ran 3.5%
             // slower than the single calls.)
             const int kstep = 4 * t.p;
-            a.Kpad = ring(c) ? b.nvpad + div_up(b.nb - b.nv, 8) * 8
+            a.Kpad = ring(i, c) ? b.nvpad + div_up(b.nb - b.nv, 8) * 8
                              : div_up(std::max(b.nvpad + b.nb - b.nv, 1), kstep) * kstep;
             a.nks = a.Kpad / 4;
             a.aligned = ring::aligned16(a.c) | ring::aligned16(a.aqsn) << 1;
@@ -1524,10 +1531,14 @@ struct GppBatch {
             if (b.nb > 0) order.push_back({{-a.nks, -b.nw}, i});
         }
         std::stable_sort(order.begin(), order.end());
-        for (const auto &o : order) {
-            const GppArgs<E> &a = args[o.second];
-            for (int tn = 0; tn < a.tiles_n; ++tn)
-                for (int tm = 0; tm < a.tiles_m; ++tm) tiles.push_back({o.second, tm, tn});
+        for (const bool on_ring : {true, false}) {
+            for (const auto &o : order) {
+                if (ring(o.second, c) != on_ring) continue;
+                const GppArgs<E> &a = args[o.second];
+                for (int tn = 0; tn < a.tiles_n; ++tn)
+                    for (int tm = 0; tm < a.tiles_m; ++tm) tiles.push_back({o.second, tm, tn});
+            }
+            if (on_ring) nring = (int)tiles.size();
         }
         ntiles = (int)tiles.size();
         std::vector<ReduceBatch> red(n);
@@ -1550,25 +1561,24 @@ struct GppBatch {
     template <class E>
     int enqueue(hipStream_t s)
     {
-        hipLaunchKernelGGL(set_int_kernel, dim3(1), dim3(64), 0, s, reinterpret_cast<int *>(at(off_counter)), 0);
+        hipLaunchKernelGGL(clear_counters_kernel, dim3(1), dim3(64), 0, s, reinterpret_cast<int *>(at(off_counter)));
         const int cblocks = (int)std::min<int64_t>((coef_total + 255) / 256, 1 << 16);
         hipLaunchKernelGGL(gpp_coef_batch_kernel<E>, dim3(std::max(cblocks, 1)), dim3(256), 0, s,
                            reinterpret_cast<const CoefBatch<E> *>(at(off_coef)), n, coef_total);
         const GppArgs<E> *args = reinterpret_cast<const GppArgs<E> *>(at(off_args));
         const BatchTile *tiles = reinterpret_cast<const BatchTile *>(at(off_tiles));
         int *counter = reinterpret_cast<int *>(at(off_counter));
-        bool done = false;
         if constexpr (sizeof(E) == sizeof(double2)) {
-            if (ring(cfg)) {
+            if (nring > 0) {
                 // no more workgroups than tiles: with idle ones the dispatch leaves some
                 // CUs three tiles and others one (512 tiles, 400 bands: 170 us, 128 so)
-                const dim3 grid(std::max(1, std::min(ncu * kRingWgs, ntiles))), block(256);
-                if (opt.mask) hipLaunchKernelGGL(gpp_ring_batch_kernel<true>, grid, block, 0, s, args, tiles, ntiles, counter);
-                else hipLaunchKernelGGL(gpp_ring_batch_kernel<false>, grid, block, 0, s, args, tiles, ntiles, counter);
-                done = true;
+                const dim3 grid(std::min(ncu * kRingWgs, nring)), block(256);
+                if (opt.mask) hipLaunchKernelGGL(gpp_ring_batch_kernel<true>, grid, block, 0, s, args, tiles, nring, counter);
+                else hipLaunchKernelGGL(gpp_ring_batch_kernel<false>, grid, block, 0, s, args, tiles, nring, counter);
             }
         }
-        if (!done) launch_batch<E>(cfg, ncu * kCfgs[cfg].minw, s, args, tiles, ntiles, counter);
+        if (ntiles > nring)
+            launch_batch<E>(cfg, ncu * kCfgs[cfg].minw, s, args, tiles + nring, ntiles - nring, counter + 1);
         hipLaunchKernelGGL(gpp_reduce_batch_kernel, dim3(2 * kMaxFreq, n), dim3(256), 0, s,
                            reinterpret_cast<const ReduceBatch *>(at(off_red)), reinterpret_cast<double2 *>(at(off_out)));
         FK_HIP(hipGetLastError());
@@ -1587,21 +1597,9 @@ struct GppBatch {
         off_nw = plan.plan(sizeof(int) * n);
         off_ptrs = plan.plan(sizeof(void *) * 2 * n);
         off_out = plan.plan(sizeof(double2) * 2 * kMaxFreq * n);
-        off_counter = plan.plan(sizeof(int));
+        off_counter = plan.plan(2 * sizeof(int));    // of the ring tiles, of the others
         max_tiles_total = 0;
         coef_total = 0;
-        // gpp_ring_tile if no problem has more than kRingOcc occupied bands and some
-        // problem, with the tiles of all on the GPU, is not ring_idle's
-        int64_t tiles64 = 0;
-        for (const fk_gpp_problem &p : src)
-            if (p.number_bands > 0) tiles64 += (int64_t)div_up(p.ngpown, 64) * div_up(p.ncouls, 64);
-        const int all = (int)std::min<int64_t>(tiles64, 1 << 20);
-        bool few_occ = true, idle = true;
-        for (const fk_gpp_problem &p : src) {
-            few_occ = few_occ && p.nvband <= kRingOcc;
-            idle = idle && ring_idle(all, p.number_bands, p.nfreq);
-        }
-        ring_tiles = few_occ && !idle;
         for (int i = 0; i < n; ++i) {
             BatchProb &b = prob[i];
             const fk_gpp_problem &p = src[i];

@@ -42,6 +42,7 @@
 #include "fk_complex.h"
 #include "fk_gpp_common.h"
 #include "fk_internal.h"
+#include "fk_mfma_ring.h"
 
 #include <algorithm>
 #include <cstddef>
@@ -80,14 +81,15 @@ __device__ __forceinline__ void split4(double x, double scale, int8_t (&s)[kSlic
 
 
 // ---------------------------------------------------------------------------
-// Slices of both operands in one launch.  A workgroup takes 4 coefficient
-// rows (the first ldm/4 workgroups) or 16 aqsn columns (the rest).  Each
+// Slices of both operands in one launch.  A workgroup takes 8 coefficient
+// rows (the first ldm/8 workgroups) or 16 aqsn columns (the rest).  Each
 // row (column) feeds three real matrices, cr, ci, cr + ci (ar, ai, ar + ai),
 // each with its own scale: the workgroup finds the three maxima over all
 // bands, then splits the three values of each band into four slices, band
-// block by band block (16 bands = the 16 bytes of one fragment lane); the
-// second pass finds the workgroup's slab in L2.  Thread t of an R-wide
-// slab: row or column R x + t%R, band blocks t/R, t/R + 256/R, ...
+// block by band block (16 bands = the 16 bytes of one fragment lane); a
+// thread's first block stays in registers in between, the others are read
+// again.  Thread t of an R-wide slab: row or column R x + t%R, band blocks t/R,
+// t/R + 512/R, ...
 // ---------------------------------------------------------------------------
 struct PrepArgs {
     const float2 *aqsm, *aqsn;
@@ -282,20 +284,7 @@ __device__ __forceinline__ void oz_tile(int b, int tiles_m, int tiles_n, int gro
 }
 
 
-// One direct global->LDS load of 16 bytes per lane: lane l's bytes land at
-// LDS byte address lds + 16 l.  Written as inline asm so that the compiler's
-// wait insertion, which cannot tell which LDS these loads write, does not
-// make every LDS read wait for every load in flight; the kernel orders its
-// loads and reads itself with explicit vmcnt waits and barriers.  The asm
-// has no register outputs.
-__device__ __forceinline__ void lds_load16(const int8_t *g, const int8_t *lds)
-{
-    // the LDS offset (low half of the shared-aperture address), uniform
-    const unsigned la = (unsigned)__builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)lds);
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(la) : "memory", "m0");
-}
-
-// The same from a wave-uniform base (kept in SGPRs) plus a per-lane byte
+// ring::lds_load16 from a wave-uniform base (kept in SGPRs) plus a per-lane byte
 // offset: one VGPR serves every load of the kernel.
 __device__ __forceinline__ void lds_load16(const int8_t *base, unsigned voff, const int8_t *lds)
 {
@@ -386,8 +375,7 @@ __device__ __forceinline__ void oz_gemm12_tiles(const GemmArgs &a, int first, in
             const int q = 2 * wave + (lane >> 5);
             const double *g = q < kProds ? a.ra + (size_t)q * a.ldm + tm * kBM
                                          : a.rb + (size_t)(q - kProds) * a.ldn + tn * kBN;
-            lds_load16(reinterpret_cast<const int8_t *>(g + 2 * (lane & 31)),
-                       reinterpret_cast<const int8_t *>(&scl[t & 1][2 * wave][0]));
+            ring::lds_load16(g + 2 * (lane & 31), &scl[t & 1][2 * wave][0]);
         }
     };
     auto read_frag = [&](const int8_t *st, Frags12 &f, int r) {
@@ -551,7 +539,7 @@ __global__ __launch_bounds__(768, 1) void gpp_oz_gemm_kernel(GemmArgs a, int til
 //
 // Measured: 512/2/32768/1638, 3 frequencies 367 us (4.7 TB/s; without the pole
 // terms 300 us, 5.7 TB/s), the form of one row and two quotients 558; a batch of
-// 12 problems of 3 to 11 frequencies 1.50 ms, before 2.65.  Two rows cost the
+// 12 problems of 3 to 11 frequencies 1.35 ms, before 2.65.  Two rows cost the
 // same at 3 frequencies and 8% more at 7, loading one iteration ahead 5% more.
 //
 // W is the kernel's class, 4, 8, 12 or 16 frequencies (exact for a single call
@@ -575,7 +563,9 @@ struct PoleArgs {
 };
 
 // Workgroups per group of rows: runs of at most 16 iterations of 256 columns,
-// shorter where the rows alone give fewer than about 8 workgroups per CU.
+// shorter where the rows alone give fewer than about 8 workgroups per CU (two to
+// three rounds of what the kernels' registers let onto one: 3 or 4, 2 for the class
+// of 16; sized without a device, so for the MI355X's 256 CUs).
 inline int pole_chunks(int G, int C, int nw)
 {
     const int iters = div_up(C, 256), groups = div_up(G, pole_rows(4 * oz_class(nw) + 4));

@@ -36,14 +36,17 @@ def test_occupied_bands(fk, fko, config, nb, nv, C, G, nw):
 
 
 @pytest.mark.parametrize("shapes", [
-    [(336, 1000, 64, 2), (400, 1500, 130, 1)],                # every problem idle on the ring: no ring
-    [(335, 1000, 64, 2), (400, 1500, 130, 1)],                # one is not
-    [(20, 900, 100, 3), (9, 64, 64, 7), (30, 5000, 500, 1)],  # more tiles than workgroups
-    [(5, 64, 64, 1)],                                         # one tile
+    [(336, 3, 1000, 64, 2), (400, 0, 1500, 130, 1)],                     # all idle on the ring: none of it
+    [(335, 3, 1000, 64, 2), (400, 3, 1500, 130, 1), (60, 9, 700, 60, 7)],   # both kernels
+    [(20, 24, 900, 100, 3), (30, 25, 900, 100, 3), (90, 60, 300, 70, 11)],
+    [(20, 3, 900, 100, 3), (9, 1, 64, 64, 7), (30, 2, 5000, 500, 1)],    # more tiles than workgroups
+    [(5, 3, 64, 64, 1)],                                                 # one tile
 ])
-def test_batch_both_sides(fk, fko, shapes):
+def test_batch_kernel_by_problem(fk, fko, shapes):
+    """Each problem of a batch takes the kernel of its single call of the same
+    configuration, and gives its bits."""
     import torch
-    ps = [fko.gpp_random(nb, 3, C, G, nw=nw, seed=nb, wtilde_re=(0.5, 5.5)) for nb, C, G, nw in shapes]
+    ps = [fko.gpp_random(max(nb, nv), nv, C, G, nw=nw, seed=nb, wtilde_re=(0.5, 5.5)) for nb, nv, C, G, nw in shapes]
     dev = [dict(nb=p.nb, nv=p.nv, ncouls=p.ncouls, ngpown=p.ngpown, wx=p.wx, inv_igp_index=p.inv_igp_index,
                 indinv=p.indinv, **{k: torch.from_numpy(np.ascontiguousarray(getattr(p, k))).to("cuda:0")
                                     for k in ("aqsm", "aqsn", "I_eps", "wtilde", "vcoul")}) for p in ps]
@@ -54,5 +57,8 @@ def test_batch_both_sides(fk, fko, shapes):
         torch.cuda.synchronize()
         for p, a, x in zip(ps, ach, asx):
             ref_ach, ref_asx, _ = fko.gpp(p, nthreads=0)
-            assert np.max(np.abs(a.cpu().numpy() - ref_ach)) <= 1e-12 * np.max(np.abs(ref_ach))
-            assert np.max(np.abs(x.cpu().numpy() - ref_asx)) <= 1e-12 * np.max(np.abs(ref_asx))
+            one_ach, one_asx, _ = fk.gpp_problem(p, config=2)
+            assert a.cpu().numpy().tobytes() == one_ach.tobytes() and x.cpu().numpy().tobytes() == one_asx.tobytes()
+            assert np.max(np.abs(one_ach - ref_ach)) <= 1e-12 * np.max(np.abs(ref_ach))
+            if p.nv:
+                assert np.max(np.abs(one_asx - ref_asx)) <= 1e-12 * np.max(np.abs(ref_asx))
