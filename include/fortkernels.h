@@ -237,15 +237,17 @@ size_t gpp_kernel_noalloc_max_workspace(void);
  * the fastest of all configurations timed on this batch -- create then
  * runs the batch 2 x 4 times, so the inputs must be valid), and captures
  * the launches of one run into a graph: one coefficient kernel, one
- * persistent kernel whose workgroups take tiles from a shared counter, one
- * reduction.  Inputs are device memory (FK_MEM_DEVICE) and are read again
+ * persistent kernel whose workgroups take tiles from a shared counter (FP64
+ * configuration 2: up to two, each problem in the kernel its single call
+ * takes), one reduction.  Inputs are device memory (FK_MEM_DEVICE) and are read again
  * on every run, so new values in the same arrays need no new batch.
  * Problems: nfreq <= 16; the arrays must outlive the batch.
  *
  * options->precision = FK_PREC_MIXED takes complex64 problems.  With
  * options->config = 0 it runs gpp_kernel's mixed path, the int8-split
- * contraction, for every problem: its operand-slice, int8 GEMM and FP64
- * pole kernels each as one launch over all problems' blocks, then one
+ * contraction, for every problem: its operand-slice and int8 GEMM kernels
+ * each as one launch over all problems' blocks, its FP64 pole kernel as one
+ * per class of frequency counts (a small batch: one for all), then one
  * reduction (error below 1e-8 against FP64 on the same values; problems of
  * at most 16000 bands).  With config 1..4 it runs the persistent tile kernel
  * with FP32 MFMA in that configuration (error ~1e-6).
